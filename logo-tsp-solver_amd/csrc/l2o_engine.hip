@@ -207,6 +207,9 @@ struct slot_t {
     bool done = false;
     bool done_reported = false;
     float slack = 1.0f;
+    // only single sweeps run on it: their candidates go to the spare pool (the
+    // row after the slots' ones), which no kernel reads
+    bool sweep_only = false;
     uint32_t group_lead = L2O_NO_GROUP;  // multi-start ILS group (first slot)
     uint32_t group_size = 0;
 };
@@ -221,6 +224,7 @@ struct logo2opt_engine {
     uint32_t max_slots = 0;
     std::vector<slot_t> slots;
     l2o_inst *d_insts = nullptr;
+    unsigned long long *d_pool = nullptr;  // L2O_POOL keys per slot, and a spare row
     unsigned *d_live = nullptr;
     unsigned *h_live = nullptr;  // pinned
     unsigned live = 0;           // host mirror, valid between runs
@@ -365,6 +369,7 @@ int upload_instance(logo2opt_engine *e, int32_t id, const uint32_t *route, uint3
         p += al(8ull * ((uint64_t)s.job.ils_rounds + 1));
     }
     if (s.job.log_cap) in.log = (l2o_move *)p;
+    in.pool = e->d_pool + (size_t)L2O_POOL * (s.sweep_only ? e->max_slots : (uint32_t)id);
     in.n = n;
     in.log_cap = s.job.log_cap;
     in.slack = s.slack;
@@ -706,7 +711,8 @@ int engine_run(logo2opt_engine *e, uint32_t max_steps, uint32_t sync_every, uint
 
 // admits an instance into slot `id` (free); group_lead / group_size as in l2o_inst
 int engine_add_at(logo2opt_engine *e, int32_t id, uint32_t n, const logo2opt_city_coords *coords,
-                  const uint32_t *route, const logo2opt_job *job, uint32_t group_lead, uint32_t group_size)
+                  const uint32_t *route, const logo2opt_job *job, uint32_t group_lead, uint32_t group_size,
+                  bool sweep_only = false)
 {
     if (n < 3 || n > LOGO2OPT_MAX_N) return LOGO2OPT_EINVAL;
     slot_t tmp;
@@ -716,6 +722,7 @@ int engine_add_at(logo2opt_engine *e, int32_t id, uint32_t n, const logo2opt_cit
     if (rc) return rc;
     tmp.group_lead = group_lead;
     tmp.group_size = group_size;
+    tmp.sweep_only = sweep_only;
     logo2opt_job j{};
     if (job) j = *job;
     if (j.kick > 1 || j.metric > LOGO2OPT_METRIC_ATT) return LOGO2OPT_EINVAL;
@@ -749,7 +756,7 @@ int engine_add_at(logo2opt_engine *e, int32_t id, uint32_t n, const logo2opt_cit
 }
 
 int engine_add(logo2opt_engine *e, uint32_t n, const logo2opt_city_coords *coords, const uint32_t *route,
-               const logo2opt_job *job, int32_t *slot_out)
+               const logo2opt_job *job, int32_t *slot_out, bool sweep_only = false)
 {
     int32_t id = -1;
     for (uint32_t k = 0; k < e->max_slots; ++k)
@@ -758,7 +765,7 @@ int engine_add(logo2opt_engine *e, uint32_t n, const logo2opt_city_coords *coord
             break;
         }
     if (id < 0) return LOGO2OPT_EAGAIN;
-    const int rc = engine_add_at(e, id, n, coords, route, job, L2O_NO_GROUP, 0);
+    const int rc = engine_add_at(e, id, n, coords, route, job, L2O_NO_GROUP, 0, sweep_only);
     if (rc == LOGO2OPT_OK) *slot_out = id;
     return rc;
 }
@@ -843,6 +850,10 @@ int engine_remove(logo2opt_engine *e, int32_t id)
         L2O_TRY(hipMemcpyAsync(&in, e->d_insts + id, sizeof(in), hipMemcpyDeviceToHost, e->stream));
         L2O_TRY(hipStreamSynchronize(e->stream));
         if (in.phase != L2O_DONE) {
+            // (a finished instance has left its pool empty)
+            if (!s.sweep_only)
+                L2O_TRY(hipMemsetAsync(e->d_pool + (size_t)L2O_POOL * id, 0xFF,
+                                       sizeof(unsigned long long) * L2O_POOL, e->stream));
             e->live -= 1;
             *e->h_live = e->live;
             L2O_TRY(hipMemcpyAsync(e->d_live, e->h_live, sizeof(unsigned), hipMemcpyHostToDevice, e->stream));
@@ -875,6 +886,7 @@ int engine_create(int device, uint64_t budget, uint32_t max_slots, logo2opt_engi
     bool ok = hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking) == hipSuccess &&
               hipMalloc(&e->d_arena, budget) == hipSuccess &&
               hipMalloc(&e->d_insts, sizeof(l2o_inst) * max_slots) == hipSuccess &&
+              hipMalloc(&e->d_pool, sizeof(unsigned long long) * L2O_POOL * (max_slots + 1)) == hipSuccess &&
               hipMalloc(&e->d_live, sizeof(unsigned)) == hipSuccess &&
               hipMalloc(&e->d_scratch, sizeof(unsigned long long) * 4) == hipSuccess &&
               hipHostMalloc(&e->h_live, sizeof(unsigned), hipHostMallocDefault) == hipSuccess &&
@@ -883,6 +895,7 @@ int engine_create(int device, uint64_t budget, uint32_t max_slots, logo2opt_engi
     if (ok) {
         e->ar.init(e->d_arena, budget);
         ok = hipMemsetAsync(e->d_insts, 0, sizeof(l2o_inst) * max_slots, e->stream) == hipSuccess &&
+             hipMemsetAsync(e->d_pool, 0xFF, sizeof(unsigned long long) * L2O_POOL * max_slots, e->stream) == hipSuccess &&
              hipMemsetAsync(e->d_live, 0, sizeof(unsigned), e->stream) == hipSuccess &&
              hipStreamSynchronize(e->stream) == hipSuccess;
     }
@@ -990,6 +1003,7 @@ int logo2opt_engine_destroy(logo2opt_engine *e)
     if (e->d_aitems) (void)hipFree(e->d_aitems);
     if (e->d_arena) (void)hipFree(e->d_arena);
     if (e->d_insts) (void)hipFree(e->d_insts);
+    if (e->d_pool) (void)hipFree(e->d_pool);
     if (e->d_live) (void)hipFree(e->d_live);
     if (e->d_scratch) (void)hipFree(e->d_scratch);
     if (e->h_live) (void)hipHostFree(e->h_live);
@@ -1209,7 +1223,7 @@ void ctx_accumulate(logo2opt_ctx *c)
     }
 }
 
-int ctx_load(logo2opt_ctx *c, const uint32_t *route, logo2opt_job job)
+int ctx_load(logo2opt_ctx *c, const uint32_t *route, logo2opt_job job, bool sweep_only = false)
 {
     job.metric = c->metric;
     if (c->slot >= 0) {
@@ -1231,7 +1245,7 @@ int ctx_load(logo2opt_ctx *c, const uint32_t *route, logo2opt_job job)
         logo2opt_engine_destroy(old);
         c->e = e;
     }
-    return engine_add(c->e, c->n, c->coords.data(), route, &job, &c->slot);
+    return engine_add(c->e, c->n, c->coords.data(), route, &job, &c->slot, sweep_only);
 }
 
 }  // namespace
@@ -1243,7 +1257,7 @@ int logo2opt_step(logo2opt_ctx *ctx, const uint32_t *route, logo2opt_best2_out *
     if (hipSetDevice(e->device) != hipSuccess) return LOGO2OPT_EDEVICE;
     const double h0 = now_ms();
     logo2opt_job job{};
-    int rc = ctx_load(ctx, route, job);
+    int rc = ctx_load(ctx, route, job, true);
     if (rc) return rc;
     e = ctx->e;  // ctx_load replaces the engine when it needs a larger one
     rc = rebuild_lists(e);
@@ -1477,7 +1491,7 @@ int logo2opt_route_length(logo2opt_ctx *ctx, const uint32_t *route, uint64_t *le
     logo2opt_engine *e = ctx->e;
     if (hipSetDevice(e->device) != hipSuccess) return LOGO2OPT_EDEVICE;
     logo2opt_job job{};
-    int rc = ctx_load(ctx, route, job);
+    int rc = ctx_load(ctx, route, job, true);
     if (rc) return rc;
     e = ctx->e;  // ctx_load replaces the engine when it needs a larger one
     L2O_TRY(hipMemsetAsync(e->d_scratch, 0, sizeof(unsigned long long), e->stream));
@@ -1549,7 +1563,7 @@ int logo2opt_time_sweep(logo2opt_ctx *ctx, const uint32_t *route, uint32_t sweep
     logo2opt_engine *e = ctx->e;
     if (hipSetDevice(e->device) != hipSuccess) return LOGO2OPT_EDEVICE;
     logo2opt_job job{};
-    int rc = ctx_load(ctx, route, job);
+    int rc = ctx_load(ctx, route, job, true);
     if (rc) return rc;
     e = ctx->e;  // ctx_load replaces the engine when it needs a larger one
     rc = rebuild_lists(e);

@@ -138,6 +138,23 @@ __device__ __forceinline__ unsigned long long uniform_u64(unsigned long long v)
     return ((unsigned long long)hi << 32) | lo;
 }
 
+// The key of a known candidate (edges e-1 -> e of positions i2 and j2) on the
+// tour after the move (i, J): r' = r[i..J-1] ++ r[i-1..0] ++ r[n-1..J].  An
+// edge keeps its two cities unless it is one of the two removed ones; its
+// direction is reversed outside [i, J-1].  Two edges of the same side keep
+// their relative direction, so the candidate keeps its gain at the mapped
+// positions; two edges of different sides would reconnect the other way.
+// L2O_SENTINEL if the candidate is gone.
+__device__ __forceinline__ unsigned long long remap_key(unsigned long long key, uint32_t i, uint32_t J, uint32_t n)
+{
+    const uint32_t i2 = (uint32_t)(key >> 20) & 0xFFFFFu, j2 = (uint32_t)key & 0xFFFFFu;
+    const bool in1 = i2 > i && i2 < J, in2 = j2 > i && j2 < J;
+    auto to = [&](uint32_t e) { return e > i && e < J ? e - i : e < i ? J - e : n + J - e; };
+    const uint32_t e1 = to(i2), e2 = to(j2);
+    if (key == L2O_SENTINEL || in1 != in2 || i2 == i || i2 == J || j2 == i || j2 == J) return L2O_SENTINEL;
+    return (key & ~((1ull << 40) - 1)) | ((unsigned long long)min(e1, e2) << 20) | max(e1, e2);
+}
+
 // point records in global memory (address space 1: the pointers come from
 // the instance record, so the space is stated for global_* instructions)
 typedef __attribute__((address_space(1))) l2o_pt gpt;
@@ -533,7 +550,7 @@ __device__ __forceinline__ void sweep_item(const l2o_sweep_item it, l2o_inst *__
     };
     // (PRUNE: read after the row test below, by waves with a live block only;
     // the row test then uses cap = -1, a valid, looser threshold)
-    if constexpr (!PRUNE) {
+    {
         const unsigned long long g = key_now();
         if (g != L2O_SENTINEL && key_gain(g) < cap) set_cap(key_gain(g));
     }
@@ -561,8 +578,6 @@ __device__ __forceinline__ void sweep_item(const l2o_sweep_item it, l2o_inst *__
             if (keep && r0 + UF <= t_end) t0_stage(lane, qx, qy, qw);
             __builtin_amdgcn_wave_barrier();
         }
-        const unsigned long long g = key_now();
-        if (g != L2O_SENTINEL && key_gain(g) < cap) set_cap(key_gain(g));
     }
     unsigned long long lbest = L2O_SENTINEL;
     unsigned long long published = L2O_SENTINEL;
@@ -598,6 +613,7 @@ __device__ __forceinline__ void sweep_item(const l2o_sweep_item it, l2o_inst *__
                             const uint32_t j = (uint32_t)(bl + k + 1);
                             const unsigned long long key = make_key(gain, i, j);
                             lbest = key < lbest ? key : lbest;
+                            atomicMin(&in->pool[(i * 0x9E3779B1u) >> 26], key);
                         }
                     }
                 }
@@ -891,6 +907,11 @@ __global__ __launch_bounds__(L2O_APPLY_THREADS) void k_apply(const l2o_apply_ite
     }
     l2o_pt p[PER], q[PER];
     uint32_t rid[PER];
+    // wave 0: the pool entries on the new tour (stored by the last chunk)
+    static_assert(L2O_POOL == 64, "one lane per pool entry");
+    unsigned long long *const pool = in->pool;
+    unsigned long long pk = L2O_SENTINEL;
+    if (threadIdx.x < L2O_POOL) pk = pool[threadIdx.x];
     // the far ends of the two new edges, loaded with the rest (one round trip)
     const l2o_pt endJ = ld_pt(P, J), endJ1 = ld_pt(P, J - 1);
 #pragma unroll
@@ -916,6 +937,9 @@ __global__ __launch_bounds__(L2O_APPLY_THREADS) void k_apply(const l2o_apply_ite
         st_pt(Pn, k, r);
         Rn[k] = rid[e];
     }
+    pk = remap_key(pk, i, J, n);
+    const unsigned long long pmin = wave_min_u64(pk);
+    asm volatile("" ::"s"(pmin));  // the pool loads have returned before the barrier
     // Every wave of the workgroup has read key, parity and its sources once
     // all are past the barrier (each loaded value feeds a store issued before
     // it), so the last chunk to count may commit the move.  No memory fence:
@@ -925,10 +949,15 @@ __global__ __launch_bounds__(L2O_APPLY_THREADS) void k_apply(const l2o_apply_ite
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    if (threadIdx.x == 0) {
+    if (threadIdx.x < 64) {
         const uint32_t nch = (n + L2O_APPLY_CHUNK - 1) / L2O_APPLY_CHUNK;
-        const uint32_t prev = atomicAdd(&in->apply_done, 1u);
-        if (prev == nch - 1) {  // last chunk of this instance: commit the move
+        uint32_t prev = 0;
+        if (threadIdx.x == 0) prev = atomicAdd(&in->apply_done, 1u);
+        prev = (uint32_t)__builtin_amdgcn_readfirstlane((int)prev);
+        if (prev != nch - 1) return;
+        // last chunk of this instance: commit the move
+        pool[threadIdx.x] = pk;
+        if (threadIdx.x == 0) {
             in->apply_done = 0;
             in->length += (unsigned long long)(long long)gain;
             if (in->moves < in->log_cap) {
@@ -941,7 +970,7 @@ __global__ __launch_bounds__(L2O_APPLY_THREADS) void k_apply(const l2o_apply_ite
             in->moves += 1;
             in->sweeps += 1;
             in->parity = par ^ 1;
-            in->key = L2O_SENTINEL;
+            in->key = pmin;
         }
     }
 }

@@ -48,7 +48,8 @@ constexpr size_t NA_OFF_TOUR = NA_OFF_COORDS + al256(sizeof(logo2opt_city_coords
 constexpr size_t NA_OFF_PTS = NA_OFF_TOUR + al256(sizeof(uint32_t) * NA_MAX_N);
 constexpr size_t NA_OFF_ITEMS = NA_OFF_PTS + al256(sizeof(l2o_pt) * NA_MAX_N);
 constexpr size_t NA_OFF_INST = NA_OFF_ITEMS + al256(sizeof(l2o_sweep_item) * NA_MAX_ITEMS);
-constexpr size_t NA_BYTES = NA_OFF_INST + al256(sizeof(l2o_inst));
+constexpr size_t NA_OFF_POOL = NA_OFF_INST + al256(sizeof(l2o_inst));  // written by the sweep, not read here
+constexpr size_t NA_BYTES = NA_OFF_POOL + al256(sizeof(unsigned long long) * L2O_POOL);
 
 }  // namespace
 
@@ -161,6 +162,7 @@ extern "C" int logo2opt_step_noalloc(int device, uint32_t n, const logo2opt_city
     std::memset(&in, 0, sizeof(in));
     in.pts[0] = in.pts[1] = (l2o_pt *)(base + NA_OFF_PTS);
     in.tour[0] = in.tour[1] = (uint32_t *)(base + NA_OFF_TOUR);
+    in.pool = (unsigned long long *)(base + NA_OFF_POOL);
     in.n = n;
     // bound on |exact gain - FP32 estimate| for the coordinate span (the
     // engine's formula, l2o_engine.hip check_coords)

@@ -71,6 +71,7 @@ struct l2o_inst {
     float est_add;
     uint32_t qshift;      // tier 0: coordinates >> qshift fit in 8 bits
     unsigned long long stop_below;  // ILS: done once best_length < stop_below (0: never)
+    unsigned long long *pool;       // L2O_POOL keys of known improving moves (L2O_SENTINEL: none)
     // ---- dynamic
     uint32_t phase;
     uint32_t parity;
@@ -101,6 +102,10 @@ struct l2o_apply_item {
     uint32_t chunk;
 };
 
+// Keys of improving candidates the sweeps have evaluated exactly, bucketed by
+// position.  k_apply carries them over to the next tour, so the next sweep
+// starts with the best of them as its key.  All L2O_SENTINEL at a local optimum.
+#define L2O_POOL 64
 #define L2O_MAX_GROUPS 32  // distinct sweep tile shapes in one engine step
 #define L2O_APPLY_CHUNK 1024
 #define L2O_APPLY_THREADS 256
