@@ -15,7 +15,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 LIB = os.path.join(HERE, "liblogo2opt.so")
-SOURCES = ["csrc/l2o_kernels.hip", "csrc/l2o_engine.hip", "csrc/l2o_workload.cpp", "csrc/l2o_server.cpp",
+SOURCES = ["csrc/l2o_kernels.hip", "csrc/l2o_sweep.hip", "csrc/l2o_engine.hip", "csrc/l2o_workload.cpp", "csrc/l2o_server.cpp",
            "csrc/l2o_tsplib.cpp", "csrc/l2o_noalloc.hip"]
 ARCH = os.environ.get("LOGO2OPT_ARCH", "gfx950")
 
@@ -35,6 +35,9 @@ def build(verbose=False):
         "-ffp-contract=off",
         # packed FP32 VALU forms are kept out of the code object
         "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+        # matrix results in VGPRs: the sweep reads every one of them with VALU
+        # instructions (in AGPRs each costs a copy: 2.7e13 -> 4.4e13 tests/s)
+        "-mllvm", "-amdgpu-mfma-vgpr-form=1",
         "-Wall", "-Wno-unused-command-line-argument",
         "-I", os.path.join(ROOT, "include"),
         "-o", LIB + ".tmp",

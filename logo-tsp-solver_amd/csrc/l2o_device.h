@@ -1,0 +1,140 @@
+// l2o_device.h -- device helpers shared by the kernels.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include "l2o_launch.h"
+#include "l2o_state.h"
+
+namespace l2o {
+
+// ---------------------------------------------------------------------------
+// exact metric length of the edge P1 -> P2 (metric_dist in l2o_launch.h)
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ int exact_dist(int x1, int y1, int x2, int y2, uint32_t metric)
+{
+    // coordinates lie in [0, 2^22): the differences and s are exact
+    const long long dx = (long long)(x1 - x2);
+    const long long dy = (long long)(y1 - y2);
+    return metric_dist(dx * dx + dy * dy, metric);
+}
+
+// FP32 estimate of the metric length: sqrt(s) * scale + add, with scale = 1,
+// add = 0 for EUC_2D (D = nint(d)), scale = 1, add = 1/2 for CEIL_2D (D in
+// [d, d+1)) and scale = 1/sqrt(10), add = 1/2 for ATT; |D - estimate| <= 1/2
+// plus the FP32 error, which the instance's slack bounds.  The integer
+// differences convert to FP32 exactly.
+__device__ __forceinline__ float est_dist(int x1, int y1, int x2, int y2, float scale, float add)
+{
+    const float dx = (float)(x1 - x2), dy = (float)(y1 - y2);
+    return __builtin_fmaf(__builtin_amdgcn_sqrtf(__builtin_fmaf(dx, dx, dy * dy)), scale, add);
+}
+
+__device__ __forceinline__ unsigned long long make_key(int gain, uint32_t i, uint32_t j)
+{
+    return ((unsigned long long)(gain + L2O_KEY_GAIN_BIAS) << 40) |
+           ((unsigned long long)i << 20) | (unsigned long long)j;
+}
+
+__device__ __forceinline__ int key_gain(unsigned long long key)
+{
+    return (int)((long long)(key >> 40) - L2O_KEY_GAIN_BIAS);
+}
+
+// one step of a 64-bit minimum scan over the lanes: DPP CTRL moves both
+// halves; lanes the move leaves without a source keep their own value
+template <int CTRL, int ROWS>
+__device__ __forceinline__ unsigned long long dpp_min_u64(unsigned long long v)
+{
+    const int lo = (int)(uint32_t)v, hi = (int)(uint32_t)(v >> 32);
+    const uint32_t l2 = (uint32_t)__builtin_amdgcn_update_dpp(lo, lo, CTRL, ROWS, 0xF, false);
+    const uint32_t h2 = (uint32_t)__builtin_amdgcn_update_dpp(hi, hi, CTRL, ROWS, 0xF, false);
+    const unsigned long long o = ((unsigned long long)h2 << 32) | l2;
+    return o < v ? o : v;
+}
+
+// minimum over the 64 lanes, returned wave-uniform (in SGPRs): row_shr 1, 2,
+// 4, 8 within each row of 16 lanes, then row_bcast 15 and 31 carry the rows
+// below upwards, so lane 63 ends with the minimum (VALU only, no LDS)
+__device__ __forceinline__ unsigned long long wave_min_u64(unsigned long long v)
+{
+    v = dpp_min_u64<0x111, 0xF>(v);
+    v = dpp_min_u64<0x112, 0xF>(v);
+    v = dpp_min_u64<0x114, 0xF>(v);
+    v = dpp_min_u64<0x118, 0xF>(v);
+    v = dpp_min_u64<0x142, 0xA>(v);
+    v = dpp_min_u64<0x143, 0xC>(v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, 63);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), 63);
+    return ((unsigned long long)hi << 32) | lo;
+}
+
+// a wave-uniform 64-bit value moved to SGPRs (readfirstlane returns int: each
+// half is taken as unsigned before it is widened)
+__device__ __forceinline__ unsigned long long uniform_u64(unsigned long long v)
+{
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+    return ((unsigned long long)hi << 32) | lo;
+}
+
+// The key of a known candidate (edges e-1 -> e of positions i2 and j2) on the
+// tour after the move (i, J): r' = r[i..J-1] ++ r[i-1..0] ++ r[n-1..J].  An
+// edge keeps its two cities unless it is one of the two removed ones; its
+// direction is reversed outside [i, J-1].  Two edges of the same side keep
+// their relative direction, so the candidate keeps its gain at the mapped
+// positions; two edges of different sides would reconnect the other way.
+// L2O_SENTINEL if the candidate is gone.
+__device__ __forceinline__ unsigned long long remap_key(unsigned long long key, uint32_t i, uint32_t J, uint32_t n)
+{
+    const uint32_t i2 = (uint32_t)(key >> 20) & 0xFFFFFu, j2 = (uint32_t)key & 0xFFFFFu;
+    const bool in1 = i2 > i && i2 < J, in2 = j2 > i && j2 < J;
+    auto to = [&](uint32_t e) { return e > i && e < J ? e - i : e < i ? J - e : n + J - e; };
+    const uint32_t e1 = to(i2), e2 = to(j2);
+    if (key == L2O_SENTINEL || in1 != in2 || i2 == i || i2 == J || j2 == i || j2 == J) return L2O_SENTINEL;
+    return (key & ~((1ull << 40) - 1)) | ((unsigned long long)min(e1, e2) << 20) | max(e1, e2);
+}
+
+// point records in global memory (address space 1: the pointers come from
+// the instance record, so the space is stated for global_* instructions)
+typedef __attribute__((address_space(1))) l2o_pt gpt;
+typedef __attribute__((address_space(1))) uint32_t gu32;
+
+__device__ __forceinline__ l2o_pt ld_pt(const gpt *P, uint32_t k)
+{
+    l2o_pt r;
+    r.x = P[k].x;
+    r.y = P[k].y;
+    r.d = P[k].d;
+    r.w = P[k].w;
+    return r;
+}
+
+__device__ __forceinline__ void st_pt(gpt *P, uint32_t k, const l2o_pt r)
+{
+    P[k].x = r.x;
+    P[k].y = r.y;
+    P[k].d = r.d;
+    P[k].w = r.w;
+}
+
+__device__ __forceinline__ unsigned wave_sum_u32(unsigned v)
+{
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+    return v;
+}
+
+// maximum over the 64 lanes, returned wave-uniform: the scan pattern of
+// wave_min_u64 with max, where a lane that a shift leaves without a source keeps its value
+__device__ __forceinline__ int wave_max_i32(int v)
+{
+    v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x111, 0xF, 0xF, false));
+    v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x112, 0xF, 0xF, false));
+    v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x114, 0xF, 0xF, false));
+    v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x118, 0xF, 0xF, false));
+    v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x142, 0xA, 0xF, false));
+    v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x143, 0xC, 0xF, false));
+    return __builtin_amdgcn_readlane(v, 63);
+}
+
+}  // namespace l2o

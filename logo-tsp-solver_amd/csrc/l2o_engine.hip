@@ -382,9 +382,12 @@ int upload_instance(logo2opt_engine *e, int32_t id, const uint32_t *route, uint3
     in.est_scale = s.job.metric == l2o::L2O_ATT ? (float)(1.0 / std::sqrt(10.0)) : 1.0f;
     in.est_add = s.job.metric == l2o::L2O_EUC_2D ? 0.0f : 0.5f;
     {
-        int32_t m = 0;
-        for (const int32_t v : s.xy) m = std::max(m, v);
-        in.qshift = l2o::tier0_shift((uint32_t)m);
+        int32_t mx = 0, my = 0;
+        for (size_t k = 0; k < s.xy.size(); k += 2) {
+            mx = std::max(mx, s.xy[k]);
+            my = std::max(my, s.xy[k + 1]);
+        }
+        l2o::set_quant(in, mx, my);
     }
     in.stop_below = s.job.ils_rounds ? s.job.stop_below : 0;
     in.phase = phase;
@@ -407,7 +410,7 @@ int upload_instance(logo2opt_engine *e, int32_t id, const uint32_t *route, uint3
         pts[k].x = xy[2 * c];
         pts[k].y = xy[2 * c + 1];
         pts[k].d = (int32_t)d;
-        pts[k].w = l2o::ceil_sqrtg((int32_t)d, l2o::tier1_g(s.job.metric));
+        pts[k].w = l2o::quant_xy(in.qs, in.qox, in.qoy, xy[2 * c], xy[2 * c + 1]);
     }
     in.length = L;
     L2O_TRY(hipMemcpyAsync(in.pts[0], pts.data(), 16ull * n, hipMemcpyHostToDevice, e->stream));
@@ -430,15 +433,6 @@ void drop_graph(logo2opt_engine *e)
 // it the pruned sweep measured 4-9% slower (per-wave fixed costs dominate),
 // from 16,000 on it wins (1.04x there, 1.2x at 24,000, 1.6x at 33,810)
 #define L2O_PRUNE_AUTO_MIN_N 16000u
-// Pruned instances below this many cities send their live blocks through
-// tier 0; larger ones, whose live blocks lie close to the columns and mostly
-// pass it, go straight to tier 1 (measured: 33,810 and 100,000 cities 3-5%
-// faster without tier 0, the 2,048-instance batch of 100-5,000 cities 7%
-// faster with it)
-#ifndef L2O_PRUNE_T0_MAX_N
-#define L2O_PRUNE_T0_MAX_N 16000u
-#endif
-
 #ifndef L2O_DIAG_WEIGHT
 #define L2O_DIAG_WEIGHT 4
 #endif
@@ -488,7 +482,7 @@ int rebuild_lists(logo2opt_engine *e)
         const uint32_t n = s.n;
         const sweep_cfg c = cfg_for(n, table);
         const bool pr = e->prune == LOGO2OPT_PRUNE_ALL || (e->prune == LOGO2OPT_PRUNE_AUTO && n >= L2O_PRUNE_AUTO_MIN_N);
-        const int mode = !pr ? l2o::L2O_SWEEP_FULL : n < L2O_PRUNE_T0_MAX_N ? l2o::L2O_SWEEP_PRUNE : l2o::L2O_SWEEP_PRUNE_T1;
+        const int mode = pr ? l2o::L2O_SWEEP_PRUNE : l2o::L2O_SWEEP_FULL;
         auto &v = by_cfg[std::make_tuple(c.k, c.t, c.waves, mode)];
         // rows a <= n-4; the first tile of a row block starts at the
         // diagonal, b0 = a0 + 2
@@ -545,9 +539,9 @@ int rebuild_lists(logo2opt_engine *e)
         for (uint64_t w : work) total += w;
         for (size_t q = 0; q < idx.size(); ++q) {
             const l2o_sweep_item it = v[idx[q]];
-            if (c.t >= 4 * L2O_TAIL_DIV && done >= total - total / L2O_TAIL_SPLIT) {
-                const uint32_t r4 = (uint32_t)c.t / L2O_TAIL_DIV;
-                for (uint32_t r = 0; r < it.rows; r += r4) sorted.push_back({it.inst, it.a0 + r, it.b0, r4});
+            if (c.t > 32 && done >= total - total / L2O_TAIL_SPLIT) {
+                const uint32_t r4 = ((uint32_t)c.t / L2O_TAIL_DIV + 31u) & ~31u;
+                for (uint32_t r = 0; r < it.rows; r += r4) sorted.push_back({it.inst, it.a0 + r, it.b0, std::min(r4, it.rows - r)});
             } else {
                 sorted.push_back(it);
             }

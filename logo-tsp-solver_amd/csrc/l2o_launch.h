@@ -2,6 +2,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <math.h>
+
 #include "l2o_state.h"
 
 namespace l2o {
@@ -31,57 +33,62 @@ __host__ __device__ inline int32_t metric_dist(long long s, uint32_t metric)
     return (int32_t)(m + (s > f * m * m + e * m ? 1 : 0));
 }
 
-// Tier-1 factor g of the sweep's integer bound.  |dx| + |dy| <= sqrt(2) d for
-// the Euclidean length d, and d < D + 1/2 (EUC_2D), d <= D (CEIL_2D),
-// d <= sqrt(10) D (ATT), so a candidate with gain <= cap has
-//   L1(a,b) + L1(a+1,b+1) <= sqrt(g) (cap + 1 + D[a+1] + D[b+1])
-// with g = 2, 2, 20.
-__host__ __device__ inline int32_t tier1_g(uint32_t metric) { return metric == L2O_ATT ? 20 : 2; }
-
-// ceil(sqrt(g) * d) for 0 <= d < 2^24, g in {2, 20}.  Neither is a square, so
-// for d >= 1 sqrt(g) d is irrational and the ceiling is isqrt(g d^2) + 1;
-// isqrt is exact after the correction.
-__host__ __device__ inline int32_t ceil_sqrtg(int32_t d, int32_t g)
+// Quantised geometry of the sweep's matrix test (see l2o_sweep.hip).  A city
+// (x, y) becomes X and Y, x qs + qox and y qs + qoy rounded to whole numbers in
+// [-L2O_QR, L2O_QR]; an edge of length D becomes E = ceil(D qk + qm) <= L2O_QE,
+// where qk >= qs kappa (kappa = sqrt(10) for ATT, else 1) and qm covers half
+// of the metric's rounding (d < D + 1/2 for EUC_2D) and of the rounding of the
+// coordinates.  With these limits every partial sum of the test is a whole
+// number below 2^24, exact in FP32 in any order.
+#define L2O_QR 640
+#define L2O_QE 1830
+__host__ inline void set_quant(l2o_inst &in, double span_x, double span_y)
 {
-    if (d <= 0) return 0;
-    const long long s = (long long)g * d * d;
-    long long k = (long long)sqrt((double)s);
-    if (k * k > s) k -= 1;
-    else if ((k + 1) * (k + 1) <= s) k += 1;
-    return (int32_t)(k + 1);
+    const double half = 0.5 * (span_x > span_y ? span_x : span_y);
+    in.qs = (float)(half * 4.0 <= 639.0 ? 4.0 : 639.0 / half);
+    in.qox = (float)(-0.5 * span_x * (double)in.qs);
+    in.qoy = (float)(-0.5 * span_y * (double)in.qs);
+    const double kappa = in.metric == L2O_ATT ? sqrt(10.0) : 1.0;
+    in.qk = nextafterf((float)((double)in.qs * kappa), 1e30f);
+    in.qm = (float)(1.02 + (in.metric == L2O_EUC_2D ? 0.5 * (double)in.qs : 0.0));
 }
 
-__host__ __device__ inline int32_t ceil_sqrt2(int32_t d) { return ceil_sqrtg(d, 2); }
-
-// The sweep's coarse test (tier 0) works on coordinates >> qshift, which must
-// fit in 8 bits: the smallest shift that brings the largest translated
-// coordinate (below 2^22) under 256.
-__host__ __device__ inline uint32_t tier0_shift(uint32_t max_coord)
+// FP16 bits of a whole number |v| <= 2048 given as a float (exact)
+__host__ __device__ inline uint32_t f16_of_whole(float v)
 {
-    uint32_t s = 0;
-    while ((max_coord >> s) > 255u) ++s;
-    return s;
+    union {
+        float f;
+        uint32_t u;
+    } b;
+    b.f = v;
+    const uint32_t m = b.u & 0x7FFFFFFFu;
+    return ((b.u >> 16) & 0x8000u) | (m ? (m >> 13) - (112u << 10) : 0u);
 }
 
-// Sweep tile shape: each workgroup has `waves` wave64s, each lane owns `k`
-// adjacent candidate columns for `t` rows (the last lane of a wave one fewer:
-// its last column is the next wave's first).  A workgroup covers
-// waves*(64k-1) columns.
+// l2o_pt.w of a city: X and Y as a pair of FP16 numbers (rounded to the nearest
+// whole number by truncation of a positive one)
+__host__ __device__ inline int32_t quant_xy(float qs, float qox, float qoy, int32_t x, int32_t y)
+{
+    const float fx = (float)x * qs + qox, fy = (float)y * qs + qoy;
+    const int32_t X = (int32_t)(fx + 1024.5f) - 1024, Y = (int32_t)(fy + 1024.5f) - 1024;
+    return (int32_t)(f16_of_whole((float)X) | (f16_of_whole((float)Y) << 16));
+}
+
+// Sweep tile shape: each workgroup has `waves` wave64s on the same `t` rows,
+// each wave with 64 k columns of its own (2 k matrix tiles of 32 columns).
 struct sweep_cfg {
     int k;
     int t;
     int waves;
-    int cols() const { return waves * (64 * k - 1); }
+    int cols() const { return waves * 64 * k; }
 };
 
 bool sweep_cfg_supported(const sweep_cfg &c);
 // compiled shapes: fills up to cap rows {k, t, waves}, returns the total count
 int sweep_shapes(int (*out)[3], int cap);
-// Sweep variants (same results): the full sweep (every block of rows through
-// tier 0), and row pruning, which first skips the blocks of rows a
-// bounding-box bound rules out and sends the rest through tier 0
-// (L2O_SWEEP_PRUNE) or straight to tier 1 (L2O_SWEEP_PRUNE_T1)
-enum { L2O_SWEEP_FULL = 0, L2O_SWEEP_PRUNE = 1, L2O_SWEEP_PRUNE_T1 = 2 };
+// Sweep variants (same results): every pair of tiles through the matrix test,
+// or only those that a bounding-box bound does not rule out
+enum { L2O_SWEEP_FULL = 0, L2O_SWEEP_PRUNE = 1 };
 // one workgroup per item, of the variant `mode`
 hipError_t launch_sweep(const sweep_cfg &cfg, const l2o_sweep_item *items, uint32_t nitems,
                         l2o_inst *insts, hipStream_t stream, int mode = L2O_SWEEP_FULL);

@@ -30,7 +30,7 @@ constexpr uint32_t NA_MAX_N = LOGO2OPT_NOALLOC_MAX_N;
 // one fixed tile shape (4 columns per lane, 128 rows, one wave): the work
 // list's length then has the closed bound below, and no tuning table is read
 constexpr int NA_K = 4, NA_T = 128, NA_W = 1;
-constexpr uint32_t NA_COLS = NA_W * (64 * NA_K - 1);
+constexpr uint32_t NA_COLS = NA_W * 64 * NA_K;
 
 // items of a sweep of n cities: row blocks a0 = 0, T, 2T, ... (a0 + 4 <= n),
 // each with floor((n - 4 - a0) / COLS) + 1 column tiles
@@ -76,7 +76,8 @@ __global__ __launch_bounds__(256) void k_na_points(unsigned char *__restrict__ b
     p.x = x;
     p.y = y;
     p.d = l2o::metric_dist(dx * dx + dy * dy, metric);
-    p.w = l2o::ceil_sqrtg(p.d, l2o::tier1_g(metric));
+    const l2o_inst *in = (const l2o_inst *)(base + NA_OFF_INST);
+    p.w = l2o::quant_xy(in->qs, in->qox, in->qoy, x, y);
     P[k] = p;
 }
 
@@ -172,7 +173,7 @@ extern "C" int logo2opt_step_noalloc(int device, uint32_t n, const logo2opt_city
     in.group_lead = L2O_NO_GROUP;
     in.est_scale = metric == LOGO2OPT_METRIC_ATT ? (float)(1.0 / std::sqrt(10.0)) : 1.0f;
     in.est_add = metric == LOGO2OPT_METRIC_EUC_2D ? 0.0f : 0.5f;
-    in.qshift = l2o::tier0_shift((uint32_t)std::fmax(mxx - mnx, mxy - mny));
+    l2o::set_quant(in, mxx - mnx, mxy - mny);
     in.phase = L2O_LO;
     in.key = L2O_SENTINEL;
 
@@ -190,7 +191,7 @@ extern "C" int logo2opt_step_noalloc(int device, uint32_t n, const logo2opt_city
     hipLaunchKernelGGL(k_na_items, dim3((rblocks + 63) / 64), dim3(64), 0, st, base, n);
     NA_TRY(hipGetLastError());
     NA_TRY(l2o::launch_sweep(l2o::sweep_cfg{NA_K, NA_T, NA_W}, (const l2o_sweep_item *)(base + NA_OFF_ITEMS),
-                             na_items(n), (l2o_inst *)(base + NA_OFF_INST), st, false));
+                             na_items(n), (l2o_inst *)(base + NA_OFF_INST), st, l2o::L2O_SWEEP_FULL));
     unsigned long long key = L2O_SENTINEL;
     NA_TRY(hipMemcpyAsync(&key, base + NA_OFF_INST + offsetof(l2o_inst, key), sizeof(key), hipMemcpyDeviceToHost,
                           st));

@@ -6,8 +6,8 @@
 //                                     coordinates shifted into [0, 2^22),
 //                                     D[k] = exact metric length of the edge
 //                                     P[k-1] -> P[k] (EUC_2D, CEIL_2D or ATT),
-//                                     D[0] the closing edge,
-//                                     W[k] = ceil(sqrt(g) D[k]), g = 2 or 20
+//                                     D[0] the closing edge, W[k] the
+//                                     quantised coordinates of P[k]
 //   tour[2][n] uint32                 city ids in the same order (ping-pong)
 //   bpts[n], btour[n]                 best tour of an ILS run
 //   log[log_cap]                      applied moves {i, J, gain}
@@ -39,7 +39,7 @@ enum l2o_phase : uint32_t {
 struct __attribute__((aligned(16))) l2o_pt {
     int32_t x, y;  // coordinates, 0 <= x, y < 2^22
     int32_t d;     // exact metric length of the edge into this point
-    int32_t w;     // ceil(sqrt(g) * d), the edge's tier-1 sweep bound
+    int32_t w;     // the point's quantised coordinates (quant_xy in l2o_launch.h)
 };
 
 struct l2o_move {
@@ -69,7 +69,8 @@ struct l2o_inst {
     uint32_t kick_src;    // slot whose best tour the next kick starts from
     float est_scale;      // FP32 tier: D ~ sqrt(s) * est_scale + est_add
     float est_add;
-    uint32_t qshift;      // tier 0: coordinates >> qshift fit in 8 bits
+    float qs, qox, qoy;   // matrix test: X ~ x qs + qox, Y ~ y qs + qoy,
+    float qk, qm;         // and E = ceil(D qk + qm) (set_quant in l2o_launch.h)
     unsigned long long stop_below;  // ILS: done once best_length < stop_below (0: never)
     unsigned long long *pool;       // L2O_POOL keys of known improving moves (L2O_SENTINEL: none)
     // ---- dynamic

@@ -1,0 +1,528 @@
+// l2o_sweep.hip -- the sweep: every 2-opt candidate of a tour through a matrix
+// test, the survivors through an FP32 estimate and the exact length.
+//
+// Candidates.  With a = i-1 and b = J-1 a candidate is a pair
+// 0 <= a, a+2 <= b <= n-2 with exact gain
+//     G = n(a,b) + n(a+1,b+1) - D[a+1] - D[b+1],
+// n(x,y) the exact metric length of P[x] -> P[y] and D[k] = n(k-1,k).  The
+// sweep returns the lexicographic minimum of (G, i, J) over G < 0 (the move the
+// reference's strict-'<' scan keeps).
+//
+// Matrix test.  Take row a as the 4-vector u = (x_a, y_a, x_a+1, y_a+1) and
+// column b as v likewise.  The new edges have Euclidean lengths d1, d2 with
+// d1^2 + d2^2 = |u - v|^2, so |u - v| <= d1 + d2, and G <= cap needs
+// d1 + d2 <= kappa (D[a+1] + D[b+1] + cap) + h (h = 1 for EUC_2D's two
+// roundings, kappa = sqrt(10) for ATT).  With the coordinates quantised to
+// whole numbers X = rint(x s + o) the vector |U - V| is at most 2 + s |u - v|
+// (each of four components is off by at most 1), so with
+//     E = ceil(s kappa D + s h / 2 + 1),   C = -2 floor(s kappa |cap| / 2)
+// a candidate that can still win has |U - V|^2 <= (E_a + E_b + C)^2.  Both
+// sides expand into an inner product of a row record and a column record
+// (the cap goes in half to each side, E' = E + C/2, N = |U|^2 - E'^2):
+//     |U - V|^2 - (E'_a + E'_b)^2 - 1
+//        = -2 U.V - 2 E'_a E'_b + N_a + N_b - 1 < 0,
+// 5 products and N split into N = 2048 Nh + Nl on each side: 10 of the 16
+// terms of v_mfma_f32_32x32x16_f16.  Every operand is a whole number of at
+// most 11 bits, exact in FP16, and every partial sum stays below 2^24
+// (L2O_QR, L2O_QE in l2o_launch.h), exact in FP32: the test has no rounding.
+// One matrix instruction tests 32 x 32 candidates; 16 results per lane are
+// combined by their sign bits (v_or3_b32, two results an instruction), so a
+// candidate costs about 0.7 VALU instructions; the 8-bit v_sad_u8 bound it
+// replaces took 2.2.
+//
+// What bounds it.  A tile of 1,024 candidates holds the matrix unit for 32
+// cycles and needs at least 8 v_or3 (32 cycles of VALU issue); the two overlap
+// only in part (a loop of nothing else: 46 cycles a tile, 5.0e13 candidates/s).
+// Measured with one MI355X, whole steps: 100,000 cities 270 -> 145 us (3.4e13
+// candidates/s), 33,810 clustered 57 -> 33 us, 7,397 20 -> 11.6 us (two
+// launches' latency).  Matrix results kept in AGPRs, as the compiler prefers,
+// cost a copy each: 2.7e13 instead of 4.4e13 tests/s (-amdgpu-mfma-vgpr-form).
+//
+// A row with E_a + C + max E_b < 0 (and a column likewise) has no candidate
+// left: its record is replaced by one that never passes.  So |E'| <= L2O_QE for
+// the others, and (E'_a + E'_b)^2 of a pair with a negative sum, which passes
+// although it cannot win, stays as small as the largest legitimate one.
+//
+// Survivors.  The 32 sign bits of a pair of tiles are stored in LDS per lane;
+// every row block the wave compacts them into full waves of candidates, which
+// load their four points, take the FP32 estimate and, if that passes, the exact
+// length (FP64 square root and integer fix-up).  Keys go to the instance's
+// shared key by atomicMin; the result is exact and independent of wave order.
+#include <hip/hip_runtime.h>
+
+#include "l2o_device.h"
+
+namespace l2o {
+
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+typedef float float16v __attribute__((ext_vector_type(16)));
+
+__device__ __forceinline__ uint32_t pk16(float a, float b)
+{
+    return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a, b));
+}
+
+// the wave's lanes below this one among `m`
+__device__ __forceinline__ int lanes_below(unsigned long long m)
+{
+    return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
+// quantised edge k -> k+1: {X, Y} and {X1, Y1} as FP16 pairs (l2o_pt.w of its
+// ends), U = |(X, Y, X1, Y1)|^2 and E of its length (l2o_pt.d of k+1)
+struct qedge {
+    uint32_t p0, p1;
+    float u, e;
+};
+
+__device__ __forceinline__ qedge quant_edge(uint32_t w0, uint32_t w1, uint32_t d1, float qk, float qm)
+{
+    const half2v a = __builtin_bit_cast(half2v, w0), b = __builtin_bit_cast(half2v, w1);
+    qedge r;
+    r.p0 = w0;
+    r.p1 = w1;
+    r.u = __builtin_amdgcn_fdot2(a, a, __builtin_amdgcn_fdot2(b, b, 0.0f, false), false);
+    r.e = __builtin_ceilf(__builtin_fmaf((float)(int)d1, qk, qm));
+    return r;
+}
+
+// E' and the limbs of N of an edge; an edge without a candidate (alive false)
+// gets an Nh that no other terms can outweigh
+struct qterms {
+    float e, nh, nl;
+};
+__device__ __forceinline__ qterms edge_terms(const qedge &q, float hc, bool alive)
+{
+    qterms t;
+    t.e = q.e - hc;
+    const float nn = __builtin_fmaf(-t.e, t.e, q.u);
+    t.nh = __builtin_floorf(nn * (1.0f / 2048.0f));
+    t.nl = __builtin_fmaf(t.nh, -2048.0f, nn);
+    t.nh = alive ? t.nh : 30000.0f;
+    return t;
+}
+
+// A operand (rows), 16 FP16 terms: lanes 0..31 {X, Y, X1, Y1, E', 1, Nl, Nh},
+// lanes 32..63 the same {2048, 1, 0, 0, 0, 0, 0, 0} for every row
+__device__ __forceinline__ uint4 row_record(const qedge &q, const qterms &t)
+{
+    return make_uint4(q.p0, q.p1, pk16(t.e, 1.0f), pk16(t.nl, t.nh));
+}
+__device__ __forceinline__ uint4 row_const() { return make_uint4(pk16(2048.0f, 1.0f), 0u, 0u, 0u); }
+
+// B operand (columns): lanes 0..31 {-2X, -2Y, -2X1, -2Y1, -2E', Nl, 1, 2048},
+// lanes 32..63 {Nh, -1, any six finite numbers}
+__device__ __forceinline__ uint4 col_record(const qedge &q, const qterms &t)
+{
+    const half2v m2 = {(_Float16)-2.0f, (_Float16)-2.0f};
+    return make_uint4(__builtin_bit_cast(uint32_t, __builtin_bit_cast(half2v, q.p0) * m2),
+                      __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2v, q.p1) * m2),
+                      pk16(-2.0f * t.e, t.nl), pk16(1.0f, 2048.0f));
+}
+__device__ __forceinline__ uint32_t col_upper(const qterms &t) { return pk16(t.nh, -1.0f); }
+
+// maximum over each half of the wave, in lanes 31 and 63 (the others hold partial ones)
+__device__ __forceinline__ float half_max_f32(float v)
+{
+    auto step = [](float x, int y) { return __builtin_fmaxf(x, __int_as_float(y)); };
+    v = step(v, __builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), 0x111, 0xF, 0xF, false));
+    v = step(v, __builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), 0x112, 0xF, 0xF, false));
+    v = step(v, __builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), 0x114, 0xF, 0xF, false));
+    v = step(v, __builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), 0x118, 0xF, 0xF, false));
+    v = step(v, __builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), 0x142, 0xA, 0xF, false));
+    return v;
+}
+
+// Box of the 32 edges of each half of the wave, both ends of the alive ones:
+// {-min X, max X, -min Y, max Y} and the largest E; lanes 31 and 63 write it
+#define L2O_BOX_NONE (-1e6f)
+__device__ __forceinline__ void edge_boxes(const qedge &q, bool alive, int lane, float *out)
+{
+    const half2v a = __builtin_bit_cast(half2v, q.p0), b = __builtin_bit_cast(half2v, q.p1);
+    const float x0 = (float)a[0], y0 = (float)a[1], x1 = (float)b[0], y1 = (float)b[1];
+    const float v[5] = {-__builtin_fminf(x0, x1), __builtin_fmaxf(x0, x1), -__builtin_fminf(y0, y1),
+                        __builtin_fmaxf(y0, y1), q.e};
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+        const float m = half_max_f32(alive ? v[k] : L2O_BOX_NONE);
+        if ((lane & 31) == 31) out[5 * (lane >> 5) + k] = m;
+    }
+}
+
+// One work item: rows [a0, a0 + rows) and the 64 K WAVES columns from b0.  A wave
+// keeps its columns' operands in registers; the rows stream through LDS in
+// chunks of one row per thread, the next chunk's points loaded while this one
+// is tested.
+template <int K, int WAVES, int MODE>
+__device__ __forceinline__ void sweep_item(const l2o_sweep_item it, l2o_inst *__restrict__ insts)
+{
+    l2o_inst *in = insts + it.inst;
+    // The fields this kernel reads but no wave writes come in one batch of
+    // scalar loads before any branch (constant address space: other kernels
+    // and the host write them, and the scalar cache starts clean)
+    const __attribute__((address_space(4))) l2o_inst *ci = (const __attribute__((address_space(4))) l2o_inst *)in;
+    const uint32_t phase = ci->phase, par = ci->parity;
+    const int n = (int)ci->n;
+    const float slack = ci->slack;
+    const uint32_t metric = ci->metric;
+    const float es = ci->est_scale, ea = ci->est_add;
+    const float qk = ci->qk, qm = ci->qm;
+    l2o_pt *const p0 = ci->pts[0], *const p1 = ci->pts[1];
+    unsigned long long *const pool = ci->pool;
+    asm volatile("" ::"s"(phase), "s"(par), "s"(n), "s"(slack), "s"(p0), "s"(p1), "s"(it.a0), "s"(it.b0),
+                 "s"(it.rows), "s"(metric), "s"(qk), "s"(pool));
+    if (phase != L2O_LO) return;
+    const gpt *__restrict__ P = (const gpt *)(par ? p1 : p0);
+
+    constexpr bool PRUNE = MODE == L2O_SWEEP_PRUNE;
+    constexpr int NT = 2 * K;         // column tiles of a wave
+    constexpr int WC = 64 * K;        // columns of a wave
+    constexpr int CH = 64 * WAVES;    // rows of a chunk
+    constexpr int HCAP = 4 * K;       // pairs of tiles kept until they are evaluated
+    __shared__ __attribute__((aligned(16))) uint4 s_row[2 * CH + 1];
+    __shared__ __attribute__((aligned(16))) uint4 s_col[WAVES * WC];
+    __shared__ uint32_t s_nh[WAVES * WC];
+    __shared__ uint32_t s_list[WAVES][128];
+    __shared__ uint32_t s_hdr[WAVES][HCAP];
+    __shared__ int s_max[2 * WAVES];
+    __shared__ float s_rbox[PRUNE ? 2 * 2 * WAVES * 5 : 1];
+    __shared__ float s_cbox[PRUNE ? WAVES * NT * 5 : 1];
+    const int a0 = (int)it.a0;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int tid = (int)threadIdx.x;
+    const int lane = tid & 63;
+    const int bw = (int)it.b0 + w * WC;                                         // first column of this wave
+    const int ncol = min(n - 1 - (int)it.b0, WAVES * WC);
+    // rows a <= n-4 have candidates, and only rows a <= b-2 of the last column b
+    const int rows = min(min((int)it.rows, n - 3 - a0), (int)it.b0 + ncol - 2 - a0);
+    if (rows <= 0) return;
+
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    typedef const __attribute__((address_space(1))) u32x2 *gdw;
+    auto dw = [&](int k) __attribute__((always_inline)) { return *(gdw)&P[min(k, n - 1)].d; };  // {d, w}
+    auto ld4 = [&](int k) __attribute__((always_inline)) {
+        return make_uint4((uint32_t)P[k].x, (uint32_t)P[k].y, (uint32_t)P[k].d, (uint32_t)P[k].w);
+    };
+    // columns bw .. bw+WC-1 per wave, the first chunk of rows, every row's length
+    qedge qc[K], qr;
+    int br = 0, bc = 0;  // largest D of the rows and bits of the largest E of the columns (E >= 1; 0: none)
+    {
+        uint32_t w0[K];
+        u32x2 v1[K];
+#pragma unroll
+        for (int m = 0; m < K; ++m) {
+            w0[m] = dw(bw + 64 * m + lane).y;
+            v1[m] = dw(bw + 64 * m + lane + 1);
+        }
+        const uint32_t rw0 = dw(a0 + tid).y;
+        const u32x2 rv1 = dw(a0 + tid + 1);
+        for (int r = tid; r < rows; r += CH) br = max(br, P[a0 + r + 1].d);
+#pragma unroll
+        for (int m = 0; m < K; ++m) qc[m] = quant_edge(w0[m], v1[m].y, v1[m].x, qk, qm);
+        qr = quant_edge(rw0, rv1.y, rv1.x, qk, qm);
+    }
+    // cap = the largest gain still worth an exact evaluation: -1 (improving
+    // moves only) or the instance's best key so far, taken inclusively (it may
+    // come from a larger i: a tie at a smaller i wins)
+    auto key_now = [&]() __attribute__((always_inline)) -> unsigned long long {
+        return uniform_u64(__hip_atomic_load(&in->key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    };
+    int cap = -1;
+    {
+        const unsigned long long g = key_now();
+        if (g != L2O_SENTINEL) cap = min(cap, key_gain(g));
+    }
+    // half of -C (waves may start with different caps: each is a valid one)
+    const float hc = __builtin_fmaxf(__builtin_floorf((float)-cap * (qk * 0.49999f) - 0.01f), 0.0f);
+    float thr = (float)cap + slack;  // tier 2
+
+#pragma unroll
+    for (int m = 0; m < K; ++m)
+        if (bw + 64 * m + lane <= n - 2) bc = max(bc, __float_as_int(qc[m].e));
+    br = wave_max_i32(br);
+    bc = wave_max_i32(bc);
+    if constexpr (WAVES > 1) {
+        if (lane == 0) {
+            s_max[w] = br;
+            s_max[WAVES + w] = bc;
+        }
+        __syncthreads();
+        br = s_max[0];
+        bc = s_max[WAVES];
+#pragma unroll
+        for (int q = 1; q < WAVES; ++q) {
+            br = max(br, s_max[q]);
+            bc = max(bc, s_max[WAVES + q]);
+        }
+    }
+    // a row is alive if E_a + C + max E_b >= 0
+    const float row_min = 2.0f * hc - __int_as_float(bc);
+    const float col_min = 2.0f * hc - __builtin_ceilf(__builtin_fmaf((float)br, qk, qm));
+
+    const bool upper = lane >= 32;
+    half8 B[NT];
+    uint4 *const scol = s_col + w * WC;
+    uint32_t *const snh = s_nh + w * WC;
+#pragma unroll
+    for (int m = 0; m < K; ++m) {
+        const bool alive = bw + 64 * m + lane <= n - 2 && qc[m].e >= col_min;
+        const qterms t = edge_terms(qc[m], hc, alive);
+        scol[64 * m + lane] = col_record(qc[m], t);
+        snh[64 * m + lane] = col_upper(t);
+        if constexpr (PRUNE) edge_boxes(qc[m], alive, lane, s_cbox + 5 * (w * NT + 2 * m));
+    }
+    asm volatile("" ::: "memory");  // (the wave's own columns: LDS keeps its order)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        uint4 v = scol[32 * t + (lane & 31)];
+        v.x = upper ? snh[32 * t + (lane & 31)] : v.x;
+        B[t] = __builtin_bit_cast(half8, v);
+    }
+    // the column stage now holds the sign masks of tile pairs with survivors
+    asm volatile("" ::: "memory");
+    uint32_t *const smask = (uint32_t *)scol;
+    uint32_t *const slist = s_list[w];
+    // row r of the item into its half of the chunk buffer
+    auto stage_row = [&](const qedge &q, int r, int half) __attribute__((always_inline)) {
+        const bool alive = r < rows && q.e >= row_min;
+        s_row[half * CH + tid] = row_record(q, edge_terms(q, hc, alive));
+        if constexpr (PRUNE) edge_boxes(q, alive, lane, s_rbox + 5 * (half * 2 * WAVES + 2 * w));
+    };
+    stage_row(qr, tid, 0);
+    if (tid == 0) s_row[2 * CH] = row_const();
+
+    unsigned long long lbest = L2O_SENTINEL, published = L2O_SENTINEL;
+    unsigned fb = 0;
+    int nh = 0;  // pairs kept
+
+    // exact evaluation of the kept pairs' survivors
+    auto drain = [&]() __attribute__((always_inline)) {
+        asm volatile("" ::: "memory");
+        int e = 0, cnt = 0;
+        uint32_t m = 0, hdr = 0;
+        for (;;) {
+            // fill the list to a full wave
+            while (cnt < 64) {
+                unsigned long long any = __ballot(m != 0);
+                if (!any) {
+                    if (e >= nh) break;
+                    m = smask[64 * e + lane];
+                    hdr = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_hdr[w][e]);
+                    ++e;
+                    any = __ballot(m != 0);
+                }
+                if (m) {
+                    const int bit = __builtin_ctz(m);
+                    m &= m - 1;
+                    const uint32_t row = (hdr >> 12) + (uint32_t)((bit & 3) + ((bit >> 2) & 3) * 8 + (lane >> 5) * 4);
+                    const uint32_t col = (hdr & 0xFFFu) + (uint32_t)((bit >> 4) * 32 + (lane & 31));
+                    slist[cnt + lanes_below(any)] = (row << 12) | col;
+                }
+                cnt += __builtin_popcountll(any);
+            }
+            if (cnt == 0) break;
+            asm volatile("" ::: "memory");
+            if (lane < cnt) {
+                const uint32_t v = slist[lane];
+                const int a = a0 + (int)(v >> 12), b = bw + (int)(v & 0xFFFu);
+                const uint4 A0 = ld4(a), A1 = ld4(a + 1), B0 = ld4(b), B1 = ld4(b + 1);
+                const int da = (int)A1.z, db = (int)B1.z;
+                const float w2 = (est_dist((int)A0.x, (int)A0.y, (int)B0.x, (int)B0.y, es, ea) +
+                                  est_dist((int)A1.x, (int)A1.y, (int)B1.x, (int)B1.y, es, ea)) - (float)db;
+                if (w2 <= thr + (float)da) {
+                    ++fb;
+                    const int gain = exact_dist((int)A0.x, (int)A0.y, (int)B0.x, (int)B0.y, metric) +
+                                     exact_dist((int)A1.x, (int)A1.y, (int)B1.x, (int)B1.y, metric) - da - db;
+                    if (gain < 0) {
+                        const uint32_t i = (uint32_t)(a + 1);
+                        const unsigned long long key = make_key(gain, i, (uint32_t)(b + 1));
+                        lbest = key < lbest ? key : lbest;
+                        atomicMin(&pool[(i * 0x9E3779B1u) >> 26], key);
+                    }
+                }
+            }
+            // what was not evaluated moves to the front of the list
+            uint32_t rest = 0;
+            if (lane < cnt - 64) rest = slist[64 + lane];
+            asm volatile("" ::: "memory");
+            if (lane < cnt - 64) slist[lane] = rest;
+            asm volatile("" ::: "memory");
+            cnt = max(cnt - 64, 0);
+            // publish an improvement at once: other waves tighten their cap
+            if (__ballot(lbest < published)) {
+                published = wave_min_u64(lbest);
+                if (key_gain(published) < cap) {
+                    cap = key_gain(published);
+                    thr = (float)cap + slack;
+                }
+                if (lane == 0) atomicMin(&in->key, published);
+            }
+        }
+        nh = 0;
+    };
+
+    const float16v zero = {0};
+    // keeps the survivors of pair p and 32 rows from a0 + r0 (the two products
+    // again: the loop below keeps only the combined signs)
+    auto keep = [&](const half8 &A, int r0, int p) __attribute__((always_inline)) {
+        const float16v c0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(A, B[2 * p], zero, 0, 0, 0);
+        const float16v c1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(A, B[2 * p + 1], zero, 0, 0, 0);
+        const int aq = a0 + r0, bp = bw + 64 * p;
+        // sign bits: bit r of c0, bit 16 + r of c1
+        uint32_t mask = 0;
+#pragma unroll
+        for (int r = 15; r >= 0; --r) mask = __builtin_amdgcn_alignbit(mask, __float_as_uint(c1[r]), 31);
+#pragma unroll
+        for (int r = 15; r >= 0; --r) mask = __builtin_amdgcn_alignbit(mask, __float_as_uint(c0[r]), 31);
+        if (bp < aq + 33) {  // the pair meets the diagonal: candidates need a + 2 <= b
+            // bit r is row (r & 3) + 8 (r >> 2) + 4 (lane >> 5) of the block: the
+            // rows up to l have their bits 0 .. 4 (l >> 3) + min(l & 7, 3)
+            auto upto = [](int l) __attribute__((always_inline)) {
+                return l < 0 ? 0u : (2u << (4 * min(l >> 3, 3) + min(l >= 32 ? 3 : l & 7, 3))) - 1u;
+            };
+            const int l = bp + (lane & 31) - 2 - aq - (lane >> 5) * 4;
+            const uint32_t ok = (upto(l) & 0xFFFFu) | upto(l + 32) << 16;
+            mask &= ok;
+        }
+        if (__ballot(mask != 0)) {
+            smask[64 * nh + lane] = mask;
+            if (lane == 0) s_hdr[w][nh] = (uint32_t)r0 << 12 | (uint32_t)(64 * p);
+            ++nh;
+        }
+    };
+    for (int c = 0, half = 0; c < rows; c += CH, half ^= 1) {
+        // the next chunk's points, in flight while this one is tested
+        uint32_t nw0 = 0;
+        u32x2 nv1 = {0, 0};
+        const bool more = c + CH < rows;
+        if (more) {
+            nw0 = dw(a0 + c + CH + tid).y;
+            nv1 = dw(a0 + c + CH + tid + 1);
+        }
+        if constexpr (WAVES > 1) __syncthreads();
+        asm volatile("" ::: "memory");
+        unsigned long long live = ~0ull;
+        if constexpr (PRUNE) {
+            // lane l tests pair (q, p) = (l / K, l mod K) of a row block and two
+            // column tiles by their boxes: every candidate has |U - V|^2 at
+            // least twice the squared distance of the boxes (both ends of an
+            // edge lie in its box) and E_a + E_b at most the sum of the largest
+            const int q = lane / K, p = lane % K;
+            bool ok = false;
+            if (q < 2 * WAVES && c + 32 * q < rows && bw + 64 * p + 63 >= a0 + c + 32 * q + 2) {
+                const float *rb = s_rbox + 5 * (half * 2 * WAVES + q);
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const float *cb = s_cbox + 5 * (w * NT + 2 * p + h);
+                    const float dx = __builtin_fmaxf(__builtin_fmaxf(-rb[0] - cb[1], -cb[0] - rb[1]), 0.0f);
+                    const float dy = __builtin_fmaxf(__builtin_fmaxf(-rb[2] - cb[3], -cb[2] - rb[3]), 0.0f);
+                    const float s = rb[4] + cb[4] - 2.0f * hc;
+                    ok = ok || (s >= 0.0f && 2.0f * (dx * dx + dy * dy) <= s * s);
+                }
+            }
+            live = __ballot(ok);
+        }
+        // rows of the chunk that this wave's columns see
+        const int cr = min(min(rows - c, CH), min(bw + WC - 1, n - 2) - 1 - a0 - c);
+        const int nq = bw > n - 2 ? 0 : (cr + 31) >> 5;
+        // lanes 0..31 step through the rows, lanes 32..63 stay at the constant
+        int ra = upper ? 2 * CH : half * CH + lane;
+        const int rstep = upper ? 0 : 32;
+        for (int q = 0; q < nq; ++q, ra += rstep) {
+            const int r0 = c + 32 * q;
+            if (PRUNE && !((live >> (q * K)) & ((1ull << K) - 1))) continue;
+            const half8 A = __builtin_bit_cast(half8, s_row[ra]);
+            uint32_t m[K], all = 0;
+            if (PRUNE || bw < a0 + r0 + 33) {
+                // pruned, or at the diagonal: pair by pair
+#pragma unroll
+                for (int p = 0; p < K; ++p) {
+                    m[p] = (PRUNE ? (live >> (q * K + p)) & 1 : bw + 64 * p + 63 >= a0 + r0 + 2) ? 0x80000000u : 0u;
+                    all |= m[p];
+                }
+            } else {
+#pragma unroll
+                for (int p = 0; p < K; ++p) {
+                    m[p] = 0;
+                    const float16v c0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(A, B[2 * p], zero, 0, 0, 0);
+                    const float16v c1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(A, B[2 * p + 1], zero, 0, 0, 0);
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) m[p] |= __float_as_uint(c0[r]) | __float_as_uint(c1[r]);
+                    all |= m[p];
+                }
+            }
+            if (__ballot((int)all < 0)) {
+#pragma unroll
+                for (int p = 0; p < K; ++p)
+                    if (__ballot((int)m[p] < 0)) keep(A, r0, p);
+                if (nh + K > HCAP) drain();
+            }
+        }
+        if (more) {
+            qr = quant_edge(nw0, nv1.y, nv1.x, qk, qm);
+            stage_row(qr, c + CH + tid, half ^ 1);
+        }
+    }
+    if (nh) drain();
+
+    const unsigned wfb = wave_sum_u32(fb);
+    if (lane == 0 && wfb) atomicAdd(&in->fallbacks, (unsigned long long)wfb);
+}
+
+// waves per SIMD that the columns' operands leave room for (8 K VGPRs and about 55)
+#define L2O_WPE(K) ((K) <= 2 ? 6 : (K) <= 4 ? 5 : (K) <= 6 ? 4 : 3)
+template <int K, int WAVES, int MODE>
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(L2O_WPE(K)))) void k_sweep(
+    const l2o_sweep_item *__restrict__ items, l2o_inst *__restrict__ insts)
+{
+    sweep_item<K, WAVES, MODE>(items[blockIdx.x], insts);
+}
+
+// column and wave counts compiled into the library, and the tile shapes {k, t,
+// waves} the autotuner chooses among per n bucket (t, the rows of an item, is
+// up to the host)
+#define L2O_SWEEP_KERNELS(X) X(1, 1) X(2, 1) X(4, 1) X(6, 1) X(8, 1) X(4, 2) X(6, 2) X(8, 2) X(2, 4) X(4, 4) X(6, 4) X(8, 4)
+static const int g_shapes[][3] = {
+    {1, 32, 1}, {1, 64, 1}, {2, 64, 1}, {2, 128, 1}, {4, 64, 1}, {4, 128, 1}, {4, 256, 1}, {6, 64, 1}, {6, 128, 1},
+    {8, 64, 1}, {8, 128, 1}, {8, 256, 1}, {4, 64, 2}, {4, 128, 2}, {6, 64, 2}, {8, 64, 2}, {8, 128, 2}, {8, 256, 2},
+    {2, 64, 4}, {4, 64, 4}, {6, 64, 4}, {8, 64, 4}, {8, 128, 4}, {6, 128, 2}, {6, 160, 1}, {6, 128, 4}, {4, 256, 2},
+    {4, 256, 4}, {2, 256, 4}, {2, 512, 4}, {4, 512, 4}};
+
+#define L2O_SWEEP_CASE(K_, W_)                                                                            \
+    if (cfg.k == K_ && cfg.waves == W_) {                                                                \
+        if (mode == L2O_SWEEP_PRUNE)                                                                      \
+            hipLaunchKernelGGL((k_sweep<K_, W_, L2O_SWEEP_PRUNE>), dim3(nitems), dim3(64 * W_), 0, stream, items, insts); \
+        else                                                                                              \
+            hipLaunchKernelGGL((k_sweep<K_, W_, L2O_SWEEP_FULL>), dim3(nitems), dim3(64 * W_), 0, stream, items, insts); \
+        return hipGetLastError();                                                                         \
+    }
+
+hipError_t launch_sweep(const sweep_cfg &cfg, const l2o_sweep_item *items, uint32_t nitems,
+                        l2o_inst *insts, hipStream_t stream, int mode)
+{
+    if (nitems == 0) return hipSuccess;
+    if (mode != L2O_SWEEP_FULL && mode != L2O_SWEEP_PRUNE) return hipErrorInvalidValue;
+    L2O_SWEEP_KERNELS(L2O_SWEEP_CASE)
+    return hipErrorInvalidValue;
+}
+
+bool sweep_cfg_supported(const sweep_cfg &c)
+{
+    for (const auto &r : g_shapes)
+        if (r[0] == c.k && r[1] == c.t && r[2] == c.waves) return true;
+    return false;
+}
+
+int sweep_shapes(int (*out)[3], int cap)
+{
+    const int m = (int)(sizeof(g_shapes) / sizeof(g_shapes[0]));
+    for (int q = 0; q < m && q < cap; ++q) {
+        out[q][0] = g_shapes[q][0];
+        out[q][1] = g_shapes[q][1];
+        out[q][2] = g_shapes[q][2];
+    }
+    return m;
+}
+
+}  // namespace l2o
