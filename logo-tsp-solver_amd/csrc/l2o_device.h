@@ -137,4 +137,73 @@ __device__ __forceinline__ int wave_max_i32(int v)
     return __builtin_amdgcn_readlane(v, 63);
 }
 
+__device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long v)
+{
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        const unsigned lo = __shfl_xor((unsigned)v, off);
+        const unsigned hi = __shfl_xor((unsigned)(v >> 32), off);
+        v += ((unsigned long long)hi << 32) | lo;
+    }
+    return v;
+}
+
+// ---------------------------------------------------------------------------
+// ILS kicks (xoshiro256**)
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ unsigned long long rotl64(unsigned long long v, int k)
+{
+    return (v << k) | (v >> (64 - k));
+}
+
+__device__ inline unsigned long long xoshiro_next(unsigned long long *s)
+{
+    const unsigned long long result = rotl64(s[1] * 5ull, 7) * 9ull;
+    const unsigned long long t = s[1] << 17;
+    s[2] ^= s[0];
+    s[3] ^= s[1];
+    s[1] ^= s[2];
+    s[0] ^= s[3];
+    s[2] ^= t;
+    s[3] = rotl64(s[3], 45);
+    return result;
+}
+
+// cut points of a kick: the reference's a, b = rand() % n, sorted
+// (ILSGlobalSolver.cpp:39-44), or for the double bridge 1 <= p1 < p2 < p3 <= n-1
+__device__ inline void draw_kick(unsigned long long *rng, uint32_t kick, uint32_t n, uint32_t *cut)
+{
+    if (kick == 1) {
+        const uint32_t a = (uint32_t)(xoshiro_next(rng) % n);
+        const uint32_t b = (uint32_t)(xoshiro_next(rng) % n);
+        cut[0] = min(a, b);
+        cut[1] = max(a, b);
+        cut[2] = 0;
+        return;
+    }
+    int have = 0;
+    while (have < 3) {
+        const uint32_t v = 1u + (uint32_t)(xoshiro_next(rng) % (unsigned long long)(n - 1));
+        bool dup = false;
+        for (int q = 0; q < have; ++q) dup |= (cut[q] == v);
+        if (!dup) cut[have++] = v;
+    }
+    const uint32_t lo = min(min(cut[0], cut[1]), cut[2]), hi = max(max(cut[0], cut[1]), cut[2]);
+    cut[1] = cut[0] ^ cut[1] ^ cut[2] ^ lo ^ hi;
+    cut[0] = lo;
+    cut[2] = hi;
+}
+
+// position of the best tour that a kick puts at position k: rotate(a) then
+// reverse from b-a (ILSGlobalSolver.cpp:46-47), or A C B D of A=[0,a) B=[a,b)
+// C=[b,c) D=[c,n)
+__device__ __forceinline__ uint32_t kick_source(uint32_t k, uint32_t n, bool ref, uint32_t a, uint32_t b, uint32_t c)
+{
+    if (ref) return k < b - a ? (a + k) % n : (n - 1 - k + b) % n;
+    if (k < a) return k;
+    if (k < a + (c - b)) return b + (k - a);
+    if (k < c) return a + (k - a - (c - b));
+    return k;
+}
+
 }  // namespace l2o

@@ -148,24 +148,6 @@ __global__ __launch_bounds__(L2O_APPLY_THREADS) void k_apply(const l2o_apply_ite
 // ---------------------------------------------------------------------------
 // ILS bookkeeping: accept/revert, kick, restart (ILSGlobalSolverSequential.cpp:73-99)
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ unsigned long long rotl64(unsigned long long v, int k)
-{
-    return (v << k) | (v >> (64 - k));
-}
-
-__device__ unsigned long long xoshiro_next(unsigned long long *s)
-{
-    const unsigned long long result = rotl64(s[1] * 5ull, 7) * 9ull;
-    const unsigned long long t = s[1] << 17;
-    s[2] ^= s[0];
-    s[3] ^= s[1];
-    s[1] ^= s[2];
-    s[0] ^= s[3];
-    s[2] ^= t;
-    s[3] = rotl64(s[3], 45);
-    return result;
-}
-
 // A plain ILS instance at L2O_LO_DONE: accept iff strictly shorter (copy to
 // the best buffers), stop after `rounds` or once the best length is below
 // stop_below, else kick its best and restart.
@@ -202,34 +184,11 @@ __global__ __launch_bounds__(L2O_ILS_THREADS) void k_ils(l2o_inst *__restrict__ 
         s_accept = acc;
         s_done = done;
         if (!done && (phase == L2O_KICK || !grouped)) {
-            unsigned long long *rng = in->rng;
-            if (in->kick == 1) {  // reference kick: a, b = rand() % n, sorted (ILSGlobalSolver.cpp:39-44)
-                uint32_t a = (uint32_t)(xoshiro_next(rng) % n);
-                uint32_t b = (uint32_t)(xoshiro_next(rng) % n);
-                if (b < a) {
-                    const uint32_t tmp = a;
-                    a = b;
-                    b = tmp;
-                }
-                s_a = a;
-                s_b = b;
-                s_c = 0;
-            } else {  // double-bridge cut points 1 <= p1 < p2 < p3 <= n-1
-                uint32_t p[3];
-                int have = 0;
-                while (have < 3) {
-                    const uint32_t v = 1u + (uint32_t)(xoshiro_next(rng) % (unsigned long long)(n - 1));
-                    bool dup = false;
-                    for (int q = 0; q < have; ++q) dup |= (p[q] == v);
-                    if (!dup) p[have++] = v;
-                }
-                if (p[0] > p[1]) { const uint32_t tmp = p[0]; p[0] = p[1]; p[1] = tmp; }
-                if (p[1] > p[2]) { const uint32_t tmp = p[1]; p[1] = p[2]; p[2] = tmp; }
-                if (p[0] > p[1]) { const uint32_t tmp = p[0]; p[0] = p[1]; p[1] = tmp; }
-                s_a = p[0];
-                s_b = p[1];
-                s_c = p[2];
-            }
+            uint32_t cut[3];
+            draw_kick(in->rng, in->kick, n, cut);
+            s_a = cut[0];
+            s_b = cut[1];
+            s_c = cut[2];
         }
     }
     __syncthreads();
@@ -264,16 +223,7 @@ __global__ __launch_bounds__(L2O_ILS_THREADS) void k_ils(l2o_inst *__restrict__ 
     const uint32_t *__restrict__ BR = src->btour;
     const uint32_t a = s_a, b = s_b, c = s_c;
     const bool ref = in->kick == 1;
-    auto src_of = [&](uint32_t k) -> uint32_t {
-        if (ref) {  // rotate(a) then reverse from b-a (ILSGlobalSolver.cpp:46-47)
-            return k < b - a ? (a + k) % n : (n - 1 - k + b) % n;
-        }
-        // A C B D: A=[0,a) B=[a,b) C=[b,c) D=[c,n)
-        if (k < a) return k;
-        if (k < a + (c - b)) return b + (k - a);
-        if (k < c) return a + (k - a - (c - b));
-        return k;
-    };
+    auto src_of = [&](uint32_t k) -> uint32_t { return kick_source(k, n, ref, a, b, c); };
     l2o_pt *__restrict__ Pn = in->pts[0];
     uint32_t *__restrict__ Rn = in->tour[0];
     const uint32_t metric = in->metric;
@@ -292,12 +242,7 @@ __global__ __launch_bounds__(L2O_ILS_THREADS) void k_ils(l2o_inst *__restrict__ 
         Pn[k] = r;
         Rn[k] = BR[s];
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        const unsigned lo = __shfl_xor((unsigned)sum, off);
-        const unsigned hi = __shfl_xor((unsigned)(sum >> 32), off);
-        sum += ((unsigned long long)hi << 32) | lo;
-    }
+    sum = wave_sum_u64(sum);
     if ((threadIdx.x & 63) == 0) s_sum[threadIdx.x >> 6] = sum;
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -364,12 +309,7 @@ __global__ __launch_bounds__(256) void k_length(const l2o_inst *__restrict__ ins
         const l2o_pt p = P[k], q = P[k == 0 ? n - 1 : k - 1];
         sum += (unsigned long long)exact_dist(q.x, q.y, p.x, p.y, in->metric);
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        const unsigned lo = __shfl_xor((unsigned)sum, off);
-        const unsigned hi = __shfl_xor((unsigned)(sum >> 32), off);
-        sum += ((unsigned long long)hi << 32) | lo;
-    }
+    sum = wave_sum_u64(sum);
     if ((threadIdx.x & 63) == 0 && sum) atomicAdd(out, sum);
 }
 

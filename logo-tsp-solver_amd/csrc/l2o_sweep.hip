@@ -18,7 +18,7 @@
 //     E = ceil(s kappa D + s h / 2 + 1),   C = -2 floor(s kappa |cap| / 2)
 // a candidate that can still win has |U - V|^2 <= (E_a + E_b + C)^2.  Both
 // sides expand into an inner product of a row record and a column record
-// (the cap goes in half to each side, E' = E + C/2, N = |U|^2 - E'^2):
+// (the cap goes in half to each side, E' = max(E + C/2, 0), N = |U|^2 - E'^2):
 //     |U - V|^2 - (E'_a + E'_b)^2 - 1
 //        = -2 U.V - 2 E'_a E'_b + N_a + N_b - 1 < 0,
 // 5 products and N split into N = 2048 Nh + Nl on each side: 10 of the 16
@@ -38,10 +38,9 @@
 // launches' latency).  Matrix results kept in AGPRs, as the compiler prefers,
 // cost a copy each: 2.7e13 instead of 4.4e13 tests/s (-amdgpu-mfma-vgpr-form).
 //
-// A row with E_a + C + max E_b < 0 (and a column likewise) has no candidate
-// left: its record is replaced by one that never passes.  So |E'| <= L2O_QE for
-// the others, and (E'_a + E'_b)^2 of a pair with a negative sum, which passes
-// although it cannot win, stays as small as the largest legitimate one.
+// E' is cut off at 0 (a larger sum only lets more pass): without it a pair of
+// short edges has a negative sum under a strong cap, and its square lets
+// thousands of candidates pass that cannot win.
 //
 // Survivors.  The 32 sign bits of a pair of tiles are stored in LDS per lane;
 // every row block the wave compacts them into full waves of candidates, which
@@ -51,76 +50,9 @@
 #include <hip/hip_runtime.h>
 
 #include "l2o_device.h"
+#include "l2o_quant.h"
 
 namespace l2o {
-
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-typedef float float16v __attribute__((ext_vector_type(16)));
-
-__device__ __forceinline__ uint32_t pk16(float a, float b)
-{
-    return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a, b));
-}
-
-// the wave's lanes below this one among `m`
-__device__ __forceinline__ int lanes_below(unsigned long long m)
-{
-    return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-}
-
-// quantised edge k -> k+1: {X, Y} and {X1, Y1} as FP16 pairs (l2o_pt.w of its
-// ends), U = |(X, Y, X1, Y1)|^2 and E of its length (l2o_pt.d of k+1)
-struct qedge {
-    uint32_t p0, p1;
-    float u, e;
-};
-
-__device__ __forceinline__ qedge quant_edge(uint32_t w0, uint32_t w1, uint32_t d1, float qk, float qm)
-{
-    const half2v a = __builtin_bit_cast(half2v, w0), b = __builtin_bit_cast(half2v, w1);
-    qedge r;
-    r.p0 = w0;
-    r.p1 = w1;
-    r.u = __builtin_amdgcn_fdot2(a, a, __builtin_amdgcn_fdot2(b, b, 0.0f, false), false);
-    r.e = __builtin_ceilf(__builtin_fmaf((float)(int)d1, qk, qm));
-    return r;
-}
-
-// E' and the limbs of N of an edge; an edge without a candidate (alive false)
-// gets an Nh that no other terms can outweigh
-struct qterms {
-    float e, nh, nl;
-};
-__device__ __forceinline__ qterms edge_terms(const qedge &q, float hc, bool alive)
-{
-    qterms t;
-    t.e = q.e - hc;
-    const float nn = __builtin_fmaf(-t.e, t.e, q.u);
-    t.nh = __builtin_floorf(nn * (1.0f / 2048.0f));
-    t.nl = __builtin_fmaf(t.nh, -2048.0f, nn);
-    t.nh = alive ? t.nh : 30000.0f;
-    return t;
-}
-
-// A operand (rows), 16 FP16 terms: lanes 0..31 {X, Y, X1, Y1, E', 1, Nl, Nh},
-// lanes 32..63 the same {2048, 1, 0, 0, 0, 0, 0, 0} for every row
-__device__ __forceinline__ uint4 row_record(const qedge &q, const qterms &t)
-{
-    return make_uint4(q.p0, q.p1, pk16(t.e, 1.0f), pk16(t.nl, t.nh));
-}
-__device__ __forceinline__ uint4 row_const() { return make_uint4(pk16(2048.0f, 1.0f), 0u, 0u, 0u); }
-
-// B operand (columns): lanes 0..31 {-2X, -2Y, -2X1, -2Y1, -2E', Nl, 1, 2048},
-// lanes 32..63 {Nh, -1, any six finite numbers}
-__device__ __forceinline__ uint4 col_record(const qedge &q, const qterms &t)
-{
-    const half2v m2 = {(_Float16)-2.0f, (_Float16)-2.0f};
-    return make_uint4(__builtin_bit_cast(uint32_t, __builtin_bit_cast(half2v, q.p0) * m2),
-                      __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2v, q.p1) * m2),
-                      pk16(-2.0f * t.e, t.nl), pk16(1.0f, 2048.0f));
-}
-__device__ __forceinline__ uint32_t col_upper(const qterms &t) { return pk16(t.nh, -1.0f); }
 
 // maximum over each half of the wave, in lanes 31 and 63 (the others hold partial ones)
 __device__ __forceinline__ float half_max_f32(float v)
@@ -134,18 +66,18 @@ __device__ __forceinline__ float half_max_f32(float v)
     return v;
 }
 
-// Box of the 32 edges of each half of the wave, both ends of the alive ones:
-// {-min X, max X, -min Y, max Y} and the largest E; lanes 31 and 63 write it
+// Box of the 32 edges of each half of the wave, both ends of the valid ones:
+// {-min X, max X, -min Y, max Y} and the largest E'; lanes 31 and 63 write it
 #define L2O_BOX_NONE (-1e6f)
-__device__ __forceinline__ void edge_boxes(const qedge &q, bool alive, int lane, float *out)
+__device__ __forceinline__ void edge_boxes(const qedge &q, float e, bool valid, int lane, float *out)
 {
     const half2v a = __builtin_bit_cast(half2v, q.p0), b = __builtin_bit_cast(half2v, q.p1);
     const float x0 = (float)a[0], y0 = (float)a[1], x1 = (float)b[0], y1 = (float)b[1];
     const float v[5] = {-__builtin_fminf(x0, x1), __builtin_fmaxf(x0, x1), -__builtin_fminf(y0, y1),
-                        __builtin_fmaxf(y0, y1), q.e};
+                        __builtin_fmaxf(y0, y1), e};
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
-        const float m = half_max_f32(alive ? v[k] : L2O_BOX_NONE);
+        const float m = half_max_f32(valid ? v[k] : L2O_BOX_NONE);
         if ((lane & 31) == 31) out[5 * (lane >> 5) + k] = m;
     }
 }
@@ -185,7 +117,6 @@ __device__ __forceinline__ void sweep_item(const l2o_sweep_item it, l2o_inst *__
     __shared__ uint32_t s_nh[WAVES * WC];
     __shared__ uint32_t s_list[WAVES][128];
     __shared__ uint32_t s_hdr[WAVES][HCAP];
-    __shared__ int s_max[2 * WAVES];
     __shared__ float s_rbox[PRUNE ? 2 * 2 * WAVES * 5 : 1];
     __shared__ float s_cbox[PRUNE ? WAVES * NT * 5 : 1];
     const int a0 = (int)it.a0;
@@ -204,9 +135,8 @@ __device__ __forceinline__ void sweep_item(const l2o_sweep_item it, l2o_inst *__
     auto ld4 = [&](int k) __attribute__((always_inline)) {
         return make_uint4((uint32_t)P[k].x, (uint32_t)P[k].y, (uint32_t)P[k].d, (uint32_t)P[k].w);
     };
-    // columns bw .. bw+WC-1 per wave, the first chunk of rows, every row's length
+    // columns bw .. bw+WC-1 per wave, the first chunk of rows
     qedge qc[K], qr;
-    int br = 0, bc = 0;  // largest D of the rows and bits of the largest E of the columns (E >= 1; 0: none)
     {
         uint32_t w0[K];
         u32x2 v1[K];
@@ -217,7 +147,6 @@ __device__ __forceinline__ void sweep_item(const l2o_sweep_item it, l2o_inst *__
         }
         const uint32_t rw0 = dw(a0 + tid).y;
         const u32x2 rv1 = dw(a0 + tid + 1);
-        for (int r = tid; r < rows; r += CH) br = max(br, P[a0 + r + 1].d);
 #pragma unroll
         for (int m = 0; m < K; ++m) qc[m] = quant_edge(w0[m], v1[m].y, v1[m].x, qk, qm);
         qr = quant_edge(rw0, rv1.y, rv1.x, qk, qm);
@@ -234,31 +163,8 @@ __device__ __forceinline__ void sweep_item(const l2o_sweep_item it, l2o_inst *__
         if (g != L2O_SENTINEL) cap = min(cap, key_gain(g));
     }
     // half of -C (waves may start with different caps: each is a valid one)
-    const float hc = __builtin_fmaxf(__builtin_floorf((float)-cap * (qk * 0.49999f) - 0.01f), 0.0f);
+    const float hc = half_cap(cap, qk);
     float thr = (float)cap + slack;  // tier 2
-
-#pragma unroll
-    for (int m = 0; m < K; ++m)
-        if (bw + 64 * m + lane <= n - 2) bc = max(bc, __float_as_int(qc[m].e));
-    br = wave_max_i32(br);
-    bc = wave_max_i32(bc);
-    if constexpr (WAVES > 1) {
-        if (lane == 0) {
-            s_max[w] = br;
-            s_max[WAVES + w] = bc;
-        }
-        __syncthreads();
-        br = s_max[0];
-        bc = s_max[WAVES];
-#pragma unroll
-        for (int q = 1; q < WAVES; ++q) {
-            br = max(br, s_max[q]);
-            bc = max(bc, s_max[WAVES + q]);
-        }
-    }
-    // a row is alive if E_a + C + max E_b >= 0
-    const float row_min = 2.0f * hc - __int_as_float(bc);
-    const float col_min = 2.0f * hc - __builtin_ceilf(__builtin_fmaf((float)br, qk, qm));
 
     const bool upper = lane >= 32;
     half8 B[NT];
@@ -266,11 +172,11 @@ __device__ __forceinline__ void sweep_item(const l2o_sweep_item it, l2o_inst *__
     uint32_t *const snh = s_nh + w * WC;
 #pragma unroll
     for (int m = 0; m < K; ++m) {
-        const bool alive = bw + 64 * m + lane <= n - 2 && qc[m].e >= col_min;
-        const qterms t = edge_terms(qc[m], hc, alive);
+        const bool valid = bw + 64 * m + lane <= n - 2;
+        const qterms t = edge_terms(qc[m], hc, valid);
         scol[64 * m + lane] = col_record(qc[m], t);
         snh[64 * m + lane] = col_upper(t);
-        if constexpr (PRUNE) edge_boxes(qc[m], alive, lane, s_cbox + 5 * (w * NT + 2 * m));
+        if constexpr (PRUNE) edge_boxes(qc[m], t.e, valid, lane, s_cbox + 5 * (w * NT + 2 * m));
     }
     asm volatile("" ::: "memory");  // (the wave's own columns: LDS keeps its order)
 #pragma unroll
@@ -285,9 +191,10 @@ __device__ __forceinline__ void sweep_item(const l2o_sweep_item it, l2o_inst *__
     uint32_t *const slist = s_list[w];
     // row r of the item into its half of the chunk buffer
     auto stage_row = [&](const qedge &q, int r, int half) __attribute__((always_inline)) {
-        const bool alive = r < rows && q.e >= row_min;
-        s_row[half * CH + tid] = row_record(q, edge_terms(q, hc, alive));
-        if constexpr (PRUNE) edge_boxes(q, alive, lane, s_rbox + 5 * (half * 2 * WAVES + 2 * w));
+        const bool valid = r < rows;
+        const qterms t = edge_terms(q, hc, valid);
+        s_row[half * CH + tid] = row_record(q, t);
+        if constexpr (PRUNE) edge_boxes(q, t.e, valid, lane, s_rbox + 5 * (half * 2 * WAVES + 2 * w));
     };
     stage_row(qr, tid, 0);
     if (tid == 0) s_row[2 * CH] = row_const();
@@ -369,21 +276,10 @@ __device__ __forceinline__ void sweep_item(const l2o_sweep_item it, l2o_inst *__
         const float16v c0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(A, B[2 * p], zero, 0, 0, 0);
         const float16v c1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(A, B[2 * p + 1], zero, 0, 0, 0);
         const int aq = a0 + r0, bp = bw + 64 * p;
-        // sign bits: bit r of c0, bit 16 + r of c1
-        uint32_t mask = 0;
-#pragma unroll
-        for (int r = 15; r >= 0; --r) mask = __builtin_amdgcn_alignbit(mask, __float_as_uint(c1[r]), 31);
-#pragma unroll
-        for (int r = 15; r >= 0; --r) mask = __builtin_amdgcn_alignbit(mask, __float_as_uint(c0[r]), 31);
+        uint32_t mask = sign_mask(c0, c1);
         if (bp < aq + 33) {  // the pair meets the diagonal: candidates need a + 2 <= b
-            // bit r is row (r & 3) + 8 (r >> 2) + 4 (lane >> 5) of the block: the
-            // rows up to l have their bits 0 .. 4 (l >> 3) + min(l & 7, 3)
-            auto upto = [](int l) __attribute__((always_inline)) {
-                return l < 0 ? 0u : (2u << (4 * min(l >> 3, 3) + min(l >= 32 ? 3 : l & 7, 3))) - 1u;
-            };
             const int l = bp + (lane & 31) - 2 - aq - (lane >> 5) * 4;
-            const uint32_t ok = (upto(l) & 0xFFFFu) | upto(l + 32) << 16;
-            mask &= ok;
+            mask &= rows_upto(l) | rows_upto(l + 32) << 16;
         }
         if (__ballot(mask != 0)) {
             smask[64 * nh + lane] = mask;
@@ -407,7 +303,7 @@ __device__ __forceinline__ void sweep_item(const l2o_sweep_item it, l2o_inst *__
             // lane l tests pair (q, p) = (l / K, l mod K) of a row block and two
             // column tiles by their boxes: every candidate has |U - V|^2 at
             // least twice the squared distance of the boxes (both ends of an
-            // edge lie in its box) and E_a + E_b at most the sum of the largest
+            // edge lie in its box) and E'_a + E'_b at most the sum of the largest
             const int q = lane / K, p = lane % K;
             bool ok = false;
             if (q < 2 * WAVES && c + 32 * q < rows && bw + 64 * p + 63 >= a0 + c + 32 * q + 2) {
@@ -417,7 +313,7 @@ __device__ __forceinline__ void sweep_item(const l2o_sweep_item it, l2o_inst *__
                     const float *cb = s_cbox + 5 * (w * NT + 2 * p + h);
                     const float dx = __builtin_fmaxf(__builtin_fmaxf(-rb[0] - cb[1], -cb[0] - rb[1]), 0.0f);
                     const float dy = __builtin_fmaxf(__builtin_fmaxf(-rb[2] - cb[3], -cb[2] - rb[3]), 0.0f);
-                    const float s = rb[4] + cb[4] - 2.0f * hc;
+                    const float s = rb[4] + cb[4];
                     ok = ok || (s >= 0.0f && 2.0f * (dx * dx + dy * dy) <= s * s);
                 }
             }
