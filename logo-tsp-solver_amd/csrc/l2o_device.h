@@ -8,14 +8,39 @@
 namespace l2o {
 
 // ---------------------------------------------------------------------------
-// exact metric length of the edge P1 -> P2 (metric_dist in l2o_launch.h)
+// exact metric length of the edge P1 -> P2 (metric_dist in l2o_launch.h) without
+// FP64: with m an estimate of floor(sqrt(s / f)) from v_sqrt_f32, at most 3 off
+// (s has a relative error of 2^-23, the root 3 ulp, and sqrt(s) < 2^22.5), the
+// remainder r = s - f m^2 is below 2^28 in magnitude, so 32-bit arithmetic holds it.
+// floor(r / (f (2m+1))) is the distance to the true root or one more, and one
+// correction each way makes m exact; then s > f m^2 + e m is r > e m.
 // ---------------------------------------------------------------------------
+template <int F>
+__device__ __forceinline__ int root_len(uint32_t s32, float fs, int e)
+{
+    int m = (int)__builtin_amdgcn_sqrtf(F == 1 ? fs : fs * 0.1f);
+    int r = (int)(s32 - (uint32_t)F * ((uint32_t)m * (uint32_t)m));
+    const int d = (int)__builtin_floorf((float)r * __builtin_amdgcn_rcpf((float)(F * (2 * m + 1))));
+    r -= F * (d * (2 * m + d));
+    m += d;
+    if (r < 0) {
+        m -= 1;
+        r += F * (2 * m + 1);
+    }
+    if (r >= F * (2 * m + 1)) {
+        r -= F * (2 * m + 1);
+        m += 1;
+    }
+    return m + (r > e * m ? 1 : 0);
+}
+
 __device__ __forceinline__ int exact_dist(int x1, int y1, int x2, int y2, uint32_t metric)
 {
-    // coordinates lie in [0, 2^22): the differences and s are exact
-    const long long dx = (long long)(x1 - x2);
-    const long long dy = (long long)(y1 - y2);
-    return metric_dist(dx * dx + dy * dy, metric);
+    // coordinates lie in [0, 2^22)
+    const int dx = x1 - x2, dy = y1 - y2;
+    const uint32_t s32 = (uint32_t)dx * (uint32_t)dx + (uint32_t)dy * (uint32_t)dy;
+    const float fs = __builtin_fmaf((float)dx, (float)dx, (float)dy * (float)dy);
+    return metric == L2O_ATT ? root_len<10>(s32, fs, 0) : root_len<1>(s32, fs, metric == L2O_EUC_2D ? 1 : 0);
 }
 
 // FP32 estimate of the metric length: sqrt(s) * scale + add, with scale = 1,
@@ -92,6 +117,26 @@ __device__ __forceinline__ unsigned long long remap_key(unsigned long long key, 
     const uint32_t e1 = to(i2), e2 = to(j2);
     if (key == L2O_SENTINEL || in1 != in2 || i2 == i || i2 == J || j2 == i || j2 == J) return L2O_SENTINEL;
     return (key & ~((1ull << 40) - 1)) | ((unsigned long long)min(e1, e2) << 20) | max(e1, e2);
+}
+
+// The largest gain the next sweep evaluates, given the pool on its tour (one
+// entry per lane) and the best entry: that one's gain while the pool holds
+// enough others, else a somewhat worse one, so that the sweep refills the pool
+// before it runs out (a move invalidates up to half of it, and a sweep without
+// a known move evaluates every improving candidate).
+#ifndef L2O_POOL_LOW
+#define L2O_POOL_LOW 16
+#endif
+#ifndef L2O_CAP_SHIFT
+#define L2O_CAP_SHIFT 3
+#endif
+__device__ __forceinline__ int worse_gain(int gain) { return min(gain - (gain >> L2O_CAP_SHIFT), -1); }
+__device__ __forceinline__ int next_cap(unsigned long long entry, unsigned long long best)
+{
+    const int left = __builtin_popcountll(__ballot(entry != L2O_SENTINEL));
+    if (best == L2O_SENTINEL) return -1;
+    const int gain = key_gain(best);
+    return left >= L2O_POOL_LOW ? gain : worse_gain(gain);
 }
 
 // point records in global memory (address space 1: the pointers come from

@@ -64,9 +64,12 @@ struct tune_row {
 
 // Two tables: 0 = one instance in flight (latency: small tiles fill the
 // device), 1 = a batch (throughput: the batch fills the device, larger tiles
-// waste less).  An engine uses table 1 when it holds L2O_BATCH_MIN or more
-// live instances.
+// waste less).  An engine uses table 1 when at least L2O_BATCH_MIN instances
+// run in its steps and their sweeps add up to L2O_BATCH_PAIRS candidates (16
+// chains of 1,501 cities, 2e7, take 1.25x as long with table 1's tiles; 180
+// instances of 1,400-5,000 cities, 7e8, 1.2x as long with table 0's).
 #define L2O_BATCH_MIN 8
+#define L2O_BATCH_PAIRS 100000000ull
 std::mutex g_tune_mu;
 std::vector<tune_row> g_tune[2] = {
     {{640, {1, 64, 1}}, {8192, {4, 128, 1}}, {LOGO2OPT_MAX_N, {8, 256, 1}}},
@@ -210,6 +213,7 @@ struct slot_t {
     // only single sweeps run on it: their candidates go to the spare pool (the
     // row after the slots' ones), which no kernel reads
     bool sweep_only = false;
+    bool local = false;  // runs in k_local (assigned at the start of a run)
     uint32_t group_lead = L2O_NO_GROUP;  // multi-start ILS group (first slot)
     uint32_t group_size = 0;
 };
@@ -224,7 +228,7 @@ struct logo2opt_engine {
     uint32_t max_slots = 0;
     std::vector<slot_t> slots;
     l2o_inst *d_insts = nullptr;
-    unsigned long long *d_pool = nullptr;  // L2O_POOL keys per slot, and a spare row
+    unsigned long long *d_pool = nullptr;  // L2O_POOL keys per slot, and a spare row (behind d_insts)
     unsigned *d_live = nullptr;
     unsigned *h_live = nullptr;  // pinned
     unsigned live = 0;           // host mirror, valid between runs
@@ -249,6 +253,20 @@ struct logo2opt_engine {
     uint32_t group_grid = 0;  // k_group covers slots [0, group_grid)
     bool dirty = true;
     unsigned live_at_build = 0;
+
+    // instances that run in k_local, one launch per workgroup size, on a stream
+    // of their own if others run in steps beside them
+    struct local_group {
+        int waves;
+        uint32_t off, count, max_n;
+    };
+    std::vector<local_group> locals;
+    uint32_t *d_lids = nullptr;
+    size_t lids_cap = 0;
+    hipStream_t lstream = nullptr;
+    uint32_t local_chains = 0;  // chains of groups among them: slots [0, local_chains)
+    bool use_local = false, local_to_end = false;  // of the last assignment
+    unsigned live_launch = 0;  // live instances that run in steps
 
     hipGraphExec_t gexec = nullptr;
     uint32_t gsteps = 0;
@@ -392,6 +410,7 @@ int upload_instance(logo2opt_engine *e, int32_t id, const uint32_t *route, uint3
     in.stop_below = s.job.ils_rounds ? s.job.stop_below : 0;
     in.phase = phase;
     in.key = L2O_SENTINEL;
+    in.cap = -1;
     // SplitMix64 -> xoshiro256** state (same seeding as the workload generators)
     uint64_t x = s.job.seed;
     for (int k = 0; k < 4; ++k) {
@@ -462,6 +481,71 @@ uint64_t item_work(const l2o_sweep_item &it, const sweep_cfg &c, uint32_t n)
     return w;
 }
 
+// Instances of at most this many cities run in k_local.  A few of them: up to
+// the size where one workgroup's step takes as long as a step's two launches
+// (707 cities 8.2 against 9.0 us, 1,000 cities 10.2 against 9.6 us; 200 cities
+// 4.0 against 11.3 us), with 16 waves, or 8 where there is little to share out.
+// Many fill the device by themselves: four waves each, which leave room for
+// several workgroups on a CU, and larger ones too, which then take no part in
+// the others' launches (512-instance batch: 346 ms without, 337 ms with them).
+#define L2O_LOCAL_MANY 64u
+#define L2O_LOCAL_MAX_N 800u
+#define L2O_LOCAL_MANY_MAX_N 1400u
+
+// which instances run in k_local, and its lists (no kernel may be running)
+// Chains of multi-start groups too, if no instance is left to the steps (their
+// rounds alternate with k_ils and k_group launches, which cover all slots) and
+// the run is not cut at a number of steps (`to_end`).
+int assign_local(logo2opt_engine *e, bool use, bool to_end)
+{
+    bool chains = to_end;
+    for (const slot_t &s : e->slots)
+        if (s.used && !s.done && s.n > (s.group_lead == L2O_NO_GROUP ? L2O_LOCAL_MAX_N : L2O_LOCAL_MANY_MAX_N))
+            chains = false;
+    auto fits = [&](const slot_t &s, uint32_t max_n) {
+        return use && s.used && !s.done &&
+               (s.group_lead == L2O_NO_GROUP ? s.n <= max_n : chains && s.n <= L2O_LOCAL_MANY_MAX_N);
+    };
+    uint32_t count = 0;
+    for (uint32_t id = 0; id < e->max_slots; ++id) count += fits(e->slots[id], L2O_LOCAL_MANY_MAX_N) ? 1 : 0;
+    const bool many = count >= L2O_LOCAL_MANY;
+    auto waves_for = [&](uint32_t n) { return many ? 4 : n > 128 ? 16 : 8; };
+    std::vector<uint32_t> ids;
+    e->local_chains = 0;
+    for (uint32_t id = 0; id < e->max_slots; ++id) {
+        slot_t &s = e->slots[id];
+        s.local = fits(s, many ? L2O_LOCAL_MANY_MAX_N : L2O_LOCAL_MAX_N);
+        if (s.local) ids.push_back(id);
+        if (s.local && s.group_lead != L2O_NO_GROUP) e->local_chains = id + 1;
+    }
+    // largest first: the longest searches start first
+    std::stable_sort(ids.begin(), ids.end(), [&](uint32_t a, uint32_t b) { return e->slots[a].n > e->slots[b].n; });
+    e->locals.clear();
+    e->use_local = use;
+    e->local_to_end = to_end;
+    for (uint32_t k = 0; k < ids.size();) {
+        const uint32_t n = e->slots[ids[k]].n;
+        const int waves = waves_for(n);
+        uint32_t m = k;
+        while (m < ids.size() && waves_for(e->slots[ids[m]].n) == waves) ++m;
+        e->locals.push_back({waves, k, m - k, n});
+        k = m;
+    }
+    if (ids.size() > e->lids_cap) {
+        if (e->d_lids) (void)hipFree(e->d_lids);
+        e->d_lids = nullptr;
+        e->lids_cap = std::max<size_t>(ids.size(), 2 * e->lids_cap);
+        L2O_TRY(hipMalloc(&e->d_lids, e->lids_cap * sizeof(uint32_t)));
+    }
+    if (!ids.empty()) {
+        L2O_TRY(hipMemcpyAsync(e->d_lids, ids.data(), ids.size() * sizeof(uint32_t), hipMemcpyHostToDevice,
+                               e->stream));
+        L2O_TRY(hipStreamSynchronize(e->stream));
+    }
+    return LOGO2OPT_OK;
+}
+
+// work lists of the steps: the live instances that do not run in k_local
 int rebuild_lists(logo2opt_engine *e)
 {
     std::map<std::tuple<int, int, int, int>, std::vector<l2o_sweep_item>> by_cfg;
@@ -473,10 +557,13 @@ int rebuild_lists(logo2opt_engine *e)
     // ones fill the tail (longest-processing-time order)
     std::vector<uint32_t> order;
     for (uint32_t id = 0; id < e->max_slots; ++id)
-        if (e->slots[id].used && !e->slots[id].done) order.push_back(id);
+        if (e->slots[id].used && !e->slots[id].done && !e->slots[id].local) order.push_back(id);
+    e->live_launch = (unsigned)order.size();
     std::stable_sort(order.begin(), order.end(),
                      [&](uint32_t a, uint32_t b) { return e->slots[a].n > e->slots[b].n; });
-    const int table = order.size() >= L2O_BATCH_MIN ? 1 : 0;
+    uint64_t all_pairs = 0;
+    for (uint32_t id : order) all_pairs += pairs_of(e->slots[id].n);
+    const int table = order.size() >= L2O_BATCH_MIN && all_pairs >= L2O_BATCH_PAIRS ? 1 : 0;
     for (uint32_t id : order) {
         const slot_t &s = e->slots[id];
         const uint32_t n = s.n;
@@ -572,7 +659,7 @@ int rebuild_lists(logo2opt_engine *e)
     L2O_TRY(hipStreamSynchronize(e->stream));
     e->n_aitems = (uint32_t)ai.size();
     e->dirty = false;
-    e->live_at_build = e->live;
+    e->live_at_build = e->live_launch;
     drop_graph(e);
     return LOGO2OPT_OK;
 }
@@ -659,8 +746,26 @@ int scan_done(logo2opt_engine *e)
         slot_t &s = e->slots[id];
         if (s.used && !s.done && h[id].phase == L2O_DONE) {
             s.done = true;
+            if (!s.local) e->live_launch -= 1;
             e->done_queue.push_back((int32_t)id);
         }
+    }
+    return LOGO2OPT_OK;
+}
+
+// `steps` sweeps of every k_local instance, on its stream
+// (with chains: a number of rounds, each to the chains' local optima)
+int start_local(logo2opt_engine *e, uint32_t steps, hipStream_t st)
+{
+    constexpr int ROUNDS = 8;
+    for (int r = 0; r < (e->local_chains ? ROUNDS : 1); ++r) {
+        for (const auto &g : e->locals)
+            L2O_TRY(l2o::launch_local(g.waves, e->d_lids + g.off, g.count, g.max_n, e->d_insts, e->d_live, steps,
+                                      st));
+        if (!e->local_chains) break;
+        L2O_TRY(l2o::launch_ils(e->d_insts, e->local_chains, e->d_live, st));    // accept, wait
+        L2O_TRY(l2o::launch_group(e->d_insts, e->local_chains, e->d_live, st));  // the round's best
+        L2O_TRY(l2o::launch_ils(e->d_insts, e->local_chains, e->d_live, st));    // kick
     }
     return LOGO2OPT_OK;
 }
@@ -669,35 +774,60 @@ int engine_run(logo2opt_engine *e, uint32_t max_steps, uint32_t sync_every, uint
 {
     if (sync_every == 0) sync_every = 1;
     const double t0 = now_ms();
-    if (e->dirty) {
-        int rc = rebuild_lists(e);
+    // one host check per step (sync_every = 1) and the timed sweeps keep every
+    // instance in steps
+    const bool use_local = sync_every > 1 && !e->timing;
+    int rc = LOGO2OPT_OK;
+    const bool to_end = max_steps == 0xFFFFFFFFu;
+    if (e->dirty || e->use_local != use_local || e->local_to_end != to_end) {
+        rc = assign_local(e, use_local, to_end);
+        if (!rc) rc = rebuild_lists(e);
         if (rc) return rc;
     }
+    // a k_local launch runs to its instances' ends, or this many steps
+    constexpr uint32_t LOCAL_STEPS = 1u << 16;
+    uint32_t local_left = max_steps;
+    bool local_running = false;
+    hipStream_t st = e->stream;
+    if (!e->locals.empty() && e->live_launch > 0) {
+        if (!e->lstream) L2O_TRY(hipStreamCreateWithFlags(&e->lstream, hipStreamNonBlocking));
+        st = e->lstream;
+    }
+    auto next_local = [&]() {
+        const uint32_t k = std::min(local_left, LOCAL_STEPS);
+        if (e->locals.empty() || k == 0 || e->live == e->live_launch) return (int)LOGO2OPT_OK;
+        if (!to_end) local_left -= k;
+        local_running = true;
+        return start_local(e, k, st);
+    };
+    auto check_live = [&](hipStream_t on, bool scan = false) {
+        L2O_TRY(hipMemcpyAsync(e->h_live, e->d_live, sizeof(unsigned), hipMemcpyDeviceToHost, on));
+        L2O_TRY(hipStreamSynchronize(on));
+        if (*e->h_live == e->live && !scan) return (int)LOGO2OPT_OK;
+        e->live = *e->h_live;
+        return scan_done(e);
+    };
+    rc = next_local();
     uint32_t steps = 0;
-    while (steps < max_steps && e->live > 0) {
+    while (!rc && steps < max_steps && e->live_launch > 0) {
         const uint32_t k = std::min(sync_every, max_steps - steps);
-        int rc = issue_steps(e, k, sync_every);
-        if (rc) return rc;
+        rc = issue_steps(e, k, sync_every);
+        if (rc) break;
         steps += k;
-        L2O_TRY(hipMemcpyAsync(e->h_live, e->d_live, sizeof(unsigned), hipMemcpyDeviceToHost, e->stream));
-        L2O_TRY(hipStreamSynchronize(e->stream));
-        if (e->timing) {
-            rc = collect_timing(e);
-            if (rc) return rc;
-        }
-        const unsigned lv = *e->h_live;
-        if (lv != e->live) {
-            e->live = lv;
-            rc = scan_done(e);
-            if (rc) return rc;
-            // drop finished instances from the work lists once they are a
-            // noticeable share of the launched workgroups
-            if (e->live == 0 || e->live * 4 < e->live_at_build * 3) {
-                rc = rebuild_lists(e);
-                if (rc) return rc;
-            }
-        }
+        rc = check_live(e->stream);
+        if (!rc && e->timing) rc = collect_timing(e);
+        // drop finished instances from the work lists once they are a
+        // noticeable share of the launched workgroups
+        if (!rc && e->live_launch < e->live_at_build && e->live_launch * 4 < e->live_at_build * 3)
+            rc = rebuild_lists(e);
     }
+    while (local_running) {
+        const int rl = check_live(st, true);  // waits for the launch
+        local_running = false;
+        if (!rc) rc = rl;
+        if (!rc) rc = next_local();
+    }
+    if (rc) return rc;
     e->wall_ms += now_ms() - t0;
     if (live_out) *live_out = e->live;
     return LOGO2OPT_OK;
@@ -877,10 +1007,12 @@ int engine_create(int device, uint64_t budget, uint32_t max_slots, logo2opt_engi
     e->max_slots = max_slots;
     e->slots.resize(max_slots);
     if (const char *g = std::getenv("LOGO2OPT_GRAPHS")) e->graphs = std::strcmp(g, "0") != 0;
+    // the pools follow the instance records
+    const size_t pool_off = (sizeof(l2o_inst) * max_slots + 511) & ~(size_t)511;
+    const size_t pool_bytes = sizeof(unsigned long long) * L2O_POOL * ((size_t)max_slots + 1);
     bool ok = hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking) == hipSuccess &&
               hipMalloc(&e->d_arena, budget) == hipSuccess &&
-              hipMalloc(&e->d_insts, sizeof(l2o_inst) * max_slots) == hipSuccess &&
-              hipMalloc(&e->d_pool, sizeof(unsigned long long) * L2O_POOL * (max_slots + 1)) == hipSuccess &&
+              hipMalloc(&e->d_insts, pool_off + pool_bytes) == hipSuccess &&
               hipMalloc(&e->d_live, sizeof(unsigned)) == hipSuccess &&
               hipMalloc(&e->d_scratch, sizeof(unsigned long long) * 4) == hipSuccess &&
               hipHostMalloc(&e->h_live, sizeof(unsigned), hipHostMallocDefault) == hipSuccess &&
@@ -888,8 +1020,9 @@ int engine_create(int device, uint64_t budget, uint32_t max_slots, logo2opt_engi
               hipEventCreate(&e->ev0) == hipSuccess && hipEventCreate(&e->ev1) == hipSuccess;
     if (ok) {
         e->ar.init(e->d_arena, budget);
-        ok = hipMemsetAsync(e->d_insts, 0, sizeof(l2o_inst) * max_slots, e->stream) == hipSuccess &&
-             hipMemsetAsync(e->d_pool, 0xFF, sizeof(unsigned long long) * L2O_POOL * max_slots, e->stream) == hipSuccess &&
+        e->d_pool = (unsigned long long *)((char *)e->d_insts + pool_off);
+        // all ones: pools empty (L2O_SENTINEL), records in no phase and no group
+        ok = hipMemsetAsync(e->d_insts, 0xFF, pool_off + pool_bytes, e->stream) == hipSuccess &&
              hipMemsetAsync(e->d_live, 0, sizeof(unsigned), e->stream) == hipSuccess &&
              hipStreamSynchronize(e->stream) == hipSuccess;
     }
@@ -992,12 +1125,13 @@ int logo2opt_engine_destroy(logo2opt_engine *e)
     if (!e) return LOGO2OPT_EINVAL;
     (void)hipSetDevice(e->device);
     if (e->stream) (void)hipStreamSynchronize(e->stream);
+    if (e->lstream) (void)hipStreamSynchronize(e->lstream);
     drop_graph(e);
     if (e->d_sitems) (void)hipFree(e->d_sitems);
     if (e->d_aitems) (void)hipFree(e->d_aitems);
     if (e->d_arena) (void)hipFree(e->d_arena);
     if (e->d_insts) (void)hipFree(e->d_insts);
-    if (e->d_pool) (void)hipFree(e->d_pool);
+    if (e->d_lids) (void)hipFree(e->d_lids);
     if (e->d_live) (void)hipFree(e->d_live);
     if (e->d_scratch) (void)hipFree(e->d_scratch);
     if (e->h_live) (void)hipHostFree(e->h_live);
@@ -1006,6 +1140,7 @@ int logo2opt_engine_destroy(logo2opt_engine *e)
     if (e->ev1) (void)hipEventDestroy(e->ev1);
     for (hipEvent_t ev : e->tev) (void)hipEventDestroy(ev);
     if (e->stream) (void)hipStreamDestroy(e->stream);
+    if (e->lstream) (void)hipStreamDestroy(e->lstream);
     delete e;
     return LOGO2OPT_OK;
 }
@@ -1254,7 +1389,8 @@ int logo2opt_step(logo2opt_ctx *ctx, const uint32_t *route, logo2opt_best2_out *
     int rc = ctx_load(ctx, route, job, true);
     if (rc) return rc;
     e = ctx->e;  // ctx_load replaces the engine when it needs a larger one
-    rc = rebuild_lists(e);
+    rc = assign_local(e, false, false);
+    if (!rc) rc = rebuild_lists(e);
     if (rc) return rc;
     const double h1 = now_ms();
     L2O_TRY(hipEventRecord(e->ev0, e->stream));
@@ -1519,7 +1655,8 @@ int logo2opt_engine_time_sweep(logo2opt_engine *e, uint32_t sweeps, double *avg_
 {
     if (!e || !avg_ms || sweeps == 0) return LOGO2OPT_EINVAL;
     if (hipSetDevice(e->device) != hipSuccess) return LOGO2OPT_EDEVICE;
-    int rc = rebuild_lists(e);
+    int rc = assign_local(e, false, false);
+    if (!rc) rc = rebuild_lists(e);
     if (rc) return rc;
     for (const auto &g : e->groups)  // untimed first launch
         L2O_TRY(launch_group_sweep(e, g));
@@ -1560,7 +1697,8 @@ int logo2opt_time_sweep(logo2opt_ctx *ctx, const uint32_t *route, uint32_t sweep
     int rc = ctx_load(ctx, route, job, true);
     if (rc) return rc;
     e = ctx->e;  // ctx_load replaces the engine when it needs a larger one
-    rc = rebuild_lists(e);
+    rc = assign_local(e, false, false);
+    if (!rc) rc = rebuild_lists(e);
     if (rc) return rc;
     // one untimed launch (code object load, caches)
     for (const auto &g : e->groups)

@@ -109,6 +109,7 @@ __global__ __launch_bounds__(L2O_APPLY_THREADS) void k_apply(const l2o_apply_ite
     }
     pk = remap_key(pk, i, J, n);
     const unsigned long long pmin = wave_min_u64(pk);
+    const int cap = next_cap(pk, pmin);
     asm volatile("" ::"s"(pmin));  // the pool loads have returned before the barrier
     // Every wave of the workgroup has read key, parity and its sources once
     // all are past the barrier (each loaded value feeds a store issued before
@@ -141,6 +142,7 @@ __global__ __launch_bounds__(L2O_APPLY_THREADS) void k_apply(const l2o_apply_ite
             in->sweeps += 1;
             in->parity = par ^ 1;
             in->key = pmin;
+            in->cap = cap;
         }
     }
 }
@@ -252,6 +254,7 @@ __global__ __launch_bounds__(L2O_ILS_THREADS) void k_ils(l2o_inst *__restrict__ 
         in->parity = 0;
         in->rounds_done += 1;
         in->key = L2O_SENTINEL;
+        in->cap = -1;
         in->apply_done = 0;
         __threadfence();
         in->phase = L2O_LO;

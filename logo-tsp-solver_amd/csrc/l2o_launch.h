@@ -95,6 +95,12 @@ hipError_t launch_sweep(const sweep_cfg &cfg, const l2o_sweep_item *items, uint3
 hipError_t launch_apply(const l2o_apply_item *items, uint32_t nitems, l2o_inst *insts, unsigned *live,
                         hipStream_t stream);
 hipError_t launch_ils(l2o_inst *insts, uint32_t nslots, unsigned *live, hipStream_t stream);
+// `steps` sweeps of each of the instances ids[0 .. count), none larger than
+// max_n cities: one workgroup each (a chain of a group stops at its local
+// optimum, L2O_LO_DONE)
+hipError_t launch_local(int waves, const uint32_t *ids, uint32_t count, uint32_t max_n, l2o_inst *insts, unsigned *live,
+                        uint32_t steps, hipStream_t stream);
+uint32_t local_lds_bytes(uint32_t n, int waves);
 hipError_t launch_group(l2o_inst *insts, uint32_t nslots, unsigned *live, hipStream_t stream);
 hipError_t launch_length(const l2o_inst *insts, uint32_t slot, uint32_t n, unsigned long long *out,
                          hipStream_t stream);

@@ -176,6 +176,7 @@ extern "C" int logo2opt_step_noalloc(int device, uint32_t n, const logo2opt_city
     l2o::set_quant(in, mxx - mnx, mxy - mny);
     in.phase = L2O_LO;
     in.key = L2O_SENTINEL;
+    in.cap = -1;
 
     hipStream_t st = hipStreamPerThread;
 #define NA_TRY(call)                                      \

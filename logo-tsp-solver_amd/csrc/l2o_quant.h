@@ -82,12 +82,13 @@ __device__ __forceinline__ uint32_t rows_upto(int l)
 // sign bits of a pair of products: bit r of c0, bit 16 + r of c1
 __device__ __forceinline__ uint32_t sign_mask(const float16v &c0, const float16v &c1)
 {
-    uint32_t mask = 0;
+    uint32_t m0 = 0, m1 = 0;  // two chains
 #pragma unroll
-    for (int r = 15; r >= 0; --r) mask = __builtin_amdgcn_alignbit(mask, __float_as_uint(c1[r]), 31);
-#pragma unroll
-    for (int r = 15; r >= 0; --r) mask = __builtin_amdgcn_alignbit(mask, __float_as_uint(c0[r]), 31);
-    return mask;
+    for (int r = 15; r >= 0; --r) {
+        m0 = __builtin_amdgcn_alignbit(m0, __float_as_uint(c0[r]), 31);
+        m1 = __builtin_amdgcn_alignbit(m1, __float_as_uint(c1[r]), 31);
+    }
+    return m0 | m1 << 16;
 }
 
 // half of -C for the largest gain `cap` still worth an exact evaluation

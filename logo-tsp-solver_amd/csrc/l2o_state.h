@@ -70,6 +70,7 @@ struct l2o_inst {
     float est_scale;      // FP32 tier: D ~ sqrt(s) * est_scale + est_add
     float est_add;
     float qs, qox, qoy;   // matrix test: X ~ x qs + qox, Y ~ y qs + qoy,
+    int32_t cap;          // largest gain the next sweep evaluates (next_cap in l2o_device.h)
     float qk, qm;         // and E = ceil(D qk + qm) (set_quant in l2o_launch.h)
     unsigned long long stop_below;  // ILS: done once best_length < stop_below (0: never)
     unsigned long long *pool;       // L2O_POOL keys of known improving moves (L2O_SENTINEL: none)

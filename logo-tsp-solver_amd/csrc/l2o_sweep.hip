@@ -151,16 +151,14 @@ __device__ __forceinline__ void sweep_item(const l2o_sweep_item it, l2o_inst *__
         for (int m = 0; m < K; ++m) qc[m] = quant_edge(w0[m], v1[m].y, v1[m].x, qk, qm);
         qr = quant_edge(rw0, rv1.y, rv1.x, qk, qm);
     }
-    // cap = the largest gain still worth an exact evaluation: -1 (improving
-    // moves only) or the instance's best key so far, taken inclusively (it may
-    // come from a larger i: a tie at a smaller i wins)
-    auto key_now = [&]() __attribute__((always_inline)) -> unsigned long long {
-        return uniform_u64(__hip_atomic_load(&in->key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-    };
-    int cap = -1;
-    {
-        const unsigned long long g = key_now();
-        if (g != L2O_SENTINEL) cap = min(cap, key_gain(g));
+    // cap = the largest gain still worth an exact evaluation: the instance's,
+    // or without a known move the best key published so far, taken inclusively
+    // (it may come from a larger i: a tie at a smaller i wins)
+    const int cap0 = ci->cap;
+    int cap = cap0;
+    if (cap0 == -1) {
+        const unsigned long long g = uniform_u64(__hip_atomic_load(&in->key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        if (g != L2O_SENTINEL) cap = min(cap, worse_gain(key_gain(g)));
     }
     // half of -C (waves may start with different caps: each is a valid one)
     const float hc = half_cap(cap, qk);
@@ -230,6 +228,7 @@ __device__ __forceinline__ void sweep_item(const l2o_sweep_item it, l2o_inst *__
             }
             if (cnt == 0) break;
             asm volatile("" ::: "memory");
+            unsigned long long key = L2O_SENTINEL;
             if (lane < cnt) {
                 const uint32_t v = slist[lane];
                 const int a = a0 + (int)(v >> 12), b = bw + (int)(v & 0xFFFu);
@@ -241,13 +240,23 @@ __device__ __forceinline__ void sweep_item(const l2o_sweep_item it, l2o_inst *__
                     ++fb;
                     const int gain = exact_dist((int)A0.x, (int)A0.y, (int)B0.x, (int)B0.y, metric) +
                                      exact_dist((int)A1.x, (int)A1.y, (int)B1.x, (int)B1.y, metric) - da - db;
-                    if (gain < 0) {
-                        const uint32_t i = (uint32_t)(a + 1);
-                        const unsigned long long key = make_key(gain, i, (uint32_t)(b + 1));
-                        lbest = key < lbest ? key : lbest;
-                        atomicMin(&pool[(i * 0x9E3779B1u) >> 26], key);
-                    }
+                    if (gain < 0) key = make_key(gain, (uint32_t)(a + 1), (uint32_t)(b + 1));
                 }
+            }
+            // into the pool; of many, the best of each 16 lanes (atomics on one
+            // line take their turns, about 14 ns each)
+            const unsigned long long got = __ballot(key != L2O_SENTINEL);
+            if (got) {
+                lbest = key < lbest ? key : lbest;
+                if (__builtin_popcountll(got) > 16) {
+                    key = dpp_min_u64<0x111, 0xF>(key);
+                    key = dpp_min_u64<0x112, 0xF>(key);
+                    key = dpp_min_u64<0x114, 0xF>(key);
+                    key = dpp_min_u64<0x118, 0xF>(key);
+                    if ((lane & 15) != 15) key = L2O_SENTINEL;
+                }
+                if (key != L2O_SENTINEL)
+                    atomicMin(&pool[(((uint32_t)(key >> 20) & 0xFFFFFu) * 0x9E3779B1u) >> 26], key);
             }
             // what was not evaluated moves to the front of the list
             uint32_t rest = 0;
@@ -259,8 +268,8 @@ __device__ __forceinline__ void sweep_item(const l2o_sweep_item it, l2o_inst *__
             // publish an improvement at once: other waves tighten their cap
             if (__ballot(lbest < published)) {
                 published = wave_min_u64(lbest);
-                if (key_gain(published) < cap) {
-                    cap = key_gain(published);
+                if (cap0 == -1) {
+                    cap = min(cap, worse_gain(key_gain(published)));
                     thr = (float)cap + slack;
                 }
                 if (lane == 0) atomicMin(&in->key, published);

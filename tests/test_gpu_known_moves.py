@@ -54,3 +54,54 @@ def test_slot_reuse_after_removal_mid_search():
             np.testing.assert_array_equal(out["log"], log)
             assert out["length"] == Lo and out["route"].tolist() == r.tolist()
             e.remove(s)
+
+
+@pytest.mark.parametrize("n", [3, 4, 8, 63, 64, 65, 66, 129, 321, 799, 800, 801])
+def test_one_workgroup_searches(n):
+    """Sizes around the 32-edge blocks, the 64-edge pairs and the largest size
+    that one workgroup takes, as a search, in slices, and as an ILS job."""
+    xy = O.gen_uniform(n, 3000, n)
+    r0 = O.random_perm(n, n + 2)
+    r, Lo, moves, _, log = O.local_search(xy, r0, threads=THREADS)
+    with L.Engine(max_slots=3) as e:
+        co = L.coords_of(xy)
+        s = e.add(co, r0, log_cap=4096)
+        k = e.add(co, r0, log_cap=4096)
+        e.run(max_steps=moves // 2, sync_every=4)
+        assert e.result(s)["moves"] == moves // 2
+        while e.run(max_steps=7, sync_every=4):
+            pass
+        for slot in (s, k):  # (the second one starts with the first)
+            out = e.result(slot, n, log_cap=4096)
+            assert out["length"] == Lo and out["sweeps"] == moves + 1
+            np.testing.assert_array_equal(out["log"], log)
+            assert out["route"].tolist() == r.tolist()
+    if n >= 8:
+        for kick in (0, 1):
+            br, bl, hist, _ = O.ils(xy, r0, 9, 6, kick=("double_bridge", "reference")[kick], threads=THREADS)
+            with L.Context(L.coords_of(xy)) as ctx:
+                gr, gl, gh = ctx.ils(r0, 9, 6, kick)
+            assert gl == bl and gh.tolist() == list(hist) and gr.tolist() == br.tolist()
+
+
+def test_many_small_instances_and_chains():
+    """More than 64 instances (four waves each) beside larger ones, and chains
+    of one instance whose rounds alternate with the group's barrier."""
+    rng = np.random.default_rng(4)
+    jobs = [(int(n), int(s)) for n, s in zip(rng.integers(8, 900, 70), rng.integers(0, 1000, 70))] + [(1500, 5), (1300, 6)]
+    with L.Engine(max_slots=80) as e:
+        slots = []
+        for n, s in jobs:
+            xy = O.gen_uniform(n, 10**4, s)
+            slots.append((e.add(L.coords_of(xy), O.nn_tour(xy, 0)), xy, n))
+        assert e.run() == 0
+        for slot, xy, n in slots:
+            r, Lo, moves, _, _ = O.local_search(xy, O.nn_tour(xy, 0), threads=THREADS)
+            out = e.result(slot, n)
+            assert (out["length"], out["moves"]) == (Lo, moves) and out["route"].tolist() == r.tolist()
+    xy = O.gen_uniform(500, 10**4, 3)
+    r0 = O.random_perm(500, 4)
+    want = O.ils_multistart(xy, r0, 11, 7, 5)
+    with L.Context(L.coords_of(xy)) as ctx:
+        got = ctx.ils_multistart(r0, 11, 7, 5)
+    assert got[1] == want[1] and got[2].tolist() == list(want[2]) and got[0].tolist() == np.asarray(want[0]).tolist()
