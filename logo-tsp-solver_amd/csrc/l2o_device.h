@@ -109,6 +109,7 @@ __device__ __forceinline__ unsigned long long uniform_u64(unsigned long long v)
 // their relative direction, so the candidate keeps its gain at the mapped
 // positions; two edges of different sides would reconnect the other way.
 // L2O_SENTINEL if the candidate is gone.
+// (i = 0, J = n: no move.)
 __device__ __forceinline__ unsigned long long remap_key(unsigned long long key, uint32_t i, uint32_t J, uint32_t n)
 {
     const uint32_t i2 = (uint32_t)(key >> 20) & 0xFFFFFu, j2 = (uint32_t)key & 0xFFFFFu;
@@ -117,26 +118,6 @@ __device__ __forceinline__ unsigned long long remap_key(unsigned long long key, 
     const uint32_t e1 = to(i2), e2 = to(j2);
     if (key == L2O_SENTINEL || in1 != in2 || i2 == i || i2 == J || j2 == i || j2 == J) return L2O_SENTINEL;
     return (key & ~((1ull << 40) - 1)) | ((unsigned long long)min(e1, e2) << 20) | max(e1, e2);
-}
-
-// The largest gain the next sweep evaluates, given the pool on its tour (one
-// entry per lane) and the best entry: that one's gain while the pool holds
-// enough others, else a somewhat worse one, so that the sweep refills the pool
-// before it runs out (a move invalidates up to half of it, and a sweep without
-// a known move evaluates every improving candidate).
-#ifndef L2O_POOL_LOW
-#define L2O_POOL_LOW 16
-#endif
-#ifndef L2O_CAP_SHIFT
-#define L2O_CAP_SHIFT 3
-#endif
-__device__ __forceinline__ int worse_gain(int gain) { return min(gain - (gain >> L2O_CAP_SHIFT), -1); }
-__device__ __forceinline__ int next_cap(unsigned long long entry, unsigned long long best)
-{
-    const int left = __builtin_popcountll(__ballot(entry != L2O_SENTINEL));
-    if (best == L2O_SENTINEL) return -1;
-    const int gain = key_gain(best);
-    return left >= L2O_POOL_LOW ? gain : worse_gain(gain);
 }
 
 // point records in global memory (address space 1: the pointers come from
@@ -162,6 +143,25 @@ __device__ __forceinline__ void st_pt(gpt *P, uint32_t k, const l2o_pt r)
     P[k].w = r.w;
 }
 
+// The tour after a move (i, J), in terms of the one before:
+// r' = r[i..J-1] ++ r[i-1..0] ++ r[n-1..J] (twoOptLocalSolver.cpp:41-48).  Without
+// a move (L2O_KEY_NONE) i = 0, J = n: the identity.
+struct move_map {
+    int i, J, L, n;
+    __device__ __forceinline__ move_map(unsigned long long key, int n_)
+    {
+        n = n_;
+        i = key == L2O_KEY_NONE ? 0 : (int)((uint32_t)(key >> 20) & 0xFFFFFu);
+        J = key == L2O_KEY_NONE ? n : (int)((uint32_t)key & 0xFFFFFu);
+        L = J - i;
+    }
+    // position before the move of the city at k
+    __device__ __forceinline__ int src(int k) const { return k < L ? k + i : k < J ? J - 1 - k : n - 1 + J - k; }
+    // length of the edge k-1 -> k (k > 0) from l2o_pt.d of its ends before the
+    // move (d0 of src(k-1), d1 of src(k)) and of the new edge at L
+    __device__ __forceinline__ int len(int k, int d0, int d1, int dL) const { return k < L ? d1 : k == L ? dL : d0; }
+};
+
 __device__ __forceinline__ unsigned wave_sum_u32(unsigned v)
 {
 #pragma unroll
@@ -180,6 +180,30 @@ __device__ __forceinline__ int wave_max_i32(int v)
     v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x142, 0xA, 0xF, false));
     v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x143, 0xC, 0xF, false));
     return __builtin_amdgcn_readlane(v, 63);
+}
+
+// The largest gain the next sweep evaluates, given the pool (one entry per
+// lane) and the move (i, J) after it: the best gain of the entries that the move
+// leaves (see remap_key) while it leaves enough of them, else a somewhat worse
+// one, so that the sweep refills the pool before it runs out (a move invalidates
+// up to half of it, and a sweep without a known move evaluates every improving
+// candidate).
+#ifndef L2O_POOL_LOW
+#define L2O_POOL_LOW 16
+#endif
+#ifndef L2O_CAP_SHIFT
+#define L2O_CAP_SHIFT 3
+#endif
+__device__ __forceinline__ int worse_gain(int gain) { return min(gain - (gain >> L2O_CAP_SHIFT), -1); }
+__device__ __forceinline__ int next_cap(unsigned long long key, uint32_t i, uint32_t J)
+{
+    const uint32_t i2 = (uint32_t)(key >> 20) & 0xFFFFFu, j2 = (uint32_t)key & 0xFFFFFu;
+    const bool stays = key != L2O_SENTINEL && (i2 > i && i2 < J) == (j2 > i && j2 < J) && i2 != i && i2 != J &&
+                       j2 != i && j2 != J;
+    const unsigned long long left = __ballot(stays);
+    if (!left) return -1;
+    const int gain = -wave_max_i32(stays ? -key_gain(key) : 0);
+    return __builtin_popcountll(left) >= L2O_POOL_LOW ? gain : worse_gain(gain);
 }
 
 __device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long v)
@@ -249,6 +273,88 @@ __device__ __forceinline__ uint32_t kick_source(uint32_t k, uint32_t n, bool ref
     if (k < a + (c - b)) return b + (k - a);
     if (k < c) return a + (k - a - (c - b));
     return k;
+}
+
+// ---------------------------------------------------------------------------
+// the tour after a move, chunk of L2O_APPLY_CHUNK positions from k0: points, edge
+// lengths and city ids gathered from buffer `b` into the other one.  A thread's
+// elements are independent: the loads of four are issued before their stores.
+// ---------------------------------------------------------------------------
+template <int NTHR>
+__device__ __forceinline__ void copy_chunk(const __attribute__((address_space(4))) l2o_inst *ci, uint32_t b,
+                                           const move_map &mm, uint32_t metric, int k0)
+{
+    const gpt *P = (const gpt *)(b ? ci->pts[1] : ci->pts[0]);
+    gpt *Pn = (gpt *)(b ? ci->pts[0] : ci->pts[1]);
+    const gu32 *R = (const gu32 *)(b ? ci->tour[1] : ci->tour[0]);
+    gu32 *Rn = (gu32 *)(b ? ci->tour[0] : ci->tour[1]);
+    const int n = mm.n;
+    const bool moved = mm.L < n;
+    // the far ends of the two new edges: P[i] -> P[J] at position 0, P[J-1] -> P[i-1] at L
+    const l2o_pt endJ = ld_pt(P, moved ? mm.J : 0), endJ1 = ld_pt(P, mm.J - 1);
+    constexpr int PER = 4;
+    for (int c = 0; c < L2O_APPLY_CHUNK; c += PER * NTHR) {
+        l2o_pt p[PER];
+        int dq[PER];
+        uint32_t rid[PER];
+#pragma unroll
+        for (int e = 0; e < PER; ++e) {
+            const int k = min(k0 + c + (int)threadIdx.x + e * NTHR, n - 1);
+            const int s = mm.src(k);
+            const int de = k < mm.L ? s : s + 1 >= n ? 0 : s + 1;
+            p[e] = ld_pt(P, (uint32_t)s);
+            dq[e] = P[de].d;
+            rid[e] = R[s];
+        }
+#pragma unroll
+        for (int e = 0; e < PER; ++e) {
+            const int k = k0 + c + (int)threadIdx.x + e * NTHR;
+            if (c + (int)threadIdx.x + e * NTHR >= L2O_APPLY_CHUNK || k >= n) continue;
+            l2o_pt r = p[e];
+            r.d = dq[e];
+            if (moved && (k == 0 || k == mm.L)) {
+                const l2o_pt o = k == 0 ? endJ : endJ1;
+                r.d = exact_dist(r.x, r.y, o.x, o.y, metric);
+            }
+            st_pt(Pn, (uint32_t)k, r);
+            Rn[k] = rid[e];
+        }
+    }
+}
+
+// a local optimum found: the pool is left empty, the instance goes to its next
+// phase (one wave; `parity` is the buffer of its tour)
+__device__ __forceinline__ void local_optimum(l2o_inst *in, unsigned *live, uint32_t parity)
+{
+    const int lane = (int)threadIdx.x & 63;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) in->pool[r * L2O_POOL + lane] = L2O_SENTINEL;
+    if (lane == 0) {
+        in->sweeps += 1;
+        in->parity = parity;
+        if (in->ils_rounds == 0) {
+            in->phase = L2O_DONE;
+            atomicSub(live, 1u);
+        } else {
+            in->phase = L2O_LO_DONE;
+        }
+    }
+}
+
+// counters and log of an applied move (one thread)
+__device__ __forceinline__ void log_move(l2o_inst *in, unsigned long long key)
+{
+    const int gain = key_gain(key);
+    in->length += (unsigned long long)(long long)gain;
+    if (in->moves < in->log_cap) {
+        l2o_move m;
+        m.i = (uint32_t)(key >> 20) & 0xFFFFFu;
+        m.j = (uint32_t)key & 0xFFFFFu;
+        m.gain = gain;
+        in->log[in->moves] = m;
+    }
+    in->moves += 1;
+    in->sweeps += 1;
 }
 
 }  // namespace l2o

@@ -210,8 +210,8 @@ struct slot_t {
     bool done = false;
     bool done_reported = false;
     float slack = 1.0f;
-    // only single sweeps run on it: their candidates go to the spare pool (the
-    // row after the slots' ones), which no kernel reads
+    // only single sweeps run on it: their candidates go to the spare pool behind
+    // the slots' ones (row 0 only, which no sweep of theirs reads)
     bool sweep_only = false;
     bool local = false;  // runs in k_local (assigned at the start of a run)
     uint32_t group_lead = L2O_NO_GROUP;  // multi-start ILS group (first slot)
@@ -228,7 +228,7 @@ struct logo2opt_engine {
     uint32_t max_slots = 0;
     std::vector<slot_t> slots;
     l2o_inst *d_insts = nullptr;
-    unsigned long long *d_pool = nullptr;  // L2O_POOL keys per slot, and a spare row (behind d_insts)
+    unsigned long long *d_pool = nullptr;  // 4 rows of L2O_POOL keys per slot, and spare ones (behind d_insts)
     unsigned *d_live = nullptr;
     unsigned *h_live = nullptr;  // pinned
     unsigned live = 0;           // host mirror, valid between runs
@@ -238,8 +238,9 @@ struct logo2opt_engine {
     // work lists
     struct group {
         sweep_cfg cfg;
-        uint32_t off, count, id;
-        int mode;  // sweep variant (L2O_SWEEP_*)
+        uint32_t off, count;    // sweep items
+        uint32_t aoff, acount;  // apply items of the same instances
+        int mode;               // sweep variant (L2O_SWEEP_*)
     };
     std::vector<group> groups;
     l2o_sweep_item *d_sitems = nullptr;
@@ -267,9 +268,11 @@ struct logo2opt_engine {
     uint32_t local_chains = 0;  // chains of groups among them: slots [0, local_chains)
     bool use_local = false, local_to_end = false;  // of the last assignment
     unsigned live_launch = 0;  // live instances that run in steps
+    uint64_t step_pairs = 0;   // candidates of a step's sweeps, at the last rebuild
 
     hipGraphExec_t gexec = nullptr;
     uint32_t gsteps = 0;
+    bool grun = false;  // captured as one run
 
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     double wall_ms = 0.0, sweep_ms = 0.0;
@@ -387,7 +390,7 @@ int upload_instance(logo2opt_engine *e, int32_t id, const uint32_t *route, uint3
         p += al(8ull * ((uint64_t)s.job.ils_rounds + 1));
     }
     if (s.job.log_cap) in.log = (l2o_move *)p;
-    in.pool = e->d_pool + (size_t)L2O_POOL * (s.sweep_only ? e->max_slots : (uint32_t)id);
+    in.pool = e->d_pool + (size_t)4 * L2O_POOL * (s.sweep_only ? e->max_slots : (uint32_t)id);
     in.n = n;
     in.log_cap = s.job.log_cap;
     in.slack = s.slack;
@@ -409,8 +412,9 @@ int upload_instance(logo2opt_engine *e, int32_t id, const uint32_t *route, uint3
     }
     in.stop_below = s.job.ils_rounds ? s.job.stop_below : 0;
     in.phase = phase;
-    in.key = L2O_SENTINEL;
     in.cap = -1;
+    in.key[3] = L2O_KEY_NONE;
+    in.key[0] = L2O_SENTINEL;
     // SplitMix64 -> xoshiro256** state (same seeding as the workload generators)
     uint64_t x = s.job.seed;
     for (int k = 0; k < 4; ++k) {
@@ -482,14 +486,16 @@ uint64_t item_work(const l2o_sweep_item &it, const sweep_cfg &c, uint32_t n)
 }
 
 // Instances of at most this many cities run in k_local.  A few of them: up to
-// the size where one workgroup's step takes as long as a step's two launches
-// (707 cities 8.2 against 9.0 us, 1,000 cities 10.2 against 9.6 us; 200 cities
-// 4.0 against 11.3 us), with 16 waves, or 8 where there is little to share out.
-// Many fill the device by themselves: four waves each, which leave room for
-// several workgroups on a CU, and larger ones too, which then take no part in
-// the others' launches (512-instance batch: 346 ms without, 337 ms with them).
+// the size where one workgroup's step takes as long as a launch of sweeps does
+// (500 cities 5.8 against 6.3 us, 707 cities 8.2 us; 200 cities 4.0 us), an ILS
+// job up to the one where it takes as long as that and a k_ils launch; with 16
+// waves, or 8 where there is little to share out.  Many fill the device by
+// themselves: four waves each, which leave room for several workgroups on a CU,
+// and larger ones too, which then take no part in the others' launches
+// (512-instance batch: 346 ms without, 337 ms with them).
 #define L2O_LOCAL_MANY 64u
-#define L2O_LOCAL_MAX_N 800u
+#define L2O_LOCAL_MAX_N 512u
+#define L2O_LOCAL_ILS_MAX_N 800u
 #define L2O_LOCAL_MANY_MAX_N 1400u
 
 // which instances run in k_local, and its lists (no kernel may be running)
@@ -502,19 +508,20 @@ int assign_local(logo2opt_engine *e, bool use, bool to_end)
     for (const slot_t &s : e->slots)
         if (s.used && !s.done && s.n > (s.group_lead == L2O_NO_GROUP ? L2O_LOCAL_MAX_N : L2O_LOCAL_MANY_MAX_N))
             chains = false;
-    auto fits = [&](const slot_t &s, uint32_t max_n) {
-        return use && s.used && !s.done &&
-               (s.group_lead == L2O_NO_GROUP ? s.n <= max_n : chains && s.n <= L2O_LOCAL_MANY_MAX_N);
+    auto fits = [&](const slot_t &s, bool many) {
+        if (!use || !s.used || s.done) return false;
+        if (s.group_lead != L2O_NO_GROUP) return chains && s.n <= L2O_LOCAL_MANY_MAX_N;
+        return s.n <= (many ? L2O_LOCAL_MANY_MAX_N : s.job.ils_rounds ? L2O_LOCAL_ILS_MAX_N : L2O_LOCAL_MAX_N);
     };
     uint32_t count = 0;
-    for (uint32_t id = 0; id < e->max_slots; ++id) count += fits(e->slots[id], L2O_LOCAL_MANY_MAX_N) ? 1 : 0;
+    for (uint32_t id = 0; id < e->max_slots; ++id) count += fits(e->slots[id], true) ? 1 : 0;
     const bool many = count >= L2O_LOCAL_MANY;
     auto waves_for = [&](uint32_t n) { return many ? 4 : n > 128 ? 16 : 8; };
     std::vector<uint32_t> ids;
     e->local_chains = 0;
     for (uint32_t id = 0; id < e->max_slots; ++id) {
         slot_t &s = e->slots[id];
-        s.local = fits(s, many ? L2O_LOCAL_MANY_MAX_N : L2O_LOCAL_MAX_N);
+        s.local = fits(s, many);
         if (s.local) ids.push_back(id);
         if (s.local && s.group_lead != L2O_NO_GROUP) e->local_chains = id + 1;
     }
@@ -548,8 +555,11 @@ int assign_local(logo2opt_engine *e, bool use, bool to_end)
 // work lists of the steps: the live instances that do not run in k_local
 int rebuild_lists(logo2opt_engine *e)
 {
-    std::map<std::tuple<int, int, int, int>, std::vector<l2o_sweep_item>> by_cfg;
-    std::vector<l2o_apply_item> ai;
+    struct lists {
+        std::vector<l2o_sweep_item> sweep;
+        std::vector<l2o_apply_item> apply;
+    };
+    std::map<std::tuple<int, int, int, int>, lists> by_cfg;
     e->ils_grid = 0;
     e->any_ils = false;
     e->group_grid = 0;
@@ -563,6 +573,7 @@ int rebuild_lists(logo2opt_engine *e)
                      [&](uint32_t a, uint32_t b) { return e->slots[a].n > e->slots[b].n; });
     uint64_t all_pairs = 0;
     for (uint32_t id : order) all_pairs += pairs_of(e->slots[id].n);
+    e->step_pairs = all_pairs;
     const int table = order.size() >= L2O_BATCH_MIN && all_pairs >= L2O_BATCH_PAIRS ? 1 : 0;
     for (uint32_t id : order) {
         const slot_t &s = e->slots[id];
@@ -570,13 +581,14 @@ int rebuild_lists(logo2opt_engine *e)
         const sweep_cfg c = cfg_for(n, table);
         const bool pr = e->prune == LOGO2OPT_PRUNE_ALL || (e->prune == LOGO2OPT_PRUNE_AUTO && n >= L2O_PRUNE_AUTO_MIN_N);
         const int mode = pr ? l2o::L2O_SWEEP_PRUNE : l2o::L2O_SWEEP_FULL;
-        auto &v = by_cfg[std::make_tuple(c.k, c.t, c.waves, mode)];
+        lists &li = by_cfg[std::make_tuple(c.k, c.t, c.waves, mode)];
+        auto &v = li.sweep;
         // rows a <= n-4; the first tile of a row block starts at the
         // diagonal, b0 = a0 + 2
         for (uint32_t a0 = 0; a0 + 4 <= n; a0 += c.t)
             for (uint32_t b0 = a0 + 2; b0 + 2 <= n; b0 += c.cols()) v.push_back({id, a0, b0, (uint32_t)c.t});
         const uint32_t nch = (n + L2O_APPLY_CHUNK - 1) / L2O_APPLY_CHUNK;
-        for (uint32_t ch = 0; ch < nch; ++ch) ai.push_back({id, ch});
+        for (uint32_t ch = 0; ch < nch; ++ch) li.apply.push_back({id, ch});
         if (s.job.ils_rounds) {
             e->any_ils = true;
             e->ils_grid = std::max(e->ils_grid, id + 1);  // `order` is not by id
@@ -584,6 +596,7 @@ int rebuild_lists(logo2opt_engine *e)
         if (s.group_lead != L2O_NO_GROUP) e->group_grid = std::max(e->group_grid, id + 1);
     }
     std::vector<l2o_sweep_item> all;
+    std::vector<l2o_apply_item> ai;
     e->groups.clear();
     for (auto &kv : by_cfg) {
         const sweep_cfg c{std::get<0>(kv.first), std::get<1>(kv.first), std::get<2>(kv.first)};
@@ -599,7 +612,7 @@ int rebuild_lists(logo2opt_engine *e)
         // rows and the far ones are mostly skipped; the same order, which
         // spreads the near-diagonal tiles over the launch, measured faster
         // than issuing them first.)
-        auto &v = kv.second;
+        auto &v = kv.second.sweep;
         std::vector<uint64_t> work(v.size());
         // In a batch the first tile of each row block (at the diagonal) is
         // ordered as if it had L2O_DIAG_WEIGHT times its candidates: its rows
@@ -637,8 +650,10 @@ int rebuild_lists(logo2opt_engine *e)
         v.swap(sorted);
         const uint32_t cnt = (uint32_t)v.size();
         if (e->groups.size() >= L2O_MAX_GROUPS) return LOGO2OPT_EINVAL;
-        e->groups.push_back({c, (uint32_t)all.size(), cnt, (uint32_t)e->groups.size(), mode});
+        const auto &a = kv.second.apply;
+        e->groups.push_back({c, (uint32_t)all.size(), cnt, (uint32_t)ai.size(), (uint32_t)a.size(), mode});
         all.insert(all.end(), v.begin(), v.end());
+        ai.insert(ai.end(), a.begin(), a.end());
     }
     if (all.size() > e->sitems_cap) {
         if (e->d_sitems) (void)hipFree(e->d_sitems);
@@ -664,12 +679,14 @@ int rebuild_lists(logo2opt_engine *e)
     return LOGO2OPT_OK;
 }
 
-// the sweep launch of one group
-hipError_t launch_group_sweep(const logo2opt_engine *e, const logo2opt_engine::group &g)
+// the sweep of one group, by itself or as sweep t of a run
+hipError_t launch_group_sweep(const logo2opt_engine *e, const logo2opt_engine::group &g, bool run = false, uint32_t t = 0)
 {
-    return l2o::launch_sweep(g.cfg, e->d_sitems + g.off, g.count, e->d_insts, e->stream, g.mode);
+    return l2o::launch_sweep(g.cfg, e->d_sitems + g.off, g.count, e->d_aitems + g.aoff, g.acount, e->d_insts, e->d_live,
+                             run, t, e->stream, g.mode);
 }
 
+// a step by itself: sweep, apply, ILS bookkeeping
 int issue_step(logo2opt_engine *e)
 {
     const bool tm = e->timing && !e->groups.empty();
@@ -691,9 +708,24 @@ int issue_step(logo2opt_engine *e)
         L2O_TRY(hipEventRecord(e->tev[e->tev_used + 1], e->stream));
         e->tev_used += 2;
     }
-    L2O_TRY(l2o::launch_apply(e->d_aitems, e->n_aitems, e->d_insts, e->d_live, e->stream));
-    if (e->any_ils) L2O_TRY(l2o::launch_ils(e->d_insts, e->ils_grid, e->d_live, e->stream));
+    L2O_TRY(l2o::launch_apply(e->d_aitems, e->n_aitems, e->d_insts, e->d_live, 0, e->stream));
+    if (e->any_ils) L2O_TRY(l2o::launch_ils(e->d_insts, e->ils_grid, e->d_live, 0, e->stream));
     if (e->group_grid) L2O_TRY(l2o::launch_group(e->d_insts, e->group_grid, e->d_live, e->stream));
+    return LOGO2OPT_OK;
+}
+
+// a run of k sweeps, each applying the move of the one before
+int issue_run(logo2opt_engine *e, uint32_t k)
+{
+    for (uint32_t t = 0; t < k; ++t) {
+        for (const auto &g : e->groups) {
+            L2O_TRY(launch_group_sweep(e, g, true, t));
+            e->sweep_launches += 1;
+        }
+        if (e->any_ils && t) L2O_TRY(l2o::launch_ils(e->d_insts, e->ils_grid, e->d_live, t + 1, e->stream));
+    }
+    L2O_TRY(l2o::launch_apply(e->d_aitems, e->n_aitems, e->d_insts, e->d_live, k, e->stream));
+    if (e->any_ils) L2O_TRY(l2o::launch_ils(e->d_insts, e->ils_grid, e->d_live, 0, e->stream));
     return LOGO2OPT_OK;
 }
 
@@ -709,15 +741,31 @@ int collect_timing(logo2opt_engine *e)
     return LOGO2OPT_OK;
 }
 
-int issue_steps(logo2opt_engine *e, uint32_t k, uint32_t sync_every)
+// A run saves a step the apply launch (about 4 us) and costs its sweeps the
+// indexing through the move (3-8%): it pays while a step's sweeps are small
+// (7,397 cities 11.0 -> 7.9 us, 20,000 pruned 19.6 -> 17.0 us, 33,810 28 -> 27
+// us, 100,000 133 -> 136 us, a batch's first steps of 7e8 candidates 326 -> 332 ms).
+#define L2O_RUN_MAX_PAIRS 1000000000ull
+
+// k steps.  As one run where that does the same: the sweeps are not timed by
+// themselves, no group waits for its chains between steps, and no ILS job is cut
+// at a number of steps (in a run it is kicked one sweep after its local optimum,
+// so after k steps it may have done fewer sweeps).
+int issue_steps(logo2opt_engine *e, uint32_t k, uint32_t sync_every, bool to_end)
 {
+    const bool run = !e->timing && !e->group_grid && (!e->any_ils || to_end) && e->step_pairs <= L2O_RUN_MAX_PAIRS;
+    auto issue = [&]() {
+        if (run) return issue_run(e, k);
+        int rc = LOGO2OPT_OK;
+        for (uint32_t s = 0; s < k && rc == LOGO2OPT_OK; ++s) rc = issue_step(e);
+        return rc;
+    };
     if (sync_every > 1 && k == sync_every && !e->timing && e->graphs) {
-        if (!e->gexec || e->gsteps != k) {
+        if (!e->gexec || e->gsteps != k || e->grun != run) {
             drop_graph(e);
             hipGraph_t g;
             L2O_TRY(hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
-            int rc = LOGO2OPT_OK;
-            for (uint32_t s = 0; s < k && rc == LOGO2OPT_OK; ++s) rc = issue_step(e);
+            const int rc = issue();
             hipError_t ce = hipStreamEndCapture(e->stream, &g);
             if (rc != LOGO2OPT_OK) return rc;
             L2O_TRY(ce);
@@ -725,15 +773,12 @@ int issue_steps(logo2opt_engine *e, uint32_t k, uint32_t sync_every)
             (void)hipGraphDestroy(g);
             L2O_TRY(ie);
             e->gsteps = k;
+            e->grun = run;
         }
         L2O_TRY(hipGraphLaunch(e->gexec, e->stream));
         return LOGO2OPT_OK;
     }
-    for (uint32_t s = 0; s < k; ++s) {
-        int rc = issue_step(e);
-        if (rc) return rc;
-    }
-    return LOGO2OPT_OK;
+    return issue();
 }
 
 // refresh host knowledge of finished slots
@@ -763,9 +808,9 @@ int start_local(logo2opt_engine *e, uint32_t steps, hipStream_t st)
             L2O_TRY(l2o::launch_local(g.waves, e->d_lids + g.off, g.count, g.max_n, e->d_insts, e->d_live, steps,
                                       st));
         if (!e->local_chains) break;
-        L2O_TRY(l2o::launch_ils(e->d_insts, e->local_chains, e->d_live, st));    // accept, wait
+        L2O_TRY(l2o::launch_ils(e->d_insts, e->local_chains, e->d_live, 0, st));    // accept, wait
         L2O_TRY(l2o::launch_group(e->d_insts, e->local_chains, e->d_live, st));  // the round's best
-        L2O_TRY(l2o::launch_ils(e->d_insts, e->local_chains, e->d_live, st));    // kick
+        L2O_TRY(l2o::launch_ils(e->d_insts, e->local_chains, e->d_live, 0, st));    // kick
     }
     return LOGO2OPT_OK;
 }
@@ -811,7 +856,7 @@ int engine_run(logo2opt_engine *e, uint32_t max_steps, uint32_t sync_every, uint
     uint32_t steps = 0;
     while (!rc && steps < max_steps && e->live_launch > 0) {
         const uint32_t k = std::min(sync_every, max_steps - steps);
-        rc = issue_steps(e, k, sync_every);
+        rc = issue_steps(e, k, sync_every, to_end);
         if (rc) break;
         steps += k;
         rc = check_live(e->stream);
@@ -976,8 +1021,8 @@ int engine_remove(logo2opt_engine *e, int32_t id)
         if (in.phase != L2O_DONE) {
             // (a finished instance has left its pool empty)
             if (!s.sweep_only)
-                L2O_TRY(hipMemsetAsync(e->d_pool + (size_t)L2O_POOL * id, 0xFF,
-                                       sizeof(unsigned long long) * L2O_POOL, e->stream));
+                L2O_TRY(hipMemsetAsync(e->d_pool + (size_t)4 * L2O_POOL * id, 0xFF,
+                                       sizeof(unsigned long long) * 4 * L2O_POOL, e->stream));
             e->live -= 1;
             *e->h_live = e->live;
             L2O_TRY(hipMemcpyAsync(e->d_live, e->h_live, sizeof(unsigned), hipMemcpyHostToDevice, e->stream));
@@ -1009,7 +1054,7 @@ int engine_create(int device, uint64_t budget, uint32_t max_slots, logo2opt_engi
     if (const char *g = std::getenv("LOGO2OPT_GRAPHS")) e->graphs = std::strcmp(g, "0") != 0;
     // the pools follow the instance records
     const size_t pool_off = (sizeof(l2o_inst) * max_slots + 511) & ~(size_t)511;
-    const size_t pool_bytes = sizeof(unsigned long long) * L2O_POOL * ((size_t)max_slots + 1);
+    const size_t pool_bytes = sizeof(unsigned long long) * 4 * L2O_POOL * ((size_t)max_slots + 1);
     bool ok = hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking) == hipSuccess &&
               hipMalloc(&e->d_arena, budget) == hipSuccess &&
               hipMalloc(&e->d_insts, pool_off + pool_bytes) == hipSuccess &&
@@ -1405,13 +1450,13 @@ int logo2opt_step(logo2opt_ctx *ctx, const uint32_t *route, logo2opt_best2_out *
     L2O_TRY(hipMemcpyAsync(&in, e->d_insts + ctx->slot, sizeof(in), hipMemcpyDeviceToHost, e->stream));
     L2O_TRY(hipStreamSynchronize(e->stream));
     const double d1 = now_ms();
-    if (in.key == L2O_SENTINEL) {
+    if (in.key[0] == L2O_SENTINEL) {
         out->i = out->j = 0;
         out->minchange = 0;
     } else {
-        out->minchange = (int32_t)((long long)(in.key >> 40) - L2O_KEY_GAIN_BIAS);
-        out->i = (uint32_t)(in.key >> 20) & 0xFFFFFu;
-        out->j = (uint32_t)in.key & 0xFFFFFu;
+        out->minchange = (int32_t)((long long)(in.key[0] >> 40) - L2O_KEY_GAIN_BIAS);
+        out->i = (uint32_t)(in.key[0] >> 20) & 0xFFFFFu;
+        out->j = (uint32_t)in.key[0] & 0xFFFFFu;
     }
     ctx->sweep_ms += ms;
     if (t) {

@@ -10,139 +10,63 @@
 namespace l2o {
 
 // ---------------------------------------------------------------------------
-// apply: rotate+reverse gather of points, edge lengths and city ids
+// the end of a run of sweeps (l2o_state.h), or of one by itself (run = 0):
+// apply the last one's move
 // ---------------------------------------------------------------------------
-// twoOptLocalSolver.cpp:41-48 gives r' = r[i..J-1] ++ r[i-1..0] ++ r[n-1..J].
-// With L = J-i:  r'[k] = r[i+k] (k < L), r[i-1-(k-L)] (L <= k < L+i),
-// r[n-1+L+i-k] (k >= L+i).  Edge lengths move with their edges; only
-// D'[0] = d(P[i],P[J]) and D'[L] = d(P[J-1],P[i-1]) are new.
 __global__ __launch_bounds__(L2O_APPLY_THREADS) void k_apply(const l2o_apply_item *__restrict__ items,
                                                              l2o_inst *__restrict__ insts,
-                                                             unsigned *__restrict__ live)
+                                                             unsigned *__restrict__ live, uint32_t run)
 {
+    const uint32_t t = run ? run : 1;
     const l2o_apply_item it = items[blockIdx.x];
     l2o_inst *in = insts + it.inst;
-    if (in->phase != L2O_LO) return;
-    const unsigned long long key = in->key;
-    const uint32_t n = in->n;
+    const __attribute__((address_space(4))) l2o_inst *ci = (const __attribute__((address_space(4))) l2o_inst *)in;
+    const unsigned long long key = ci->key[(t - 1) & 3];
+    const uint32_t phase = ci->phase, b = (ci->base + t - 1) & 1;
+    const int n = (int)ci->n;
+    if (phase != L2O_LO) return;
     if (key == L2O_SENTINEL) {
         // no improving move: the local search has converged (sweeps = moves + 1)
-        if (it.chunk == 0 && threadIdx.x == 0) {
-            in->sweeps += 1;
-            if (in->ils_rounds == 0) {
-                in->phase = L2O_DONE;
-                atomicSub(live, 1u);
-            } else {
-                in->phase = L2O_LO_DONE;
-            }
-        }
+        if (it.chunk == 0 && threadIdx.x < 64) local_optimum(in, live, b);
         return;
     }
-    const int gain = key_gain(key);
-    const uint32_t i = (uint32_t)(key >> 20) & 0xFFFFFu;
-    const uint32_t J = (uint32_t)key & 0xFFFFFu;
-    const uint32_t L = J - i;
-    const uint32_t par = in->parity;
-    const uint32_t metric = in->metric;
-    const gpt *__restrict__ P = (const gpt *)in->pts[par];
-    const gu32 *__restrict__ R = (const gu32 *)in->tour[par];
-    gpt *__restrict__ Pn = (gpt *)in->pts[par ^ 1];
-    gu32 *__restrict__ Rn = (gu32 *)in->tour[par ^ 1];
-    const uint32_t k0 = it.chunk * L2O_APPLY_CHUNK;
-    const uint32_t k1 = min(n, k0 + L2O_APPLY_CHUNK);
-    // A thread's CHUNK/THREADS elements are independent: their sources are
-    // computed first and all their loads issued before the first store.
-    constexpr int PER = L2O_APPLY_CHUNK / L2O_APPLY_THREADS;
-    uint32_t src[PER], de[PER];  // source point; position whose edge length lands here
-    bool ok[PER];
-#pragma unroll
-    for (int e = 0; e < PER; ++e) {
-        const uint32_t k = k0 + threadIdx.x + e * L2O_APPLY_THREADS;
-        ok[e] = k < k1;
-        uint32_t sr, dr;
-        if (k < L) {
-            sr = i + k;
-            dr = sr;
-        } else if (k == L) {
-            sr = i - 1;
-            dr = sr;
-        } else if (k < L + i) {
-            sr = i - 1 - (k - L);
-            dr = sr + 1;
-        } else {
-            sr = n - 1 + L + i - k;
-            dr = sr + 1 == n ? 0 : sr + 1;
-        }
-        src[e] = ok[e] ? sr : 0;
-        de[e] = ok[e] ? dr : 0;
-    }
-    l2o_pt p[PER];
-    int32_t dq[PER];
-    uint32_t rid[PER];
+    const move_map mm(key, n);
     // wave 0: the pool entries on the new tour (stored by the last chunk)
     static_assert(L2O_POOL == 64, "one lane per pool entry");
-    unsigned long long *const pool = in->pool;
+    unsigned long long *const pool = ci->pool;
     unsigned long long pk = L2O_SENTINEL;
-    if (threadIdx.x < L2O_POOL) pk = pool[threadIdx.x];
-    // the far ends of the two new edges, loaded with the rest (one round trip)
-    const l2o_pt endJ = ld_pt(P, J), endJ1 = ld_pt(P, J - 1);
-#pragma unroll
-    for (int e = 0; e < PER; ++e) {
-        p[e] = ld_pt(P, src[e]);
-        dq[e] = P[de[e]].d;
-        rid[e] = R[src[e]];
+    if (threadIdx.x < L2O_POOL) {
+        pk = pool[((t - 1) & 3) * L2O_POOL + threadIdx.x];
+        if (!run) pk = min(pk, pool[3 * L2O_POOL + threadIdx.x]);  // (a run's sweeps carry it over)
     }
-#pragma unroll
-    for (int e = 0; e < PER; ++e) {
-        const uint32_t k = k0 + threadIdx.x + e * L2O_APPLY_THREADS;
-        if (!ok[e]) continue;
-        l2o_pt r = p[e];
-        if (k == 0 || k == L) {
-            // the two new edges: P[i] -> P[J] at position 0, P[J-1] -> P[i-1] at L
-            const l2o_pt o = k == 0 ? endJ : endJ1;
-            r.d = exact_dist(r.x, r.y, o.x, o.y, metric);
-        } else {
-            r.d = dq[e];
-        }
-        st_pt(Pn, k, r);
-        Rn[k] = rid[e];
-    }
-    pk = remap_key(pk, i, J, n);
-    const unsigned long long pmin = wave_min_u64(pk);
-    const int cap = next_cap(pk, pmin);
-    asm volatile("" ::"s"(pmin));  // the pool loads have returned before the barrier
-    // Every wave of the workgroup has read key, parity and its sources once
-    // all are past the barrier (each loaded value feeds a store issued before
-    // it), so the last chunk to count may commit the move.  No memory fence:
-    // nothing in this kernel reads the new buffers, and the next kernel sees
-    // them at the kernel boundary; the empty asm keeps the compiler from
-    // moving memory operations across the barrier.
+    copy_chunk<L2O_APPLY_THREADS>(ci, b, mm, ci->metric, (int)(it.chunk * L2O_APPLY_CHUNK));
+    pk = remap_key(pk, (uint32_t)mm.i, (uint32_t)mm.J, (uint32_t)n);
+    const int cap = next_cap(pk, 0, (uint32_t)n);
+    asm volatile("" ::"s"(cap));  // the pool loads have returned before the barrier
+    // Every wave of the workgroup has read key, base and its sources once all
+    // are past the barrier (each loaded value feeds a store issued before it),
+    // so the last chunk to count may commit the move.  No memory fence: nothing
+    // in this kernel reads the new buffers, and the next kernel sees them at the
+    // kernel boundary; the empty asm keeps the compiler from moving memory
+    // operations across the barrier.
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     if (threadIdx.x < 64) {
-        const uint32_t nch = (n + L2O_APPLY_CHUNK - 1) / L2O_APPLY_CHUNK;
+        const uint32_t nch = ((uint32_t)n + L2O_APPLY_CHUNK - 1) / L2O_APPLY_CHUNK;
         uint32_t prev = 0;
         if (threadIdx.x == 0) prev = atomicAdd(&in->apply_done, 1u);
         prev = (uint32_t)__builtin_amdgcn_readfirstlane((int)prev);
         if (prev != nch - 1) return;
-        // last chunk of this instance: commit the move
-        pool[threadIdx.x] = pk;
+        pool[3 * L2O_POOL + threadIdx.x] = pk;
+        pool[threadIdx.x] = L2O_SENTINEL;
         if (threadIdx.x == 0) {
             in->apply_done = 0;
-            in->length += (unsigned long long)(long long)gain;
-            if (in->moves < in->log_cap) {
-                l2o_move m;
-                m.i = i;
-                m.j = J;
-                m.gain = gain;
-                in->log[in->moves] = m;
-            }
-            in->moves += 1;
-            in->sweeps += 1;
-            in->parity = par ^ 1;
-            in->key = pmin;
+            in->parity = in->base = b ^ 1;
             in->cap = cap;
+            if (key != L2O_KEY_NONE) log_move(in, key);
+            in->key[3] = L2O_KEY_NONE;
+            in->key[0] = L2O_SENTINEL;
         }
     }
 }
@@ -157,7 +81,9 @@ __global__ __launch_bounds__(L2O_APPLY_THREADS) void k_apply(const l2o_apply_ite
 // and waits (L2O_WAIT) for k_group; at L2O_KICK it kicks the best tour of
 // `kick_src` that k_group chose.  While any chain of a group is at L2O_KICK,
 // all of them are, so no best buffer is written while a kick reads it.
-__global__ __launch_bounds__(L2O_ILS_THREADS) void k_ils(l2o_inst *__restrict__ insts, unsigned *__restrict__ live)
+// The kicked tour goes where the run's next sweep, tnext, reads it.
+__global__ __launch_bounds__(L2O_ILS_THREADS) void k_ils(l2o_inst *__restrict__ insts, unsigned *__restrict__ live,
+                                                         uint32_t tnext)
 {
     l2o_inst *in = insts + blockIdx.x;
     const uint32_t phase = in->phase;
@@ -219,15 +145,16 @@ __global__ __launch_bounds__(L2O_ILS_THREADS) void k_ils(l2o_inst *__restrict__ 
         }
         return;
     }
-    // new current tour = kick(best of the source), written to buffer 0
+    // new current tour = kick(best of the source), written to the next sweep's buffer
     const l2o_inst *src = grouped ? insts + in->kick_src : in;
     const l2o_pt *__restrict__ BP = src->bpts;
     const uint32_t *__restrict__ BR = src->btour;
     const uint32_t a = s_a, b = s_b, c = s_c;
     const bool ref = in->kick == 1;
     auto src_of = [&](uint32_t k) -> uint32_t { return kick_source(k, n, ref, a, b, c); };
-    l2o_pt *__restrict__ Pn = in->pts[0];
-    uint32_t *__restrict__ Rn = in->tour[0];
+    const uint32_t nb = (in->base + (tnext ? tnext - 1 : 0)) & 1;
+    l2o_pt *__restrict__ Pn = in->pts[nb];
+    uint32_t *__restrict__ Rn = in->tour[nb];
     const uint32_t metric = in->metric;
     unsigned long long sum = 0;
     for (uint32_t k = threadIdx.x; k < n; k += L2O_ILS_THREADS) {
@@ -251,10 +178,11 @@ __global__ __launch_bounds__(L2O_ILS_THREADS) void k_ils(l2o_inst *__restrict__ 
         unsigned long long L = 0;
         for (int k = 0; k < L2O_ILS_THREADS / 64; ++k) L += s_sum[k];
         in->length = L;
-        in->parity = 0;
-        in->rounds_done += 1;
-        in->key = L2O_SENTINEL;
+        in->parity = nb;
         in->cap = -1;
+        in->rounds_done += 1;
+        in->key[(tnext - 1) & 3] = L2O_KEY_NONE;
+        in->key[tnext & 3] = L2O_SENTINEL;
         in->apply_done = 0;
         __threadfence();
         in->phase = L2O_LO;
@@ -349,18 +277,18 @@ __global__ __launch_bounds__(256) void k_sqrt_ulp(uint32_t lo, uint32_t hi, unsi
 
 namespace l2o {
 
-hipError_t launch_apply(const l2o_apply_item *items, uint32_t nitems, l2o_inst *insts, unsigned *live,
+hipError_t launch_apply(const l2o_apply_item *items, uint32_t nitems, l2o_inst *insts, unsigned *live, uint32_t t,
                         hipStream_t stream)
 {
     if (nitems == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_apply, dim3(nitems), dim3(L2O_APPLY_THREADS), 0, stream, items, insts, live);
+    hipLaunchKernelGGL(k_apply, dim3(nitems), dim3(L2O_APPLY_THREADS), 0, stream, items, insts, live, t);
     return hipGetLastError();
 }
 
-hipError_t launch_ils(l2o_inst *insts, uint32_t nslots, unsigned *live, hipStream_t stream)
+hipError_t launch_ils(l2o_inst *insts, uint32_t nslots, unsigned *live, uint32_t tnext, hipStream_t stream)
 {
     if (nslots == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_ils, dim3(nslots), dim3(L2O_ILS_THREADS), 0, stream, insts, live);
+    hipLaunchKernelGGL(k_ils, dim3(nslots), dim3(L2O_ILS_THREADS), 0, stream, insts, live, tnext);
     return hipGetLastError();
 }
 

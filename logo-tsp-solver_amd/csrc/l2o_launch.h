@@ -89,12 +89,16 @@ int sweep_shapes(int (*out)[3], int cap);
 // Sweep variants (same results): every pair of tiles through the matrix test,
 // or only those that a bounding-box bound does not rule out
 enum { L2O_SWEEP_FULL = 0, L2O_SWEEP_PRUNE = 1 };
-// one workgroup per item, of the variant `mode`
+// one workgroup per item, of the variant `mode`: sweep t of a run (l2o_state.h),
+// with one workgroup per apply item of the same instances, or a sweep by itself
 hipError_t launch_sweep(const sweep_cfg &cfg, const l2o_sweep_item *items, uint32_t nitems,
-                        l2o_inst *insts, hipStream_t stream, int mode = L2O_SWEEP_FULL);
-hipError_t launch_apply(const l2o_apply_item *items, uint32_t nitems, l2o_inst *insts, unsigned *live,
+                        const l2o_apply_item *aitems, uint32_t na, l2o_inst *insts, unsigned *live, bool run,
+                        uint32_t t, hipStream_t stream, int mode);
+// the end of a run of t sweeps, or of a sweep by itself (t = 0)
+hipError_t launch_apply(const l2o_apply_item *items, uint32_t nitems, l2o_inst *insts, unsigned *live, uint32_t t,
                         hipStream_t stream);
-hipError_t launch_ils(l2o_inst *insts, uint32_t nslots, unsigned *live, hipStream_t stream);
+// ILS bookkeeping before sweep tnext of a run
+hipError_t launch_ils(l2o_inst *insts, uint32_t nslots, unsigned *live, uint32_t tnext, hipStream_t stream);
 // `steps` sweeps of each of the instances ids[0 .. count), none larger than
 // max_n cities: one workgroup each (a chain of a group stops at its local
 // optimum, L2O_LO_DONE)

@@ -128,9 +128,11 @@ __global__ __launch_bounds__(64 * NW) void k_local(const uint32_t *__restrict__ 
             const l2o_pt p = G[k];
             lds[k] = pack(p.x, p.y, p.d, p.w, R[k]);
         }
-        if (tid < L2O_POOL) s_pool[tid] = gpool[tid];
+        if (tid < L2O_POOL) s_pool[tid] = gpool[3 * L2O_POOL + tid];
     }
-    unsigned long long pmin = uniform_u64(in->key);  // the best known move of the current tour
+    // the best known move of the current tour, and the largest gain its sweep evaluates
+    const unsigned long long known = gpool[3 * L2O_POOL + lane];
+    unsigned long long pmin = wave_min_u64(known);
     int cap = (int)ci->cap;
     if (tid == 0) {
         s_key[0] = pmin;
@@ -273,7 +275,7 @@ __global__ __launch_bounds__(64 * NW) void k_local(const uint32_t *__restrict__ 
             }
             const unsigned long long pk = remap_key(s_pool[t * L2O_POOL + lane], (uint32_t)i, (uint32_t)J, (uint32_t)n);
             pmin = wave_min_u64(pk);
-            cap = next_cap(pk, pmin);
+            cap = next_cap(pk, 0, (uint32_t)n);
             if (w == 0) s_pool[t1 * L2O_POOL + lane] = pk;
             if (tid == 0) {
                 if (moves < log_cap) {
@@ -379,7 +381,7 @@ __global__ __launch_bounds__(64 * NW) void k_local(const uint32_t *__restrict__ 
     }
     if (w == 0) {
         // the pool of the current tour: the last sweep's, mapped (empty at the end)
-        gpool[lane] = done ? L2O_SENTINEL : s_pool[(sweeps & 1) * L2O_POOL + lane];
+        gpool[3 * L2O_POOL + lane] = done ? L2O_SENTINEL : s_pool[(sweeps & 1) * L2O_POOL + lane];
     }
     const unsigned wfb = wave_sum_u32(fb);
     if (lane == 0 && wfb) atomicAdd(&in->fallbacks, (unsigned long long)wfb);
@@ -389,7 +391,6 @@ __global__ __launch_bounds__(64 * NW) void k_local(const uint32_t *__restrict__ 
         in->length = length;
         in->moves = moves;
         in->sweeps += sweeps;
-        in->key = done ? L2O_SENTINEL : pmin;
         in->cap = done ? -1 : cap;
         if (done && chain) {
             in->phase = L2O_LO_DONE;

@@ -48,8 +48,8 @@ constexpr size_t NA_OFF_TOUR = NA_OFF_COORDS + al256(sizeof(logo2opt_city_coords
 constexpr size_t NA_OFF_PTS = NA_OFF_TOUR + al256(sizeof(uint32_t) * NA_MAX_N);
 constexpr size_t NA_OFF_ITEMS = NA_OFF_PTS + al256(sizeof(l2o_pt) * NA_MAX_N);
 constexpr size_t NA_OFF_INST = NA_OFF_ITEMS + al256(sizeof(l2o_sweep_item) * NA_MAX_ITEMS);
-constexpr size_t NA_OFF_POOL = NA_OFF_INST + al256(sizeof(l2o_inst));  // written by the sweep, not read here
-constexpr size_t NA_BYTES = NA_OFF_POOL + al256(sizeof(unsigned long long) * L2O_POOL);
+constexpr size_t NA_OFF_POOL = NA_OFF_INST + al256(sizeof(l2o_inst));
+constexpr size_t NA_BYTES = NA_OFF_POOL + al256(sizeof(unsigned long long) * 4 * L2O_POOL);
 
 }  // namespace
 
@@ -175,8 +175,12 @@ extern "C" int logo2opt_step_noalloc(int device, uint32_t n, const logo2opt_city
     in.est_add = metric == LOGO2OPT_METRIC_EUC_2D ? 0.0f : 0.5f;
     l2o::set_quant(in, mxx - mnx, mxy - mny);
     in.phase = L2O_LO;
-    in.key = L2O_SENTINEL;
     in.cap = -1;
+    in.key[3] = L2O_KEY_NONE;
+    in.key[0] = L2O_SENTINEL;
+
+    unsigned long long empty[4 * L2O_POOL];
+    std::memset(empty, 0xFF, sizeof(empty));
 
     hipStream_t st = hipStreamPerThread;
 #define NA_TRY(call)                                      \
@@ -186,15 +190,17 @@ extern "C" int logo2opt_step_noalloc(int device, uint32_t n, const logo2opt_city
     NA_TRY(hipMemcpyAsync(base + NA_OFF_COORDS, coords, sizeof(logo2opt_city_coords) * n, hipMemcpyHostToDevice, st));
     NA_TRY(hipMemcpyAsync(base + NA_OFF_TOUR, route, sizeof(uint32_t) * n, hipMemcpyHostToDevice, st));
     NA_TRY(hipMemcpyAsync(base + NA_OFF_INST, &in, sizeof(in), hipMemcpyHostToDevice, st));
+    NA_TRY(hipMemcpyAsync(base + NA_OFF_POOL, empty, sizeof(empty), hipMemcpyHostToDevice, st));
     hipLaunchKernelGGL(k_na_points, dim3((n + 255) / 256), dim3(256), 0, st, base, n, (uint32_t)metric, mnx, mny);
     NA_TRY(hipGetLastError());
     const uint32_t rblocks = (n - 4) / NA_T + 1;
     hipLaunchKernelGGL(k_na_items, dim3((rblocks + 63) / 64), dim3(64), 0, st, base, n);
     NA_TRY(hipGetLastError());
     NA_TRY(l2o::launch_sweep(l2o::sweep_cfg{NA_K, NA_T, NA_W}, (const l2o_sweep_item *)(base + NA_OFF_ITEMS),
-                             na_items(n), (l2o_inst *)(base + NA_OFF_INST), st, l2o::L2O_SWEEP_FULL));
+                             na_items(n), nullptr, 0, (l2o_inst *)(base + NA_OFF_INST), nullptr, false, 0, st,
+                             l2o::L2O_SWEEP_FULL));
     unsigned long long key = L2O_SENTINEL;
-    NA_TRY(hipMemcpyAsync(&key, base + NA_OFF_INST + offsetof(l2o_inst, key), sizeof(key), hipMemcpyDeviceToHost,
+    NA_TRY(hipMemcpyAsync(&key, base + NA_OFF_INST + offsetof(l2o_inst, key[0]), sizeof(key), hipMemcpyDeviceToHost,
                           st));
     NA_TRY(hipStreamSynchronize(st));
 #undef NA_TRY

@@ -70,16 +70,17 @@ struct l2o_inst {
     float est_scale;      // FP32 tier: D ~ sqrt(s) * est_scale + est_add
     float est_add;
     float qs, qox, qoy;   // matrix test: X ~ x qs + qox, Y ~ y qs + qoy,
-    int32_t cap;          // largest gain the next sweep evaluates (next_cap in l2o_device.h)
     float qk, qm;         // and E = ceil(D qk + qm) (set_quant in l2o_launch.h)
     unsigned long long stop_below;  // ILS: done once best_length < stop_below (0: never)
-    unsigned long long *pool;       // L2O_POOL keys of known improving moves (L2O_SENTINEL: none)
+    unsigned long long *pool;       // 4 rows of L2O_POOL keys of known improving moves (below)
     // ---- dynamic
     uint32_t phase;
-    uint32_t parity;
+    uint32_t parity;      // buffer of the current tour (outside of a run of sweeps)
+    uint32_t base;        // buffer of the tour that a run's first sweep reads (below)
+    int32_t cap;          // largest gain the sweep of T_0 evaluates (next_cap in l2o_device.h)
     uint32_t apply_done;  // last-workgroup counter of the apply kernel
     uint32_t rounds_done;
-    unsigned long long key;
+    unsigned long long key[4];
     unsigned long long length;
     unsigned long long best_length;
     unsigned long long moves;
@@ -104,9 +105,22 @@ struct l2o_apply_item {
     uint32_t chunk;
 };
 
+// A run of sweeps.  Sweep t of a run (t = 0, 1, ...) works on the tour T_t and
+// leaves its best move in key[t & 3].  T_0 is in buffer `base`; T_t (t > 0) is
+// the tour of buffer (base + t - 1) & 1 after the move key[(t-1) & 3], which the
+// sweep applies to every index it reads while some of its workgroups write T_t
+// to the other buffer.  So a move costs one launch.  key[(t-1) & 3] is
+// L2O_KEY_NONE where there is no move to apply (t = 0, or a new tour from a
+// kick) and L2O_SENTINEL where T_(t-1) was a local optimum.  Sweep t also
+// empties key and pool row t+1.  After the last sweep k_apply brings the tour
+// to a buffer of its own and the state back to t = 0: key[3] = L2O_KEY_NONE,
+// key[0] = L2O_SENTINEL, the pool in row 3, row 0 empty.
+#define L2O_KEY_NONE 0ull
+
 // Keys of improving candidates the sweeps have evaluated exactly, bucketed by
-// position.  k_apply carries them over to the next tour, so the next sweep
-// starts with the best of them as its key.  All L2O_SENTINEL at a local optimum.
+// position: row t & 3 for those of T_t.  They are carried over to the next tour,
+// whose sweep starts with the best of them as its bound.  All rows are
+// L2O_SENTINEL at a local optimum.
 #define L2O_POOL 64
 #define L2O_MAX_GROUPS 32  // distinct sweep tile shapes in one engine step
 #define L2O_APPLY_CHUNK 1024

@@ -86,15 +86,19 @@ __device__ __forceinline__ void edge_boxes(const qedge &q, float e, bool valid, 
 // keeps its columns' operands in registers; the rows stream through LDS in
 // chunks of one row per thread, the next chunk's points loaded while this one
 // is tested.
-template <int K, int WAVES, int MODE>
-__device__ __forceinline__ void sweep_item(const l2o_sweep_item it, l2o_inst *__restrict__ insts)
+// RUN: sweep t of a run (l2o_state.h), on the tour after the move of the sweep
+// before; otherwise t = 0 and the tour is the buffer's.
+template <int K, int WAVES, int MODE, bool RUN>
+__device__ __forceinline__ void sweep_item(const l2o_sweep_item it, l2o_inst *__restrict__ insts, uint32_t t_)
 {
+    const uint32_t t = RUN ? t_ : 0;
     l2o_inst *in = insts + it.inst;
     // The fields this kernel reads but no wave writes come in one batch of
     // scalar loads before any branch (constant address space: other kernels
     // and the host write them, and the scalar cache starts clean)
     const __attribute__((address_space(4))) l2o_inst *ci = (const __attribute__((address_space(4))) l2o_inst *)in;
-    const uint32_t phase = ci->phase, par = ci->parity;
+    const uint32_t phase = ci->phase, buf = (ci->base + (t ? t - 1 : 0)) & 1;
+    const unsigned long long kprev = RUN ? ci->key[(t - 1) & 3] : L2O_KEY_NONE;
     const int n = (int)ci->n;
     const float slack = ci->slack;
     const uint32_t metric = ci->metric;
@@ -102,10 +106,13 @@ __device__ __forceinline__ void sweep_item(const l2o_sweep_item it, l2o_inst *__
     const float qk = ci->qk, qm = ci->qm;
     l2o_pt *const p0 = ci->pts[0], *const p1 = ci->pts[1];
     unsigned long long *const pool = ci->pool;
-    asm volatile("" ::"s"(phase), "s"(par), "s"(n), "s"(slack), "s"(p0), "s"(p1), "s"(it.a0), "s"(it.b0),
+    asm volatile("" ::"s"(phase), "s"(buf), "s"(kprev), "s"(n), "s"(slack), "s"(p0), "s"(p1), "s"(it.a0), "s"(it.b0),
                  "s"(it.rows), "s"(metric), "s"(qk), "s"(pool));
-    if (phase != L2O_LO) return;
-    const gpt *__restrict__ P = (const gpt *)(par ? p1 : p0);
+    if (phase != L2O_LO || kprev == L2O_SENTINEL) return;
+    const gpt *__restrict__ P = (const gpt *)(buf ? p1 : p0);
+    // the tour of this sweep: that of the buffer after the move kprev
+    const move_map mm(kprev, n);
+    auto src = [&](int k) __attribute__((always_inline)) { return RUN ? mm.src(k) : k; };
 
     constexpr bool PRUNE = MODE == L2O_SWEEP_PRUNE;
     constexpr int NT = 2 * K;         // column tiles of a wave
@@ -131,33 +138,76 @@ __device__ __forceinline__ void sweep_item(const l2o_sweep_item it, l2o_inst *__
 
     typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
     typedef const __attribute__((address_space(1))) u32x2 *gdw;
-    auto dw = [&](int k) __attribute__((always_inline)) { return *(gdw)&P[min(k, n - 1)].d; };  // {d, w}
+    auto dw = [&](int k) __attribute__((always_inline)) { return *(gdw)&P[src(min(k, n - 1))].d; };  // {d, w}
     auto ld4 = [&](int k) __attribute__((always_inline)) {
-        return make_uint4((uint32_t)P[k].x, (uint32_t)P[k].y, (uint32_t)P[k].d, (uint32_t)P[k].w);
+        const int s = src(k);
+        return make_uint4((uint32_t)P[s].x, (uint32_t)P[s].y, (uint32_t)P[s].d, (uint32_t)P[s].w);
+    };
+    // the move's new edge at position L (the one at 0 is no candidate's)
+    int dL = 0;
+    if constexpr (RUN) {
+        const __attribute__((address_space(4))) l2o_pt *S = (const __attribute__((address_space(4))) l2o_pt *)(buf ? p1 : p0);
+        const int u = mm.J - 1, v = max(mm.i - 1, 0);
+        dL = exact_dist(S[u].x, S[u].y, S[v].x, S[v].y, metric);
+    }
+    // A range of positions mostly lies in one piece of the move: position k is then
+    // S k + O before it, and an edge's length its later (S = 1) or earlier end's.
+    struct piece {
+        int S, O;
+    };
+    auto len = [&](int k, int d0, int d1) __attribute__((always_inline)) { return RUN ? mm.len(k, d0, d1, dL) : d1; };
+    auto piece_of = [&](int lo, int hi) __attribute__((always_inline)) {  // S = 0: no single piece
+        piece r{0, 0};
+        if (!RUN) {
+            if (hi < n) r = {1, 0};
+        } else if (hi < n) {
+            if (hi < mm.L) r = {1, mm.i};
+            else if (lo >= mm.J) r = {-1, n - 1 + mm.J};
+            else if (lo >= mm.L && hi < mm.J) r = {-1, mm.J - 1};
+        }
+        return r;
+    };
+    // {d, w} of position k and of k + 1
+    struct ends {
+        u32x2 v0, v1;
+    };
+    auto load_edge = [&](const piece &r, int k) __attribute__((always_inline)) {
+        ends v;
+        if (r.S) {
+            const int s = RUN ? r.S * k + r.O : k;
+            v.v0 = *(gdw)&P[s].d;
+            v.v1 = *(gdw)&P[s + (RUN ? r.S : 1)].d;
+        } else {
+            v.v0 = dw(k);
+            v.v1 = dw(k + 1);
+        }
+        return v;
+    };
+    auto edge = [&](const piece &r, int k, const ends &v) __attribute__((always_inline)) {  // k -> k+1
+        const int d = !RUN || r.S > 0 ? (int)v.v1.x : r.S < 0 ? (int)v.v0.x : len(k + 1, (int)v.v0.x, (int)v.v1.x);
+        return quant_edge(v.v0.y, v.v1.y, (uint32_t)d, qk, qm);
     };
     // columns bw .. bw+WC-1 per wave, the first chunk of rows
     qedge qc[K], qr;
     {
-        uint32_t w0[K];
-        u32x2 v1[K];
+        const piece pc = piece_of(bw, bw + WC), pr = piece_of(a0, a0 + CH);
+        ends vc[K];
 #pragma unroll
-        for (int m = 0; m < K; ++m) {
-            w0[m] = dw(bw + 64 * m + lane).y;
-            v1[m] = dw(bw + 64 * m + lane + 1);
-        }
-        const uint32_t rw0 = dw(a0 + tid).y;
-        const u32x2 rv1 = dw(a0 + tid + 1);
+        for (int m = 0; m < K; ++m) vc[m] = load_edge(pc, bw + 64 * m + lane);
+        const ends vr = load_edge(pr, a0 + tid);
 #pragma unroll
-        for (int m = 0; m < K; ++m) qc[m] = quant_edge(w0[m], v1[m].y, v1[m].x, qk, qm);
-        qr = quant_edge(rw0, rv1.y, rv1.x, qk, qm);
+        for (int m = 0; m < K; ++m) qc[m] = edge(pc, bw + 64 * m + lane, vc[m]);
+        qr = edge(pr, a0 + tid, vr);
     }
     // cap = the largest gain still worth an exact evaluation: the instance's,
     // or without a known move the best key published so far, taken inclusively
     // (it may come from a larger i: a tie at a smaller i wins)
-    const int cap0 = ci->cap;
+    unsigned long long *const row = pool + (t & 3) * L2O_POOL;
+    const int cap0 = RUN ? next_cap(pool[((t - 1) & 3) * L2O_POOL + lane], (uint32_t)mm.i, (uint32_t)mm.J) : ci->cap;
     int cap = cap0;
     if (cap0 == -1) {
-        const unsigned long long g = uniform_u64(__hip_atomic_load(&in->key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        const unsigned long long g =
+            uniform_u64(__hip_atomic_load(&in->key[t & 3], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
         if (g != L2O_SENTINEL) cap = min(cap, worse_gain(key_gain(g)));
     }
     // half of -C (waves may start with different caps: each is a valid one)
@@ -233,7 +283,7 @@ __device__ __forceinline__ void sweep_item(const l2o_sweep_item it, l2o_inst *__
                 const uint32_t v = slist[lane];
                 const int a = a0 + (int)(v >> 12), b = bw + (int)(v & 0xFFFu);
                 const uint4 A0 = ld4(a), A1 = ld4(a + 1), B0 = ld4(b), B1 = ld4(b + 1);
-                const int da = (int)A1.z, db = (int)B1.z;
+                const int da = len(a + 1, (int)A0.z, (int)A1.z), db = len(b + 1, (int)B0.z, (int)B1.z);
                 const float w2 = (est_dist((int)A0.x, (int)A0.y, (int)B0.x, (int)B0.y, es, ea) +
                                   est_dist((int)A1.x, (int)A1.y, (int)B1.x, (int)B1.y, es, ea)) - (float)db;
                 if (w2 <= thr + (float)da) {
@@ -256,7 +306,7 @@ __device__ __forceinline__ void sweep_item(const l2o_sweep_item it, l2o_inst *__
                     if ((lane & 15) != 15) key = L2O_SENTINEL;
                 }
                 if (key != L2O_SENTINEL)
-                    atomicMin(&pool[(((uint32_t)(key >> 20) & 0xFFFFFu) * 0x9E3779B1u) >> 26], key);
+                    atomicMin(&row[(((uint32_t)(key >> 20) & 0xFFFFFu) * 0x9E3779B1u) >> 26], key);
             }
             // what was not evaluated moves to the front of the list
             uint32_t rest = 0;
@@ -272,7 +322,7 @@ __device__ __forceinline__ void sweep_item(const l2o_sweep_item it, l2o_inst *__
                     cap = min(cap, worse_gain(key_gain(published)));
                     thr = (float)cap + slack;
                 }
-                if (lane == 0) atomicMin(&in->key, published);
+                if (lane == 0) atomicMin(&in->key[t & 3], published);
             }
         }
         nh = 0;
@@ -298,12 +348,12 @@ __device__ __forceinline__ void sweep_item(const l2o_sweep_item it, l2o_inst *__
     };
     for (int c = 0, half = 0; c < rows; c += CH, half ^= 1) {
         // the next chunk's points, in flight while this one is tested
-        uint32_t nw0 = 0;
-        u32x2 nv1 = {0, 0};
+        ends nv{};
+        piece np{};
         const bool more = c + CH < rows;
         if (more) {
-            nw0 = dw(a0 + c + CH + tid).y;
-            nv1 = dw(a0 + c + CH + tid + 1);
+            np = piece_of(a0 + c + CH, a0 + c + 2 * CH);
+            nv = load_edge(np, a0 + c + CH + tid);
         }
         if constexpr (WAVES > 1) __syncthreads();
         asm volatile("" ::: "memory");
@@ -365,7 +415,7 @@ __device__ __forceinline__ void sweep_item(const l2o_sweep_item it, l2o_inst *__
             }
         }
         if (more) {
-            qr = quant_edge(nw0, nv1.y, nv1.x, qk, qm);
+            qr = edge(np, a0 + c + CH + tid, nv);
             stage_row(qr, c + CH + tid, half ^ 1);
         }
     }
@@ -377,11 +427,46 @@ __device__ __forceinline__ void sweep_item(const l2o_sweep_item it, l2o_inst *__
 
 // waves per SIMD that the columns' operands leave room for (8 K VGPRs and about 55)
 #define L2O_WPE(K) ((K) <= 2 ? 6 : (K) <= 4 ? 5 : (K) <= 6 ? 4 : 3)
-template <int K, int WAVES, int MODE>
-__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(L2O_WPE(K)))) void k_sweep(
-    const l2o_sweep_item *__restrict__ items, l2o_inst *__restrict__ insts)
+// In a run, the first workgroups of a launch (na of them) write the
+// sweep's tour to the other buffer and keep the books of the move they apply;
+// the first chunk of an instance also carries its pool over and empties the
+// next sweep's key and pool row.
+template <int NTHR>
+__device__ __forceinline__ void apply_item(const l2o_apply_item it, l2o_inst *__restrict__ insts,
+                                           unsigned *__restrict__ live, uint32_t t)
 {
-    sweep_item<K, WAVES, MODE>(items[blockIdx.x], insts);
+    l2o_inst *in = insts + it.inst;
+    const __attribute__((address_space(4))) l2o_inst *ci = (const __attribute__((address_space(4))) l2o_inst *)in;
+    const unsigned long long kprev = ci->key[(t - 1) & 3];
+    const uint32_t phase = ci->phase, buf = (ci->base + (t ? t - 1 : 0)) & 1;
+    if (phase != L2O_LO) return;
+    if (kprev == L2O_SENTINEL) {
+        // no improving move: the local search has converged (sweeps = moves + 1)
+        if (it.chunk == 0 && threadIdx.x < 64) local_optimum(in, live, buf);
+        return;
+    }
+    const move_map mm(kprev, (int)ci->n);
+    if (it.chunk == 0 && threadIdx.x < 64) {
+        unsigned long long *const pool = ci->pool;
+        const unsigned long long known = remap_key(pool[((t - 1) & 3) * L2O_POOL + threadIdx.x], (uint32_t)mm.i,
+                                                   (uint32_t)mm.J, (uint32_t)mm.n);
+        if (known != L2O_SENTINEL) atomicMin(&pool[(t & 3) * L2O_POOL + threadIdx.x], known);
+        pool[((t + 1) & 3) * L2O_POOL + threadIdx.x] = L2O_SENTINEL;
+        if (threadIdx.x == 0) {
+            in->key[(t + 1) & 3] = L2O_SENTINEL;
+            if (kprev != L2O_KEY_NONE) log_move(in, kprev);
+        }
+    }
+    if (t) copy_chunk<NTHR>(ci, buf, mm, ci->metric, (int)(it.chunk * L2O_APPLY_CHUNK));
+}
+
+template <int K, int WAVES, int MODE, bool RUN>
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(L2O_WPE(K)))) void k_sweep(
+    const l2o_sweep_item *__restrict__ items, const l2o_apply_item *__restrict__ aitems, uint32_t na,
+    l2o_inst *__restrict__ insts, unsigned *__restrict__ live, uint32_t t)
+{
+    if (RUN && blockIdx.x < na) apply_item<64 * WAVES>(aitems[blockIdx.x], insts, live, t);
+    else sweep_item<K, WAVES, MODE, RUN>(items[blockIdx.x - (RUN ? na : 0)], insts, t);
 }
 
 // column and wave counts compiled into the library, and the tile shapes {k, t,
@@ -394,17 +479,30 @@ static const int g_shapes[][3] = {
     {2, 64, 4}, {4, 64, 4}, {6, 64, 4}, {8, 64, 4}, {8, 128, 4}, {6, 128, 2}, {6, 160, 1}, {6, 128, 4}, {4, 256, 2},
     {4, 256, 4}, {2, 256, 4}, {2, 512, 4}, {4, 512, 4}};
 
-#define L2O_SWEEP_CASE(K_, W_)                                                                            \
-    if (cfg.k == K_ && cfg.waves == W_) {                                                                \
-        if (mode == L2O_SWEEP_PRUNE)                                                                      \
-            hipLaunchKernelGGL((k_sweep<K_, W_, L2O_SWEEP_PRUNE>), dim3(nitems), dim3(64 * W_), 0, stream, items, insts); \
-        else                                                                                              \
-            hipLaunchKernelGGL((k_sweep<K_, W_, L2O_SWEEP_FULL>), dim3(nitems), dim3(64 * W_), 0, stream, items, insts); \
-        return hipGetLastError();                                                                         \
+template <int K, int W, int MODE>
+static void launch_shape(uint32_t nitems, uint32_t na, bool run, hipStream_t stream, const l2o_sweep_item *items,
+                         const l2o_apply_item *aitems, l2o_inst *insts, unsigned *live, uint32_t t)
+{
+    if (run)
+        hipLaunchKernelGGL((k_sweep<K, W, MODE, true>), dim3(na + nitems), dim3(64 * W), 0, stream, items, aitems, na,
+                           insts, live, t);
+    else
+        hipLaunchKernelGGL((k_sweep<K, W, MODE, false>), dim3(nitems), dim3(64 * W), 0, stream, items, aitems, 0u, insts,
+                           live, 0u);
+}
+
+#define L2O_SWEEP_CASE(K_, W_)                                                                              \
+    if (cfg.k == K_ && cfg.waves == W_) {                                                                  \
+        if (mode == L2O_SWEEP_PRUNE)                                                                        \
+            launch_shape<K_, W_, L2O_SWEEP_PRUNE>(nitems, na, run, stream, items, aitems, insts, live, t);  \
+        else                                                                                                \
+            launch_shape<K_, W_, L2O_SWEEP_FULL>(nitems, na, run, stream, items, aitems, insts, live, t);   \
+        return hipGetLastError();                                                                           \
     }
 
 hipError_t launch_sweep(const sweep_cfg &cfg, const l2o_sweep_item *items, uint32_t nitems,
-                        l2o_inst *insts, hipStream_t stream, int mode)
+                        const l2o_apply_item *aitems, uint32_t na, l2o_inst *insts, unsigned *live, bool run,
+                        uint32_t t, hipStream_t stream, int mode)
 {
     if (nitems == 0) return hipSuccess;
     if (mode != L2O_SWEEP_FULL && mode != L2O_SWEEP_PRUNE) return hipErrorInvalidValue;

@@ -27,7 +27,7 @@ def test_move_log_with_ties(n, side, metric, prune):
     r, Lo, moves, sweeps, log = O.local_search(xy, r0, threads=THREADS, metric=metric)
     with L.Context(L.coords_of(xy), metric=metric) as ctx:
         ctx.set_pruning(prune)
-        for sync in (1, 64):
+        for sync in (1, 2, 3, 5, 64):
             out = ctx.optimize(r0, log_cap=1 << 14, sync_every=sync)
             np.testing.assert_array_equal(out["log"], log)
             assert out["length"] == Lo and out["route"].tolist() == r.tolist()
