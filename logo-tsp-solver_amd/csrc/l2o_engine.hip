@@ -552,6 +552,11 @@ int assign_local(logo2opt_engine *e, bool use, bool to_end)
     return LOGO2OPT_OK;
 }
 
+bool prunes(const logo2opt_engine *e, uint32_t n)
+{
+    return e->prune == LOGO2OPT_PRUNE_ALL || (e->prune == LOGO2OPT_PRUNE_AUTO && n >= L2O_PRUNE_AUTO_MIN_N);
+}
+
 // work lists of the steps: the live instances that do not run in k_local
 int rebuild_lists(logo2opt_engine *e)
 {
@@ -573,14 +578,15 @@ int rebuild_lists(logo2opt_engine *e)
                      [&](uint32_t a, uint32_t b) { return e->slots[a].n > e->slots[b].n; });
     uint64_t all_pairs = 0;
     for (uint32_t id : order) all_pairs += pairs_of(e->slots[id].n);
-    e->step_pairs = all_pairs;
+    // (a pruned sweep tests fewer: 60,000 cities take 35.5 us either way, 100,000 73 us in a run, 69 us not)
+    e->step_pairs = 0;
+    for (uint32_t id : order) e->step_pairs += pairs_of(e->slots[id].n) / (prunes(e, e->slots[id].n) ? 4 : 1);
     const int table = order.size() >= L2O_BATCH_MIN && all_pairs >= L2O_BATCH_PAIRS ? 1 : 0;
     for (uint32_t id : order) {
         const slot_t &s = e->slots[id];
         const uint32_t n = s.n;
         const sweep_cfg c = cfg_for(n, table);
-        const bool pr = e->prune == LOGO2OPT_PRUNE_ALL || (e->prune == LOGO2OPT_PRUNE_AUTO && n >= L2O_PRUNE_AUTO_MIN_N);
-        const int mode = pr ? l2o::L2O_SWEEP_PRUNE : l2o::L2O_SWEEP_FULL;
+        const int mode = prunes(e, n) ? l2o::L2O_SWEEP_PRUNE : l2o::L2O_SWEEP_FULL;
         lists &li = by_cfg[std::make_tuple(c.k, c.t, c.waves, mode)];
         auto &v = li.sweep;
         // rows a <= n-4; the first tile of a row block starts at the

@@ -54,32 +54,49 @@
 
 namespace l2o {
 
-// maximum over each half of the wave, in lanes 31 and 63 (the others hold partial ones)
-__device__ __forceinline__ float half_max_f32(float v)
+// maximum over each half of the wave of a pair of FP16 numbers, in lanes 31 and
+// 63 (the others hold partial ones)
+__device__ __forceinline__ uint32_t half_max_pk(uint32_t v)
 {
-    auto step = [](float x, int y) { return __builtin_fmaxf(x, __int_as_float(y)); };
-    v = step(v, __builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), 0x111, 0xF, 0xF, false));
-    v = step(v, __builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), 0x112, 0xF, 0xF, false));
-    v = step(v, __builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), 0x114, 0xF, 0xF, false));
-    v = step(v, __builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), 0x118, 0xF, 0xF, false));
-    v = step(v, __builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), 0x142, 0xA, 0xF, false));
+    auto step = [](uint32_t x, int y) {
+        return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(half2v, x),
+                                                                      __builtin_bit_cast(half2v, (uint32_t)y)));
+    };
+    v = step(v, __builtin_amdgcn_update_dpp((int)v, (int)v, 0x111, 0xF, 0xF, false));
+    v = step(v, __builtin_amdgcn_update_dpp((int)v, (int)v, 0x112, 0xF, 0xF, false));
+    v = step(v, __builtin_amdgcn_update_dpp((int)v, (int)v, 0x114, 0xF, 0xF, false));
+    v = step(v, __builtin_amdgcn_update_dpp((int)v, (int)v, 0x118, 0xF, 0xF, false));
+    v = step(v, __builtin_amdgcn_update_dpp((int)v, (int)v, 0x142, 0xA, 0xF, false));
     return v;
 }
 
 // Box of the 32 edges of each half of the wave, both ends of the valid ones:
-// {-min X, max X, -min Y, max Y} and the largest E'; lanes 31 and 63 write it
-#define L2O_BOX_NONE (-1e6f)
-__device__ __forceinline__ void edge_boxes(const qedge &q, float e, bool valid, int lane, float *out)
+// {max X, max Y}, {-min X, -min Y} and the largest E' (pairs of FP16 whole
+// numbers); lanes 31 and 63 write it
+__device__ __forceinline__ void edge_boxes(const qedge &q, float hc, bool valid, int lane, uint4 *out)
 {
     const half2v a = __builtin_bit_cast(half2v, q.p0), b = __builtin_bit_cast(half2v, q.p1);
-    const float x0 = (float)a[0], y0 = (float)a[1], x1 = (float)b[0], y1 = (float)b[1];
-    const float v[5] = {-__builtin_fminf(x0, x1), __builtin_fmaxf(x0, x1), -__builtin_fminf(y0, y1),
-                        __builtin_fmaxf(y0, y1), e};
-#pragma unroll
-    for (int k = 0; k < 5; ++k) {
-        const float m = half_max_f32(valid ? v[k] : L2O_BOX_NONE);
-        if ((lane & 31) == 31) out[5 * (lane >> 5) + k] = m;
-    }
+    const uint32_t none = 0xE800E800u;  // {-2048, -2048}
+    const uint32_t hi = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(a, b));
+    const uint32_t lo = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(-a, -b));
+    uint4 r;
+    r.x = half_max_pk(valid ? hi : none);
+    r.y = half_max_pk(valid ? lo : none);
+    r.z = half_max_pk(valid ? pk16(__builtin_fmaxf(q.e - hc, 0.0f), 0.0f) : none);
+    r.w = 0;
+    if ((lane & 31) == 31) out[lane >> 5] = r;
+}
+
+// whether a candidate of a row block and a column tile can pass: its |U - V|^2 is
+// at least twice the squared distance of the boxes (both ends of an edge lie in
+// its box) and its E'_a + E'_b at most the sum of the largest
+__device__ __forceinline__ bool boxes_meet(const uint4 &r, const uint4 &c)
+{
+    auto h2 = [](uint32_t v) { return __builtin_bit_cast(half2v, v); };
+    const half2v zero = {(_Float16)0.0f, (_Float16)0.0f};
+    const half2v g = __builtin_elementwise_max(__builtin_elementwise_max(-(h2(r.y) + h2(c.x)), -(h2(c.y) + h2(r.x))), zero);
+    const float s = (float)h2(r.z)[0] + (float)h2(c.z)[0];
+    return s >= 0.0f && 2.0f * __builtin_amdgcn_fdot2(g, g, 0.0f, false) <= s * s;
 }
 
 // One work item: rows [a0, a0 + rows) and the 64 K WAVES columns from b0.  A wave
@@ -88,6 +105,7 @@ __device__ __forceinline__ void edge_boxes(const qedge &q, float e, bool valid, 
 // is tested.
 // RUN: sweep t of a run (l2o_state.h), on the tour after the move of the sweep
 // before; otherwise t = 0 and the tour is the buffer's.
+#define L2O_SWEEP_MAX_T 512
 template <int K, int WAVES, int MODE, bool RUN>
 __device__ __forceinline__ void sweep_item(const l2o_sweep_item it, l2o_inst *__restrict__ insts, uint32_t t_)
 {
@@ -124,8 +142,8 @@ __device__ __forceinline__ void sweep_item(const l2o_sweep_item it, l2o_inst *__
     __shared__ uint32_t s_nh[WAVES * WC];
     __shared__ uint32_t s_list[WAVES][128];
     __shared__ uint32_t s_hdr[WAVES][HCAP];
-    __shared__ float s_rbox[PRUNE ? 2 * 2 * WAVES * 5 : 1];
-    __shared__ float s_cbox[PRUNE ? WAVES * NT * 5 : 1];
+    __shared__ uint4 s_rbox[PRUNE ? L2O_SWEEP_MAX_T / 32 + 2 * WAVES : 1], s_cbox[PRUNE ? WAVES * NT : 1];
+    __shared__ int s_any[PRUNE ? WAVES : 1];
     const int a0 = (int)it.a0;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int tid = (int)threadIdx.x;
@@ -214,6 +232,46 @@ __device__ __forceinline__ void sweep_item(const l2o_sweep_item it, l2o_inst *__
     const float hc = half_cap(cap, qk);
     float thr = (float)cap + slack;  // tier 2
 
+    // PRUNE: the boxes of the columns and of all rows; an item without a pair of
+    // tiles whose boxes meet ends here, before any operand is made (60,000
+    // cities: 44.3 -> 35.5 us a step, most items end here; with five FP32
+    // maxima a box and the operands made first they spent 700 VALU instructions
+    // a wave)
+    // (bit q K + p of live_of(c): row block q of the chunk from c, column pair p)
+    auto live_of = [&](int c) __attribute__((always_inline)) -> unsigned long long {
+        const int q = lane / K, p = lane % K;
+        bool ok = false;
+        if (q < 2 * WAVES && c + 32 * q < rows && bw + 64 * p + 63 >= a0 + c + 32 * q + 2) {
+            const uint4 r = s_rbox[c / 32 + q], *cb = s_cbox + w * NT + 2 * p;
+            ok = boxes_meet(r, cb[0]) || boxes_meet(r, cb[1]);
+        }
+        return __ballot(ok);
+    };
+    bool wave_live = true;
+    if constexpr (PRUNE) {
+#pragma unroll
+        for (int m = 0; m < K; ++m) edge_boxes(qc[m], hc, bw + 64 * m + lane <= n - 2, lane, s_cbox + w * NT + 2 * m);
+        edge_boxes(qr, hc, tid < rows, lane, s_rbox + 2 * w);
+        for (int c = CH; c < rows; c += CH) {
+            const piece pr = piece_of(a0 + c, a0 + c + CH);
+            const qedge q = edge(pr, a0 + c + tid, load_edge(pr, a0 + c + tid));
+            edge_boxes(q, hc, c + tid < rows, lane, s_rbox + c / 32 + 2 * w);
+        }
+        if constexpr (WAVES > 1) __syncthreads();
+        asm volatile("" ::: "memory");
+        wave_live = false;
+        for (int c = 0; c < rows; c += CH) wave_live = wave_live || live_of(c) != 0;
+        bool item_live = wave_live;
+        if constexpr (WAVES > 1) {
+            if (lane == 0) s_any[w] = wave_live;
+            __syncthreads();
+            item_live = false;
+#pragma unroll
+            for (int q = 0; q < WAVES; ++q) item_live = item_live || __builtin_amdgcn_readfirstlane(s_any[q]) != 0;
+        }
+        if (!item_live) return;
+    }
+
     const bool upper = lane >= 32;
     half8 B[NT];
     uint4 *const scol = s_col + w * WC;
@@ -224,7 +282,6 @@ __device__ __forceinline__ void sweep_item(const l2o_sweep_item it, l2o_inst *__
         const qterms t = edge_terms(qc[m], hc, valid);
         scol[64 * m + lane] = col_record(qc[m], t);
         snh[64 * m + lane] = col_upper(t);
-        if constexpr (PRUNE) edge_boxes(qc[m], t.e, valid, lane, s_cbox + 5 * (w * NT + 2 * m));
     }
     asm volatile("" ::: "memory");  // (the wave's own columns: LDS keeps its order)
 #pragma unroll
@@ -242,7 +299,6 @@ __device__ __forceinline__ void sweep_item(const l2o_sweep_item it, l2o_inst *__
         const bool valid = r < rows;
         const qterms t = edge_terms(q, hc, valid);
         s_row[half * CH + tid] = row_record(q, t);
-        if constexpr (PRUNE) edge_boxes(q, t.e, valid, lane, s_rbox + 5 * (half * 2 * WAVES + 2 * w));
     };
     stage_row(qr, tid, 0);
     if (tid == 0) s_row[2 * CH] = row_const();
@@ -357,27 +413,7 @@ __device__ __forceinline__ void sweep_item(const l2o_sweep_item it, l2o_inst *__
         }
         if constexpr (WAVES > 1) __syncthreads();
         asm volatile("" ::: "memory");
-        unsigned long long live = ~0ull;
-        if constexpr (PRUNE) {
-            // lane l tests pair (q, p) = (l / K, l mod K) of a row block and two
-            // column tiles by their boxes: every candidate has |U - V|^2 at
-            // least twice the squared distance of the boxes (both ends of an
-            // edge lie in its box) and E'_a + E'_b at most the sum of the largest
-            const int q = lane / K, p = lane % K;
-            bool ok = false;
-            if (q < 2 * WAVES && c + 32 * q < rows && bw + 64 * p + 63 >= a0 + c + 32 * q + 2) {
-                const float *rb = s_rbox + 5 * (half * 2 * WAVES + q);
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const float *cb = s_cbox + 5 * (w * NT + 2 * p + h);
-                    const float dx = __builtin_fmaxf(__builtin_fmaxf(-rb[0] - cb[1], -cb[0] - rb[1]), 0.0f);
-                    const float dy = __builtin_fmaxf(__builtin_fmaxf(-rb[2] - cb[3], -cb[2] - rb[3]), 0.0f);
-                    const float s = rb[4] + cb[4];
-                    ok = ok || (s >= 0.0f && 2.0f * (dx * dx + dy * dy) <= s * s);
-                }
-            }
-            live = __ballot(ok);
-        }
+        const unsigned long long live = !PRUNE ? ~0ull : wave_live ? live_of(c) : 0ull;
         // rows of the chunk that this wave's columns see
         const int cr = min(min(rows - c, CH), min(bw + WC - 1, n - 2) - 1 - a0 - c);
         const int nq = bw > n - 2 ? 0 : (cr + 31) >> 5;
@@ -473,7 +509,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(L2O_
 // waves} the autotuner chooses among per n bucket (t, the rows of an item, is
 // up to the host)
 #define L2O_SWEEP_KERNELS(X) X(1, 1) X(2, 1) X(4, 1) X(6, 1) X(8, 1) X(4, 2) X(6, 2) X(8, 2) X(2, 4) X(4, 4) X(6, 4) X(8, 4)
-static const int g_shapes[][3] = {
+static const int g_shapes[][3] = {  // t <= L2O_SWEEP_MAX_T
     {1, 32, 1}, {1, 64, 1}, {2, 64, 1}, {2, 128, 1}, {4, 64, 1}, {4, 128, 1}, {4, 256, 1}, {6, 64, 1}, {6, 128, 1},
     {8, 64, 1}, {8, 128, 1}, {8, 256, 1}, {4, 64, 2}, {4, 128, 2}, {6, 64, 2}, {8, 64, 2}, {8, 128, 2}, {8, 256, 2},
     {2, 64, 4}, {4, 64, 4}, {6, 64, 4}, {8, 64, 4}, {8, 128, 4}, {6, 128, 2}, {6, 160, 1}, {6, 128, 4}, {4, 256, 2},
