@@ -192,24 +192,26 @@ struct arena {
     }
 };
 
-// exact metric length of the edge a -> b on the host (same function as the kernels)
-inline uint32_t dist_i(const int32_t *xy, uint32_t a, uint32_t b, uint32_t metric)
-{
-    const int64_t dx = (int64_t)xy[2 * a] - xy[2 * b], dy = (int64_t)xy[2 * a + 1] - xy[2 * b + 1];
-    return (uint32_t)l2o::metric_dist((long long)(dx * dx + dy * dy), metric);
-}
-
 uint64_t pairs_of(uint32_t n) { return n >= 4 ? (uint64_t)(n - 2) * (uint64_t)(n - 3) / 2 : 0; }
+
+// an instance's cities: translated integer coordinates, their spans, and the
+// bound on |exact gain - FP32 estimate|
+struct cities {
+    std::vector<int32_t> xy;
+    int32_t span_x = 0, span_y = 0;
+    float slack = 1.0f;
+};
 
 struct slot_t {
     bool used = false;
     uint32_t n = 0;
     uint64_t off = 0, bytes = 0;
     logo2opt_job job{};
-    std::vector<int32_t> xy;  // translated integer coordinates
     bool done = false;
     bool done_reported = false;
-    float slack = 1.0f;
+    // counters of its record, as last read (`counted`: nothing has run since)
+    bool counted = false;
+    uint64_t sweeps = 0, moves = 0, fallbacks = 0;
     // only single sweeps run on it: their candidates go to the spare pool behind
     // the slots' ones (row 0 only, which no sweep of theirs reads)
     bool sweep_only = false;
@@ -233,7 +235,9 @@ struct logo2opt_engine {
     unsigned *h_live = nullptr;  // pinned
     unsigned live = 0;           // host mirror, valid between runs
     unsigned long long *d_scratch = nullptr;
-    unsigned long long *h_scratch = nullptr;  // pinned
+    unsigned long long *h_scratch = nullptr;  // pinned (behind h_live)
+    char *h_stage = nullptr;  // pinned, for copies on the stream (stage_get)
+    size_t stage_cap = 0, stage_used = 0;
 
     // work lists
     struct group {
@@ -253,6 +257,7 @@ struct logo2opt_engine {
     bool any_ils = false;
     uint32_t group_grid = 0;  // k_group covers slots [0, group_grid)
     bool dirty = true;
+    std::vector<uint32_t> sig;  // what the lists were made for (rebuild_lists)
     unsigned live_at_build = 0;
 
     // instances that run in k_local, one launch per workgroup size, on a stream
@@ -301,7 +306,7 @@ struct logo2opt_ctx {
     uint32_t n = 0;
     uint32_t metric = LOGO2OPT_METRIC_EUC_2D;
     int prune = LOGO2OPT_PRUNE_OFF;  // applied to ge when it is created
-    std::vector<logo2opt_city_coords> coords;
+    cities ct;
     int32_t slot = -1;
     uint64_t sweeps = 0, moves = 0, evals = 0, fallbacks = 0;
     double wall_ms = 0.0, sweep_ms = 0.0;
@@ -309,9 +314,10 @@ struct logo2opt_ctx {
 
 namespace {
 
-int check_coords(uint32_t n, const logo2opt_city_coords *c, std::vector<int32_t> &xy, float *slack)
+int check_coords(uint32_t n, const logo2opt_city_coords *c, cities &out)
 {
     if (!c) return LOGO2OPT_EINVAL;
+    std::vector<int32_t> &xy = out.xy;
     xy.resize(2 * (size_t)n);
     double mnx = INFINITY, mny = INFINITY, mxx = -INFINITY, mxy = -INFINITY;
     for (uint32_t k = 0; k < n; ++k) {
@@ -338,7 +344,9 @@ int check_coords(uint32_t n, const logo2opt_city_coords *c, std::vector<int32_t>
     // dmax * 2^-23.  Total <= 1 + dmax * 2^-18; 2^-8 margin.
     const double dmax = std::sqrt((mxx - mnx) * (mxx - mnx) + (mxy - mny) * (mxy - mny));
     const double s = 1.0 + dmax * std::ldexp(1.0, -18) + std::ldexp(1.0, -8);
-    *slack = std::nextafter((float)s, INFINITY);
+    out.slack = std::nextafter((float)s, INFINITY);
+    out.span_x = (int32_t)(mxx - mnx);
+    out.span_y = (int32_t)(mxy - mny);
     return LOGO2OPT_OK;
 }
 
@@ -366,9 +374,56 @@ uint64_t bytes_for(uint32_t n, const logo2opt_job *job)
 // log, plus 16 MiB
 uint64_t ctx_budget(uint32_t n, const logo2opt_job &job) { return bytes_for(n, &job) + (1ull << 24); }
 
-// writes the ordered points / tour of `route` into slot buffers and the
-// instance record; the stream must be idle for this slot.
-int upload_instance(logo2opt_engine *e, int32_t id, const uint32_t *route, uint32_t phase)
+// `bytes` of pinned host memory for a copy on the engine's stream: parts of one
+// buffer in turn, which the stream is waited for before they are used again
+int stage_get(logo2opt_engine *e, size_t bytes, char **out)
+{
+    bytes = (bytes + 255) & ~(size_t)255;
+    if (e->stage_used + bytes > e->stage_cap) {
+        L2O_TRY(hipStreamSynchronize(e->stream));
+        e->stage_used = 0;
+        if (bytes > e->stage_cap) {
+            const size_t cap = std::max<size_t>(2 * bytes, 1u << 18);
+            char *h = nullptr;
+            L2O_TRY(hipHostMalloc(&h, cap, hipHostMallocDefault));
+            if (e->h_stage) (void)hipHostFree(e->h_stage);
+            e->h_stage = h;
+            e->stage_cap = cap;
+        }
+    }
+    *out = e->h_stage + e->stage_used;
+    e->stage_used += bytes;
+    return LOGO2OPT_OK;
+}
+
+// an instance's record and result tour (tour_out may be NULL), by way of pinned
+// memory; waits for the stream
+int fetch(logo2opt_engine *e, int32_t id, l2o_inst *in, uint32_t *tour_out)
+{
+    slot_t &s = e->slots[id];
+    const size_t rec = (sizeof(l2o_inst) + 255) & ~(size_t)255, bytes = tour_out ? 4ull * s.n : 0;
+    char *h = nullptr;
+    const int rc = stage_get(e, rec + bytes, &h);
+    if (rc) return rc;
+    L2O_TRY(l2o::launch_fetch(e->d_insts, (uint32_t)id, s.n, (l2o_inst *)h, tour_out ? (uint32_t *)(h + rec) : nullptr,
+                              e->stream));
+    L2O_TRY(hipStreamSynchronize(e->stream));
+    e->stage_used = 0;
+    std::memcpy(in, h, sizeof(*in));
+    if (tour_out) std::memcpy(tour_out, h + rec, bytes);
+    s.sweeps = in->sweeps;
+    s.moves = in->moves;
+    s.fallbacks = in->fallbacks;
+    s.counted = true;
+    return LOGO2OPT_OK;
+}
+
+// admits the instance of a slot on the engine's stream, without waiting for it:
+// its record, cities and start tour go to HBM, k_load makes the ordered points
+// of them.  (Made on the host, with a copy and a wait each for points, tour,
+// record and counter, a single sweep of 200 cities took 153 us and one of 33,810
+// cities 655 us; now 40 and 127 us, and 512 admissions about 35 ms less.)
+int upload_instance(logo2opt_engine *e, int32_t id, const cities &ct, const uint32_t *route, uint32_t phase)
 {
     slot_t &s = e->slots[id];
     const uint32_t n = s.n;
@@ -393,7 +448,7 @@ int upload_instance(logo2opt_engine *e, int32_t id, const uint32_t *route, uint3
     in.pool = e->d_pool + (size_t)4 * L2O_POOL * (s.sweep_only ? e->max_slots : (uint32_t)id);
     in.n = n;
     in.log_cap = s.job.log_cap;
-    in.slack = s.slack;
+    in.slack = ct.slack;
     in.ils_rounds = s.job.ils_rounds;
     in.kick = s.job.kick;
     in.metric = s.job.metric;
@@ -402,14 +457,7 @@ int upload_instance(logo2opt_engine *e, int32_t id, const uint32_t *route, uint3
     in.kick_src = (uint32_t)id;
     in.est_scale = s.job.metric == l2o::L2O_ATT ? (float)(1.0 / std::sqrt(10.0)) : 1.0f;
     in.est_add = s.job.metric == l2o::L2O_EUC_2D ? 0.0f : 0.5f;
-    {
-        int32_t mx = 0, my = 0;
-        for (size_t k = 0; k < s.xy.size(); k += 2) {
-            mx = std::max(mx, s.xy[k]);
-            my = std::max(my, s.xy[k + 1]);
-        }
-        l2o::set_quant(in, mx, my);
-    }
+    l2o::set_quant(in, ct.span_x, ct.span_y);
     in.stop_below = s.job.ils_rounds ? s.job.stop_below : 0;
     in.phase = phase;
     in.cap = -1;
@@ -423,23 +471,14 @@ int upload_instance(logo2opt_engine *e, int32_t id, const uint32_t *route, uint3
         z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
         in.rng[k] = z ^ (z >> 31);
     }
-    std::vector<l2o_pt> pts(n);
-    uint64_t L = 0;
-    const int32_t *xy = s.xy.data();
-    for (uint32_t k = 0; k < n; ++k) {
-        const uint32_t c = route[k], pc = route[k == 0 ? n - 1 : k - 1];
-        const uint32_t d = dist_i(xy, pc, c, s.job.metric);
-        L += d;
-        pts[k].x = xy[2 * c];
-        pts[k].y = xy[2 * c + 1];
-        pts[k].d = (int32_t)d;
-        pts[k].w = l2o::quant_xy(in.qs, in.qox, in.qoy, xy[2 * c], xy[2 * c + 1]);
-    }
-    in.length = L;
-    L2O_TRY(hipMemcpyAsync(in.pts[0], pts.data(), 16ull * n, hipMemcpyHostToDevice, e->stream));
-    L2O_TRY(hipMemcpyAsync(in.tour[0], route, 4ull * n, hipMemcpyHostToDevice, e->stream));
-    L2O_TRY(hipMemcpyAsync(e->d_insts + id, &in, sizeof(in), hipMemcpyHostToDevice, e->stream));
-    L2O_TRY(hipStreamSynchronize(e->stream));
+    const size_t raw = 12ull * n, rec = (sizeof(in) + 255) & ~(size_t)255;
+    char *h = nullptr;
+    const int rc = stage_get(e, rec + raw, &h);
+    if (rc) return rc;
+    std::memcpy(h, &in, sizeof(in));
+    std::memcpy(h + rec, ct.xy.data(), 8ull * n);
+    std::memcpy(h + rec + 8ull * n, route, 4ull * n);
+    L2O_TRY(l2o::launch_load(e->d_insts, (uint32_t)id, n, (const l2o_inst *)h, h + rec, e->d_live, e->stream));
     return LOGO2OPT_OK;
 }
 
@@ -582,6 +621,33 @@ int rebuild_lists(logo2opt_engine *e)
     e->step_pairs = 0;
     for (uint32_t id : order) e->step_pairs += pairs_of(e->slots[id].n) / (prunes(e, e->slots[id].n) ? 4 : 1);
     const int table = order.size() >= L2O_BATCH_MIN && all_pairs >= L2O_BATCH_PAIRS ? 1 : 0;
+    // The lists and the captured steps depend on these alone: a program that
+    // makes call after call on tours of the same size keeps them.
+    std::vector<uint32_t> sig(1, (uint32_t)order.size());  // (never empty)
+    sig.reserve(1 + 4 * order.size());
+    for (uint32_t id : order) {
+        const slot_t &s = e->slots[id];
+        const sweep_cfg c = cfg_for(s.n, table);
+        sig.insert(sig.end(), {id, s.n,
+                               (uint32_t)(table | (prunes(e, s.n) ? 2 : 0) | (s.job.ils_rounds ? 4 : 0) |
+                                          (s.group_lead != L2O_NO_GROUP ? 8 : 0)),
+                               (uint32_t)((c.k << 20) | (c.t << 8) | c.waves)});
+        if (s.job.ils_rounds) {
+            e->any_ils = true;
+            e->ils_grid = std::max(e->ils_grid, id + 1);  // `order` is not by id
+        }
+        if (s.group_lead != L2O_NO_GROUP) e->group_grid = std::max(e->group_grid, id + 1);
+    }
+    if (sig == e->sig) {
+        e->dirty = false;
+        e->live_at_build = e->live_launch;
+        return LOGO2OPT_OK;
+    }
+    e->sig.clear();  // until the lists are in place
+    drop_graph(e);
+    std::vector<l2o_sweep_item> all;
+    std::vector<l2o_apply_item> ai;
+    e->groups.clear();
     for (uint32_t id : order) {
         const slot_t &s = e->slots[id];
         const uint32_t n = s.n;
@@ -595,15 +661,7 @@ int rebuild_lists(logo2opt_engine *e)
             for (uint32_t b0 = a0 + 2; b0 + 2 <= n; b0 += c.cols()) v.push_back({id, a0, b0, (uint32_t)c.t});
         const uint32_t nch = (n + L2O_APPLY_CHUNK - 1) / L2O_APPLY_CHUNK;
         for (uint32_t ch = 0; ch < nch; ++ch) li.apply.push_back({id, ch});
-        if (s.job.ils_rounds) {
-            e->any_ils = true;
-            e->ils_grid = std::max(e->ils_grid, id + 1);  // `order` is not by id
-        }
-        if (s.group_lead != L2O_NO_GROUP) e->group_grid = std::max(e->group_grid, id + 1);
     }
-    std::vector<l2o_sweep_item> all;
-    std::vector<l2o_apply_item> ai;
-    e->groups.clear();
     for (auto &kv : by_cfg) {
         const sweep_cfg c{std::get<0>(kv.first), std::get<1>(kv.first), std::get<2>(kv.first)};
         const int mode = std::get<3>(kv.first);
@@ -679,9 +737,9 @@ int rebuild_lists(logo2opt_engine *e)
                                e->stream));
     L2O_TRY(hipStreamSynchronize(e->stream));
     e->n_aitems = (uint32_t)ai.size();
+    e->sig.swap(sig);
     e->dirty = false;
     e->live_at_build = e->live_launch;
-    drop_graph(e);
     return LOGO2OPT_OK;
 }
 
@@ -825,6 +883,7 @@ int engine_run(logo2opt_engine *e, uint32_t max_steps, uint32_t sync_every, uint
 {
     if (sync_every == 0) sync_every = 1;
     const double t0 = now_ms();
+    for (slot_t &s : e->slots) s.counted = false;
     // one host check per step (sync_every = 1) and the timed sweeps keep every
     // instance in steps
     const bool use_local = sync_every > 1 && !e->timing;
@@ -842,6 +901,7 @@ int engine_run(logo2opt_engine *e, uint32_t max_steps, uint32_t sync_every, uint
     hipStream_t st = e->stream;
     if (!e->locals.empty() && e->live_launch > 0) {
         if (!e->lstream) L2O_TRY(hipStreamCreateWithFlags(&e->lstream, hipStreamNonBlocking));
+        L2O_TRY(hipStreamSynchronize(e->stream));  // admissions
         st = e->lstream;
     }
     auto next_local = [&]() {
@@ -885,19 +945,11 @@ int engine_run(logo2opt_engine *e, uint32_t max_steps, uint32_t sync_every, uint
 }
 
 // admits an instance into slot `id` (free); group_lead / group_size as in l2o_inst
-int engine_add_at(logo2opt_engine *e, int32_t id, uint32_t n, const logo2opt_city_coords *coords,
-                  const uint32_t *route, const logo2opt_job *job, uint32_t group_lead, uint32_t group_size,
-                  bool sweep_only = false)
+int engine_add_at(logo2opt_engine *e, int32_t id, uint32_t n, const cities &ct, const uint32_t *route,
+                  const logo2opt_job *job, uint32_t group_lead, uint32_t group_size, bool sweep_only = false)
 {
-    if (n < 3 || n > LOGO2OPT_MAX_N) return LOGO2OPT_EINVAL;
-    slot_t tmp;
-    int rc = check_coords(n, coords, tmp.xy, &tmp.slack);
+    int rc = check_tour(n, route);
     if (rc) return rc;
-    rc = check_tour(n, route);
-    if (rc) return rc;
-    tmp.group_lead = group_lead;
-    tmp.group_size = group_size;
-    tmp.sweep_only = sweep_only;
     logo2opt_job j{};
     if (job) j = *job;
     if (j.kick > 1 || j.metric > LOGO2OPT_METRIC_ATT) return LOGO2OPT_EINVAL;
@@ -908,30 +960,35 @@ int engine_add_at(logo2opt_engine *e, int32_t id, uint32_t n, const logo2opt_cit
     uint64_t off;
     if (!e->ar.alloc(bytes, &off)) return LOGO2OPT_EAGAIN;
     slot_t &s = e->slots[id];
-    s = std::move(tmp);
+    s = slot_t();
     s.used = true;
     s.n = n;
     s.off = off;
     s.bytes = bytes;
     s.job = j;
-    s.done = false;
-    s.done_reported = false;
-    rc = upload_instance(e, id, route, L2O_LO);
+    s.group_lead = group_lead;
+    s.group_size = group_size;
+    s.sweep_only = sweep_only;
+    rc = upload_instance(e, id, ct, route, L2O_LO);
     if (rc) {
         e->ar.release(off, bytes);
         s = slot_t();
         return rc;
     }
     e->live += 1;
-    *e->h_live = e->live;
-    L2O_TRY(hipMemcpyAsync(e->d_live, e->h_live, sizeof(unsigned), hipMemcpyHostToDevice, e->stream));
-    L2O_TRY(hipStreamSynchronize(e->stream));
     e->dirty = true;
     return LOGO2OPT_OK;
 }
 
-int engine_add(logo2opt_engine *e, uint32_t n, const logo2opt_city_coords *coords, const uint32_t *route,
-               const logo2opt_job *job, int32_t *slot_out, bool sweep_only = false)
+// checks an instance's cities as engine_add does
+int cities_of(uint32_t n, const logo2opt_city_coords *coords, cities &ct)
+{
+    if (n < 3 || n > LOGO2OPT_MAX_N) return LOGO2OPT_EINVAL;
+    return check_coords(n, coords, ct);
+}
+
+int engine_add(logo2opt_engine *e, uint32_t n, const cities &ct, const uint32_t *route, const logo2opt_job *job,
+               int32_t *slot_out, bool sweep_only = false)
 {
     int32_t id = -1;
     for (uint32_t k = 0; k < e->max_slots; ++k)
@@ -940,7 +997,7 @@ int engine_add(logo2opt_engine *e, uint32_t n, const logo2opt_city_coords *coord
             break;
         }
     if (id < 0) return LOGO2OPT_EAGAIN;
-    const int rc = engine_add_at(e, id, n, coords, route, job, L2O_NO_GROUP, 0, sweep_only);
+    const int rc = engine_add_at(e, id, n, ct, route, job, L2O_NO_GROUP, 0, sweep_only);
     if (rc == LOGO2OPT_OK) *slot_out = id;
     return rc;
 }
@@ -949,8 +1006,8 @@ int engine_remove(logo2opt_engine *e, int32_t id);
 
 // `chains` ILS chains of one instance in consecutive slots; chain c uses the
 // seed job->seed + c
-int engine_add_group(logo2opt_engine *e, uint32_t n, const logo2opt_city_coords *coords, const uint32_t *route,
-                     const logo2opt_job *job, uint32_t chains, int32_t *first_out)
+int engine_add_group(logo2opt_engine *e, uint32_t n, const cities &ct, const uint32_t *route, const logo2opt_job *job,
+                     uint32_t chains, int32_t *first_out)
 {
     if (!job || job->ils_rounds == 0 || chains == 0 || chains > e->max_slots) return LOGO2OPT_EINVAL;
     int32_t first = -1;
@@ -964,7 +1021,7 @@ int engine_add_group(logo2opt_engine *e, uint32_t n, const logo2opt_city_coords 
     for (uint32_t c = 0; c < chains; ++c) {
         logo2opt_job j = *job;
         j.seed = job->seed + c;
-        const int rc = engine_add_at(e, first + (int32_t)c, n, coords, route, &j, (uint32_t)first, chains);
+        const int rc = engine_add_at(e, first + (int32_t)c, n, ct, route, &j, (uint32_t)first, chains);
         if (rc) {
             for (uint32_t q = 0; q < c; ++q) e->slots[first + q].group_lead = L2O_NO_GROUP;
             for (uint32_t q = 0; q < c; ++q) (void)engine_remove(e, first + (int32_t)q);
@@ -979,8 +1036,8 @@ int engine_result(logo2opt_engine *e, int32_t id, uint32_t *route_out, logo2opt_
 {
     if (id < 0 || (uint32_t)id >= e->max_slots || !e->slots[id].used) return LOGO2OPT_ENOTFOUND;
     l2o_inst in;
-    L2O_TRY(hipMemcpyAsync(&in, e->d_insts + id, sizeof(in), hipMemcpyDeviceToHost, e->stream));
-    L2O_TRY(hipStreamSynchronize(e->stream));
+    const int rc = fetch(e, id, &in, route_out);
+    if (rc) return rc;
     const bool ils = in.ils_rounds > 0;
     if (res) {
         res->length = ils && in.have_best ? in.best_length : in.length;
@@ -990,15 +1047,13 @@ int engine_result(logo2opt_engine *e, int32_t id, uint32_t *route_out, logo2opt_
         res->rounds_done = in.rounds_done;
         res->done = in.phase == L2O_DONE;
     }
-    if (route_out) {
-        const uint32_t *src = ils && in.have_best ? in.btour : in.tour[in.parity];
-        L2O_TRY(hipMemcpyAsync(route_out, src, 4ull * in.n, hipMemcpyDeviceToHost, e->stream));
-    }
     if (log && in.log_cap) {
         const uint64_t m = std::min<uint64_t>(in.moves, in.log_cap);
-        if (m) L2O_TRY(hipMemcpyAsync(log, in.log, 12ull * m, hipMemcpyDeviceToHost, e->stream));
+        if (m) {
+            L2O_TRY(hipMemcpyAsync(log, in.log, 12ull * m, hipMemcpyDeviceToHost, e->stream));
+            L2O_TRY(hipStreamSynchronize(e->stream));
+        }
     }
-    L2O_TRY(hipStreamSynchronize(e->stream));
     return LOGO2OPT_OK;
 }
 
@@ -1019,26 +1074,9 @@ int engine_remove(logo2opt_engine *e, int32_t id)
         }
     }
     slot_t &s = e->slots[id];
-    if (!s.done) {
-        // retire a running instance: mark it done on the device first
-        l2o_inst in;
-        L2O_TRY(hipMemcpyAsync(&in, e->d_insts + id, sizeof(in), hipMemcpyDeviceToHost, e->stream));
-        L2O_TRY(hipStreamSynchronize(e->stream));
-        if (in.phase != L2O_DONE) {
-            // (a finished instance has left its pool empty)
-            if (!s.sweep_only)
-                L2O_TRY(hipMemsetAsync(e->d_pool + (size_t)4 * L2O_POOL * id, 0xFF,
-                                       sizeof(unsigned long long) * 4 * L2O_POOL, e->stream));
-            e->live -= 1;
-            *e->h_live = e->live;
-            L2O_TRY(hipMemcpyAsync(e->d_live, e->h_live, sizeof(unsigned), hipMemcpyHostToDevice, e->stream));
-        }
-    }
-    l2o_inst blank;
-    std::memset(&blank, 0, sizeof(blank));
-    blank.phase = L2O_FREE;
-    L2O_TRY(hipMemcpyAsync(e->d_insts + id, &blank, sizeof(blank), hipMemcpyHostToDevice, e->stream));
-    L2O_TRY(hipStreamSynchronize(e->stream));
+    // (the host knows: a run ends with the state of its finished instances read)
+    if (!s.done) e->live -= 1;
+    L2O_TRY(l2o::launch_free(e->d_insts, (uint32_t)id, e->d_live, !s.done, !s.done && !s.sweep_only, e->stream));
     e->ar.release(s.off, s.bytes);
     s = slot_t();
     e->dirty = true;
@@ -1066,10 +1104,10 @@ int engine_create(int device, uint64_t budget, uint32_t max_slots, logo2opt_engi
               hipMalloc(&e->d_insts, pool_off + pool_bytes) == hipSuccess &&
               hipMalloc(&e->d_live, sizeof(unsigned)) == hipSuccess &&
               hipMalloc(&e->d_scratch, sizeof(unsigned long long) * 4) == hipSuccess &&
-              hipHostMalloc(&e->h_live, sizeof(unsigned), hipHostMallocDefault) == hipSuccess &&
-              hipHostMalloc(&e->h_scratch, sizeof(unsigned long long) * 4, hipHostMallocDefault) == hipSuccess &&
+              hipHostMalloc(&e->h_live, 64, hipHostMallocDefault) == hipSuccess &&
               hipEventCreate(&e->ev0) == hipSuccess && hipEventCreate(&e->ev1) == hipSuccess;
     if (ok) {
+        e->h_scratch = (unsigned long long *)((char *)e->h_live + 32);
         e->ar.init(e->d_arena, budget);
         e->d_pool = (unsigned long long *)((char *)e->d_insts + pool_off);
         // all ones: pools empty (L2O_SENTINEL), records in no phase and no group
@@ -1186,7 +1224,7 @@ int logo2opt_engine_destroy(logo2opt_engine *e)
     if (e->d_live) (void)hipFree(e->d_live);
     if (e->d_scratch) (void)hipFree(e->d_scratch);
     if (e->h_live) (void)hipHostFree(e->h_live);
-    if (e->h_scratch) (void)hipHostFree(e->h_scratch);
+    if (e->h_stage) (void)hipHostFree(e->h_stage);
     if (e->ev0) (void)hipEventDestroy(e->ev0);
     if (e->ev1) (void)hipEventDestroy(e->ev1);
     for (hipEvent_t ev : e->tev) (void)hipEventDestroy(ev);
@@ -1203,7 +1241,14 @@ int logo2opt_engine_add(logo2opt_engine *e, uint32_t n, const logo2opt_city_coor
 {
     if (!e || !slot) return LOGO2OPT_EINVAL;
     if (hipSetDevice(e->device) != hipSuccess) return LOGO2OPT_EDEVICE;
-    return engine_add(e, n, coords, route, job, slot);
+    // (a full engine first, as the cheaper answer)
+    bool room = false;
+    for (const slot_t &s : e->slots) room = room || !s.used;
+    if (!room) return LOGO2OPT_EAGAIN;
+    cities ct;
+    const int rc = cities_of(n, coords, ct);
+    if (rc) return rc;
+    return engine_add(e, n, ct, route, job, slot);
 }
 
 int logo2opt_engine_add_group(logo2opt_engine *e, uint32_t n, const logo2opt_city_coords *coords,
@@ -1211,7 +1256,11 @@ int logo2opt_engine_add_group(logo2opt_engine *e, uint32_t n, const logo2opt_cit
 {
     if (!e || !first_slot) return LOGO2OPT_EINVAL;
     if (hipSetDevice(e->device) != hipSuccess) return LOGO2OPT_EDEVICE;
-    return engine_add_group(e, n, coords, route, job, chains, first_slot);
+    if (!job || job->ils_rounds == 0 || chains == 0 || chains > e->max_slots) return LOGO2OPT_EINVAL;
+    cities ct;
+    const int rc = cities_of(n, coords, ct);
+    if (rc) return rc;
+    return engine_add_group(e, n, ct, route, job, chains, first_slot);
 }
 
 int logo2opt_engine_group_result(logo2opt_engine *e, int32_t first_slot, uint32_t *route_out, logo2opt_result *res,
@@ -1288,16 +1337,27 @@ int logo2opt_engine_stats(logo2opt_engine *e, logo2opt_stats *st)
 {
     if (!e || !st) return LOGO2OPT_EINVAL;
     if (hipSetDevice(e->device) != hipSuccess) return LOGO2OPT_EDEVICE;
-    std::vector<l2o_inst> h(e->max_slots);
-    L2O_TRY(hipMemcpyAsync(h.data(), e->d_insts, sizeof(l2o_inst) * e->max_slots, hipMemcpyDeviceToHost, e->stream));
-    L2O_TRY(hipStreamSynchronize(e->stream));
+    bool counted = true;
+    for (const slot_t &s : e->slots) counted = counted && (!s.used || s.counted);
+    if (!counted) {
+        std::vector<l2o_inst> h(e->max_slots);
+        L2O_TRY(hipMemcpyAsync(h.data(), e->d_insts, sizeof(l2o_inst) * e->max_slots, hipMemcpyDeviceToHost, e->stream));
+        L2O_TRY(hipStreamSynchronize(e->stream));
+        for (uint32_t id = 0; id < e->max_slots; ++id) {
+            slot_t &s = e->slots[id];
+            s.sweeps = h[id].sweeps;
+            s.moves = h[id].moves;
+            s.fallbacks = h[id].fallbacks;
+            s.counted = s.used;
+        }
+    }
     std::memset(st, 0, sizeof(*st));
-    for (uint32_t id = 0; id < e->max_slots; ++id) {
-        if (!e->slots[id].used) continue;
-        st->sweeps += h[id].sweeps;
-        st->moves += h[id].moves;
-        st->evals += h[id].sweeps * pairs_of(h[id].n);
-        st->fallbacks += h[id].fallbacks;
+    for (const slot_t &s : e->slots) {
+        if (!s.used) continue;
+        st->sweeps += s.sweeps;
+        st->moves += s.moves;
+        st->evals += s.sweeps * pairs_of(s.n);
+        st->fallbacks += s.fallbacks;
     }
     st->wall_ms = e->wall_ms;
     st->sweep_ms = e->sweep_ms;
@@ -1358,15 +1418,15 @@ int logo2opt_create_metric(int device, uint32_t n, const logo2opt_city_coords *c
 {
     if (!out || !coords || n < 3 || n > LOGO2OPT_MAX_N) return LOGO2OPT_EINVAL;
     if (metric < LOGO2OPT_METRIC_EUC_2D || metric > LOGO2OPT_METRIC_ATT) return LOGO2OPT_EINVAL;
-    std::vector<int32_t> xy;
-    float slack;
-    int rc = check_coords(n, coords, xy, &slack);
-    if (rc) return rc;
     logo2opt_ctx *c = new (std::nothrow) logo2opt_ctx();
     if (!c) return LOGO2OPT_ENOMEM;
+    int rc = check_coords(n, coords, c->ct);
+    if (rc) {
+        delete c;
+        return rc;
+    }
     c->n = n;
     c->metric = (uint32_t)metric;
-    c->coords.assign(coords, coords + n);
     // room for one ILS instance with a modest move log; ctx_load replaces the
     // engine by a larger one when a call needs more
     logo2opt_job j{};
@@ -1425,7 +1485,7 @@ int ctx_load(logo2opt_ctx *c, const uint32_t *route, logo2opt_job job, bool swee
         logo2opt_engine_destroy(old);
         c->e = e;
     }
-    return engine_add(c->e, c->n, c->coords.data(), route, &job, &c->slot, sweep_only);
+    return engine_add(c->e, c->n, c->ct, route, &job, &c->slot, sweep_only);
 }
 
 }  // namespace
@@ -1448,14 +1508,14 @@ int logo2opt_step(logo2opt_ctx *ctx, const uint32_t *route, logo2opt_best2_out *
     for (const auto &g : e->groups)
         L2O_TRY(launch_group_sweep(e, g));
     L2O_TRY(hipEventRecord(e->ev1, e->stream));
-    L2O_TRY(hipEventSynchronize(e->ev1));
-    float ms = 0.0f;
-    L2O_TRY(hipEventElapsedTime(&ms, e->ev0, e->ev1));
+    if (t) L2O_TRY(hipEventSynchronize(e->ev1));  // the caller's times by part
     const double d0 = now_ms();
     l2o_inst in;
-    L2O_TRY(hipMemcpyAsync(&in, e->d_insts + ctx->slot, sizeof(in), hipMemcpyDeviceToHost, e->stream));
-    L2O_TRY(hipStreamSynchronize(e->stream));
+    rc = fetch(e, ctx->slot, &in, nullptr);
+    if (rc) return rc;
     const double d1 = now_ms();
+    float ms = 0.0f;
+    L2O_TRY(hipEventElapsedTime(&ms, e->ev0, e->ev1));
     if (in.key[0] == L2O_SENTINEL) {
         out->i = out->j = 0;
         out->minchange = 0;
@@ -1631,7 +1691,7 @@ int logo2opt_ils_multistart(logo2opt_ctx *ctx, uint32_t *route_inout, uint64_t s
             if (rc) return rc;
         }
     int32_t first = -1;
-    rc = engine_add_group(e, ctx->n, ctx->coords.data(), route_inout, &job, chains, &first);
+    rc = engine_add_group(e, ctx->n, ctx->ct, route_inout, &job, chains, &first);
     if (rc) return rc;
     const double t0 = now_ms();
     uint32_t live = 1;
@@ -1706,6 +1766,7 @@ int logo2opt_engine_time_sweep(logo2opt_engine *e, uint32_t sweeps, double *avg_
 {
     if (!e || !avg_ms || sweeps == 0) return LOGO2OPT_EINVAL;
     if (hipSetDevice(e->device) != hipSuccess) return LOGO2OPT_EDEVICE;
+    for (slot_t &s : e->slots) s.counted = false;
     int rc = assign_local(e, false, false);
     if (!rc) rc = rebuild_lists(e);
     if (rc) return rc;

@@ -227,6 +227,74 @@ __global__ __launch_bounds__(64) void k_group(l2o_inst *__restrict__ insts, uint
 }
 
 // ---------------------------------------------------------------------------
+// admission and release of a slot.  Kernels that read and write pinned host
+// memory, in place of copies: a copy of a few hundred bytes between launches
+// takes longer than a launch does.
+// ---------------------------------------------------------------------------
+// host memory to HBM: an instance's record, and its coordinates by city (int32
+// x, y) and start tour (n times 12 bytes) into its other point buffer
+__global__ __launch_bounds__(256) void k_stage(l2o_inst *__restrict__ in, const l2o_inst *__restrict__ rec,
+                                               uint4 *__restrict__ raw, const uint4 *__restrict__ host, uint32_t words)
+{
+    if (blockIdx.x == 0)
+        for (uint32_t k = threadIdx.x; k < sizeof(l2o_inst) / 4; k += 256) ((uint32_t *)in)[k] = ((const uint32_t *)rec)[k];
+    for (uint32_t k = blockIdx.x * 256 + threadIdx.x; k < words; k += gridDim.x * 256) raw[k] = host[k];
+}
+
+// the tour-ordered points of an admitted instance: coordinates, exact edge
+// lengths, quantised coordinates; city ids and the tour's length
+__global__ __launch_bounds__(256) void k_load(l2o_inst *__restrict__ insts, uint32_t slot, unsigned *__restrict__ live)
+{
+    l2o_inst *in = insts + slot;
+    const int n = (int)in->n;
+    const uint32_t metric = in->metric;
+    const int2 *__restrict__ xy = (const int2 *)in->pts[1];
+    const uint32_t *__restrict__ route = (const uint32_t *)(xy + n);
+    l2o_pt *__restrict__ P = in->pts[0];
+    uint32_t *__restrict__ R = in->tour[0];
+    unsigned long long sum = 0;
+    for (int k = (int)(blockIdx.x * 256 + threadIdx.x); k < n; k += (int)gridDim.x * 256) {
+        const uint32_t c = route[k], pc = route[k ? k - 1 : n - 1];
+        const int2 a = xy[c], b = xy[pc];
+        l2o_pt r;
+        r.x = a.x;
+        r.y = a.y;
+        r.d = exact_dist(b.x, b.y, a.x, a.y, metric);
+        r.w = quant_xy(in->qs, in->qox, in->qoy, a.x, a.y);
+        sum += (unsigned long long)r.d;
+        P[k] = r;
+        R[k] = c;
+    }
+    sum = wave_sum_u64(sum);
+    if ((threadIdx.x & 63) == 0 && sum) atomicAdd(&in->length, sum);
+    if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(live, 1u);
+}
+
+// release of a slot: its record blank, its pool empty (`running`: it was live)
+__global__ __launch_bounds__(256) void k_free(l2o_inst *__restrict__ insts, uint32_t slot, unsigned *__restrict__ live,
+                                              int running, int clear_pool)
+{
+    l2o_inst *in = insts + slot;
+    unsigned long long *const pool = in->pool;
+    if (clear_pool) pool[threadIdx.x] = L2O_SENTINEL;  // 4 L2O_POOL entries
+    __syncthreads();
+    for (uint32_t k = threadIdx.x; k < sizeof(l2o_inst) / 4; k += 256) ((uint32_t *)in)[k] = 0;  // L2O_FREE
+    if (running && threadIdx.x == 0) atomicSub(live, 1u);
+}
+
+// an instance's record and result tour into host memory
+__global__ __launch_bounds__(256) void k_fetch(const l2o_inst *__restrict__ insts, uint32_t slot,
+                                               l2o_inst *__restrict__ rec, uint32_t *__restrict__ tour)
+{
+    const l2o_inst *in = insts + slot;
+    if (blockIdx.x == 0)
+        for (uint32_t k = threadIdx.x; k < sizeof(l2o_inst) / 4; k += 256) ((uint32_t *)rec)[k] = ((const uint32_t *)in)[k];
+    if (!tour) return;
+    const uint32_t *src = in->ils_rounds && in->have_best ? in->btour : in->tour[in->parity];
+    for (uint32_t k = blockIdx.x * 256 + threadIdx.x; k < in->n; k += gridDim.x * 256) tour[k] = src[k];
+}
+
+// ---------------------------------------------------------------------------
 // exact tour length of the current buffer: sum of D (headers.h:170-189)
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_length(const l2o_inst *__restrict__ insts, uint32_t slot,
@@ -296,6 +364,33 @@ hipError_t launch_group(l2o_inst *insts, uint32_t nslots, unsigned *live, hipStr
 {
     if (nslots == 0) return hipSuccess;
     hipLaunchKernelGGL(k_group, dim3((nslots + 63) / 64), dim3(64), 0, stream, insts, nslots, live);
+    return hipGetLastError();
+}
+
+static uint32_t blocks_for(uint32_t n) { return n < 256 * 256 ? (n + 255) / 256 : 256; }
+
+hipError_t launch_load(l2o_inst *insts, uint32_t slot, uint32_t n, const l2o_inst *rec, const void *raw, unsigned *live,
+                       hipStream_t stream)
+{
+    const uint32_t words = (12 * n + 15) / 16;  // (the point buffer holds 16 n bytes)
+    hipLaunchKernelGGL(k_stage, dim3(blocks_for(words)), dim3(256), 0, stream, insts + slot, rec, (uint4 *)rec->pts[1],
+                       (const uint4 *)raw, words);
+    const hipError_t err = hipGetLastError();
+    if (err != hipSuccess) return err;
+    hipLaunchKernelGGL(k_load, dim3(blocks_for(n)), dim3(256), 0, stream, insts, slot, live);
+    return hipGetLastError();
+}
+
+hipError_t launch_free(l2o_inst *insts, uint32_t slot, unsigned *live, bool running, bool clear_pool, hipStream_t stream)
+{
+    hipLaunchKernelGGL(k_free, dim3(1), dim3(256), 0, stream, insts, slot, live, running ? 1 : 0, clear_pool ? 1 : 0);
+    return hipGetLastError();
+}
+
+hipError_t launch_fetch(const l2o_inst *insts, uint32_t slot, uint32_t n, l2o_inst *rec, uint32_t *tour,
+                        hipStream_t stream)
+{
+    hipLaunchKernelGGL(k_fetch, dim3(tour ? blocks_for(n) : 1), dim3(256), 0, stream, insts, slot, rec, tour);
     return hipGetLastError();
 }
 

@@ -106,6 +106,13 @@ hipError_t launch_local(int waves, const uint32_t *ids, uint32_t count, uint32_t
                         uint32_t steps, hipStream_t stream);
 uint32_t local_lds_bytes(uint32_t n, int waves);
 hipError_t launch_group(l2o_inst *insts, uint32_t nslots, unsigned *live, hipStream_t stream);
+// admission, release and result of a slot (l2o_kernels.hip)
+// (`rec` and `raw`: pinned host memory, 16-byte aligned, a multiple of 16 bytes)
+hipError_t launch_load(l2o_inst *insts, uint32_t slot, uint32_t n, const l2o_inst *rec, const void *raw, unsigned *live,
+                       hipStream_t stream);
+hipError_t launch_free(l2o_inst *insts, uint32_t slot, unsigned *live, bool running, bool clear_pool, hipStream_t stream);
+hipError_t launch_fetch(const l2o_inst *insts, uint32_t slot, uint32_t n, l2o_inst *rec, uint32_t *tour,
+                        hipStream_t stream);
 hipError_t launch_length(const l2o_inst *insts, uint32_t slot, uint32_t n, unsigned long long *out,
                          hipStream_t stream);
 hipError_t launch_sqrt_ulp(uint32_t lo, uint32_t hi, unsigned *max_ulp, hipStream_t stream);
