@@ -8,14 +8,19 @@ improvement local search on the GPU, on the 33,810-city clustered instance
 One "step" is one full local search from the same start tour.  The
 coordinates are copied to the device once, before the timed region; each
 step hands the library the 135 KB start tour, as TwoOptLocalSolver::optimize's
-caller does, and the library rebuilds and uploads the tour-ordered point
-array with its exact edge lengths (541 KB) before the first sweep -- this is
-inside the timed region (about 1 ms of the ~0.3 s step).
+caller does, and the library uploads it with the cities and makes the
+tour-ordered point array with its exact edge lengths (541 KB) before the first
+sweep -- this is
+inside the timed region (about 0.1 ms of the ~0.14 s step).
 
 Also reported on the same line:
-  roofline      sweep kernel, 14 algorithmic FP32 FLOP per evaluated move,
-                average kernel duration from HIP events on the engine stream
-                over one timed local search (same trajectory as the steps)
+  roofline      sweep kernel, 32 matrix FLOP per evaluated move (its test is
+                one output of a 16-term FP16 product), average kernel duration
+                from HIP events on the engine stream over one timed local
+                search (same trajectory as the steps; the timed steps fuse the
+                apply into the sweep, which is slower per launch); contract:
+                the same in 14 algorithmic FP32 FLOP per move, which the
+                kernel does not execute
   cpu_baseline  the reference's own CPU sweep (CPUSolver::optimizeStep built
                 from its sources, oracle/_ref) timed on this host on a bounded
                 sample of sweeps of the same instance and start tour
@@ -50,22 +55,25 @@ import logo2opt as L  # noqa: E402
 
 METRIC = "2-opt move evals/sec + instances/sec batched vs plain, bit-exact tour length"
 # algorithmic work of one move evaluation, the unit the roofline is priced in:
-# 2 new edges x (2 sub + mul + fma(2) + sqrt + add); the kernel's own filter
-# does less (integer L1 bounds, see l2o_kernels.hip) and is priced the same
+# 2 new edges x (2 sub + mul + fma(2) + sqrt + add); the kernel's own test is
+# a matrix product (below) and is priced the same in `contract`
 FLOP_PER_EVAL = 14
 # HBM bytes per sweep launch of the 33,810-city search, from two rocprofv3 --pmc runs of this
-# benchmark (FETCH_SIZE 2,680.2 KiB x 2.0 + WRITE_SIZE 4.42 KiB x 1.0, factors from a 256 MiB copy;
+# benchmark (FETCH_SIZE 2,399.66 KiB x 2.0 + WRITE_SIZE 1.05 KiB x 1.0, factors from a 256 MiB copy;
 # profiles/k_sweep_config2_counters.md).  Reported only for the kernel that was profiled.
-PROFILED_TRAFFIC = {"l2o::k_sweep<4,256,2,0>": 2680.17 * 1024 * 2.0 + 4.41877 * 1024 * 1.0}
+PROFILED_TRAFFIC = {"l2o::k_sweep<4, 4, 0, false>": 2399.66 * 1024 * 2.0 + 1.04508 * 1024 * 1.0}
 REF_FLOP_PER_EVAL = 36    # the reference's GPU GFLOPS convention (solver.c:305-306)
 PEAK_FP32_TFLOPS = 157.3  # MI355X published FP32 vector peak
-# The sweep's own bound: VALU instruction issue.  Each of the 1,024 SIMDs
-# (256 CUs x 4) issues one wave64 VALU instruction per 4 cycles at 2.4 GHz
-# (the FP32 peak above is this rate x 64 lanes x 2 for FMA x 2 for packed
-# FP32).  VALU instructions per candidate come from SQ_INSTS_VALU of the
-# profiled kernel (per dispatch / candidates per dispatch, wave instructions).
+# The sweep's own bounds: its test is one matrix output per candidate
+# (v_mfma_f32_32x32x16_f16: 32 FLOP each on the matrix units' dense 2.5
+# PFLOP/s), and the outputs' signs are combined on the VALU.  Each of the 1,024
+# SIMDs (256 CUs x 4) issues one wave64 VALU instruction per 4 cycles at 2.4
+# GHz.  VALU instructions per candidate come from SQ_INSTS_VALU of the profiled
+# kernel (per dispatch / candidates per dispatch, wave instructions).
+MFMA_FLOP_PER_EVAL = 32
+PEAK_MFMA_F16_TFLOPS = 2500.0
 VALU_ISSUE_PEAK = 1024 * 2.4e9 / 4
-PROFILED_VALU_PER_EVAL = {"l2o::k_sweep<4,256,2,0>": 1.96806e7 / 571473528}
+PROFILED_VALU_PER_EVAL = {"l2o::k_sweep<4, 4, 0, false>": 8.92234e6 / (571473528 * 4847 / 4864)}
 
 
 def log(*a):
@@ -80,7 +88,7 @@ def sweep_kernel_name(n, table=None):
     """Name of the sweep kernel instance the library launches for size n."""
     rows = L.tuning_get(L.TABLE_SINGLE if table is None else table)
     k, t, w = next((sh for mx, sh in rows if n <= mx), rows[-1][1])
-    return f"l2o::k_sweep<{k},{t},{w},0>"  # mode 0: the full sweep
+    return f"l2o::k_sweep<{k}, {w}, 0, false>"  # mode 0: the full sweep; false: a step by itself
 
 
 def config2(seed=2):
@@ -467,8 +475,11 @@ def main():
     flop_per_launch = FLOP_PER_EVAL * pairs(n) * work_sweeps / launches
     achieved = flop_per_launch / (avg_ms * 1e-3) / 1e12
     kname = sweep_kernel_name(n)
-    roofline = {"bound": "valu", "achieved": achieved, "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
-                "frac": achieved / PEAK_FP32_TFLOPS, "traffic": PROFILED_TRAFFIC.get(kname),
+    matrix = achieved * MFMA_FLOP_PER_EVAL / FLOP_PER_EVAL
+    roofline = {"bound": "mfma", "achieved": matrix, "peak": PEAK_MFMA_F16_TFLOPS, "unit": "TFLOP/s",
+                "frac": matrix / PEAK_MFMA_F16_TFLOPS, "traffic": PROFILED_TRAFFIC.get(kname),
+                "contract": {"flop_per_eval": FLOP_PER_EVAL, "tflops": achieved,
+                             "of_fp32_vector_peak": achieved / PEAK_FP32_TFLOPS},
                 "kernel": kname, "avg_kernel_ms": avg_ms, "launches": launches,
                 "evals_per_s_kernel": pairs(n) * work_sweeps / launches / (avg_ms * 1e-3),
                 "ref_convention_tflops": achieved * REF_FLOP_PER_EVAL / FLOP_PER_EVAL}
@@ -478,9 +489,8 @@ def main():
         roofline["valu_issue"] = {
             "achieved": rate, "peak": VALU_ISSUE_PEAK, "unit": "wave64 VALU instructions/s",
             "frac": rate / VALU_ISSUE_PEAK, "valu_per_eval_x64": vpe * 64,
-            "note": "the kernel's integer VALU issue rate (SQ_INSTS_VALU per candidate from the profiled "
-                    "counters x candidates/s in the kernel) against the issue peak; frac above is the 14-FLOP "
-                    "contract figure"}
+            "note": "the kernel's VALU issue rate (SQ_INSTS_VALU per candidate from the profiled counters x "
+                    "candidates/s in the kernel) against the issue peak"}
     ctx.close()
 
     pruned = None
@@ -507,9 +517,10 @@ def main():
         "metric": METRIC, "value": evals / dt, "unit": "evals/s", "n_gpus": 1, "steps": args.steps,
         "warmup": args.warmup, "ms_per_step": dt / args.steps * 1e3, "higher_is_better": True,
         "scaling": "weak", "vs_baseline": None, "dtype": "i32", "data": "synthetic",
-        "dtype_note": "the sweep's hot loop is integer VALU (v_sad_u8 on 8-bit coordinates for every candidate, "
-                      "v_sad_u32 L1 bounds for the blocks that pass); FP32 sqrt re-checks the rare survivors and "
-                      "FP64 + integer fix-up gives their exact lengths; lengths are exact integers",
+        "dtype_note": "gains and lengths are exact 32/64-bit integers; every candidate passes a bound on the matrix "
+                      "cores whose operands and sums are whole numbers held exactly (FP16 x FP16 into FP32), which "
+                      "drops only candidates that cannot win; FP32 sqrt re-checks the survivors and integer "
+                      "arithmetic gives their exact lengths",
         "config": {"workload": "33,810 clustered cities (60 Gaussian clusters, sigma 2% of side, + 10% uniform "
                                "noise) in [0,1e6)^2, greedy NN start, best-improvement 2-opt to a local optimum",
                    "n": n, "seed": 2, "moves": out["moves"], "sweeps": sweeps_per, "length": out["length"],

@@ -184,7 +184,7 @@ typedef struct {
     uint64_t sweeps;        /* sweeps since create (moves + 1 per local search)  */
     uint64_t moves;         /* applied 2-opt moves                                */
     uint64_t evals;         /* candidate moves evaluated, (n-2)(n-3)/2 per sweep  */
-    uint64_t fallbacks;     /* candidates re-evaluated on the exact FP64 path     */
+    uint64_t fallbacks;     /* candidates whose exact gain was computed           */
     double   sweep_ms;      /* device time of timed sweep kernels (HIP events)    */
     double   wall_ms;       /* host wall time inside optimize/ils/run             */
     uint64_t sweep_launches;/* sweep kernel launches (timed mode: all are timed)  */
@@ -285,16 +285,16 @@ int logo2opt_engine_set_timing(logo2opt_engine *e, int on);
 /* on = 0: issue every step as direct launches instead of replaying captured
  * HIP graphs (also LOGO2OPT_GRAPHS=0 in the environment at engine creation). */
 int logo2opt_engine_set_graphs(logo2opt_engine *e, int on);
-/* Row pruning: sweeps skip the blocks of 4 rows in which no candidate can
- * pass the integer bound (a row's L1 distance to the bounding box of a wave's
- * columns already exceeds it).  The selected moves, tours and lengths are
- * identical; fewer candidates are evaluated, so the sweep's evals/s figure
+/* Row pruning: sweeps skip the blocks of 32 rows by 32 columns in which no
+ * candidate can pass the matrix test (the bounding boxes of their edges lie too
+ * far apart for their longest edges).  The selected moves, tours and lengths
+ * are identical; fewer candidates are evaluated, so the sweep's evals/s figure
  * does not apply.  mode: LOGO2OPT_PRUNE_OFF (the default), LOGO2OPT_PRUNE_ALL
  * (every instance), or LOGO2OPT_PRUNE_AUTO (instances of 16,000 cities or
- * more).  On MI355X a lone instance's local search gains from about 16,000
- * cities (4-9% slower below: AUTO); batches of many instances gain at every
- * size measured (ALL).  No counterpart in the reference (its kernels evaluate
- * every pair, opt_kernel.cu:34-262). */
+ * more).  On MI355X a lone instance's local search gains from about 20,000
+ * cities (5-15% slower from 4,000 to 16,000: AUTO leaves those alone; 1.1x at
+ * 33,810, 1.9x at 100,000).  No counterpart in the reference (its kernels
+ * evaluate every pair, opt_kernel.cu:34-262). */
 #define LOGO2OPT_PRUNE_OFF  0
 #define LOGO2OPT_PRUNE_ALL  1
 #define LOGO2OPT_PRUNE_AUTO 2
@@ -370,15 +370,16 @@ int logo2opt_server_replay(logo2opt_server *s, uint32_t count, const double *arr
 /* ======================================================================== */
 /* Sweep tile shapes (autotuning)                                            */
 /* ======================================================================== */
-/* A shape is {k, t, waves}: a workgroup of `waves` wave64s whose lanes each
- * own k adjacent candidate columns of the triangle for t rows.  The
+/* A shape is {k, t, waves}: a workgroup of `waves` wave64s, each of which
+ * tests 64 k columns of the triangle against t rows.  The
  * reference hard-codes <<<64,1024>>> and 2048-point tiles
  * (CUDASolver.cpp:122-128, cuda_defs.h:24-37); here the shape is chosen per
  * n bucket from a table written by the autotuner (tune.py). */
 /* Shapes compiled into the library (3 ints per row); count = total rows. */
 int logo2opt_tuning_shapes(int32_t *out, uint32_t cap, uint32_t *count);
-/* Two tables: table 0 is used while an engine holds fewer than 8 live
- * instances (latency), table 1 for larger batches (throughput).  Replace a
+/* Two tables: table 1 (throughput) is used while at least 8 live instances of
+ * an engine, with 1e8 candidates in all, take steps together, table 0 (latency)
+ * otherwise; instances that run in one workgroup need neither.  Replace a
  * table: row r applies to n <= max_n[r] (the last row to all larger n); work
  * lists built afterwards use it. */
 int logo2opt_tuning_set(int table, const uint32_t *max_n, const int32_t *shapes, uint32_t rows);

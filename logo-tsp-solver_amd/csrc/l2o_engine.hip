@@ -1,9 +1,11 @@
 // l2o_engine.hip -- host side of the C ABI declared in include/logo2opt.h.
 //
 // An engine owns one HIP stream, one HBM arena (the admission budget) and an
-// array of instance slots (l2o_inst, device resident).  A batched step is
+// array of instance slots (l2o_inst, device resident).  Small instances run
+// whole searches in k_local, one workgroup each.  The others take batched steps:
 //   sweep  (one launch per tile shape, covering every live instance)
-//   apply  (one launch, gathers the winning move of every instance)
+//   apply  (one launch, gathers the winning move of every instance), or, in a
+//          run of sweeps, the first workgroups of the next sweep's launch
 //   ils    (one launch, accept/revert + kick for instances at a local optimum)
 // Steps are issued back to back; the host looks at the device only every
 // `sync_every` steps, and then through one 4-byte counter of live instances.
@@ -491,16 +493,19 @@ void drop_graph(logo2opt_engine *e)
     e->gsteps = 0;
 }
 
-// LOGO2OPT_PRUNE_AUTO prunes instances of at least this many cities: below
-// it the pruned sweep measured 4-9% slower (per-wave fixed costs dominate),
-// from 16,000 on it wins (1.04x there, 1.2x at 24,000, 1.6x at 33,810)
+// LOGO2OPT_PRUNE_AUTO prunes instances of at least this many cities, as its
+// documentation says.  Whole searches of one instance, full against pruned:
+// 8,000 cities 10.6 and 12.5 ms, 16,000 28.6 and 30.2, 20,000 43.2 and 43.0,
+// 24,000 65.0 and 62.2, 33,810 147 and 129, 60,000 490 and 313, 100,000 1,874
+// and 976 ms: below 20,000 the boxes cost a little more than they save.
 #define L2O_PRUNE_AUTO_MIN_N 16000u
 #ifndef L2O_DIAG_WEIGHT
 #define L2O_DIAG_WEIGHT 4
 #endif
 
 // 1/L2O_TAIL_SPLIT of a launch's work, at its end, goes in items of
-// 1/L2O_TAIL_DIV of the shape's rows (T/L2O_TAIL_DIV must stay a multiple of 4)
+// 1/L2O_TAIL_DIV of the shape's rows, rounded up to whole blocks of 32 (33,810
+// cities: 196 ms a search without, 139 ms with it; a batch 288 and 293 ms)
 #ifndef L2O_TAIL_SPLIT
 #define L2O_TAIL_SPLIT 8
 #endif
@@ -681,12 +686,10 @@ int rebuild_lists(logo2opt_engine *e)
         // In a batch the first tile of each row block (at the diagonal) is
         // ordered as if it had L2O_DIAG_WEIGHT times its candidates: its rows
         // and columns are tour neighbours, close in the plane, so more of its
-        // blocks pass tier 0 and it runs longer than its count says.  Issued
-        // earlier it no longer ends the launch: the 2,048-instance batch
-        // measured 2.15 -> 1.84 s (the same for weights 3 to 8).  One
-        // instance keeps the plain order: there every slow path publishes to
-        // the same key, and the near-diagonal tiles run best spread over the
-        // launch (weighted, the config-2 local search took 0.39 s, not 0.285).
+        // candidates pass the matrix test and it runs longer than its count
+        // says (512 instances: 304 ms without, 292 ms with it).  One instance
+        // keeps the plain order: there every survivor publishes to the same
+        // key, and the near-diagonal tiles run best spread over the launch.
         for (size_t q = 0; q < v.size(); ++q) {
             work[q] = item_work(v[q], c, e->slots[v[q].inst].n);
             if (table == 1 && v[q].b0 == v[q].a0 + 2) work[q] *= L2O_DIAG_WEIGHT;

@@ -58,7 +58,7 @@ static __device__ __align__(256) unsigned char scratch[NA_BYTES];
 namespace {
 
 // tour-ordered points: P[k] = city route[k] translated by (-mx, -my), with the
-// exact metric length of the edge route[k-1] -> route[k] and its tier-1 bound
+// exact metric length of the edge route[k-1] -> route[k]
 __global__ __launch_bounds__(256) void k_na_points(unsigned char *__restrict__ base, uint32_t n, uint32_t metric,
                                                    double mx, double my)
 {

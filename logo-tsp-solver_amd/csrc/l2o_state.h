@@ -67,7 +67,7 @@ struct l2o_inst {
     uint32_t group_size;  // chains in the group (slots group_lead .. group_lead+size-1)
     uint32_t improved;    // the chain's last local search improved its own best
     uint32_t kick_src;    // slot whose best tour the next kick starts from
-    float est_scale;      // FP32 tier: D ~ sqrt(s) * est_scale + est_add
+    float est_scale;      // FP32 estimate: D ~ sqrt(s) * est_scale + est_add
     float est_add;
     float qs, qox, qoy;   // matrix test: X ~ x qs + qox, Y ~ y qs + qoy,
     float qk, qm;         // and E = ceil(D qk + qm) (set_quant in l2o_launch.h)

@@ -26,16 +26,17 @@
 // most 11 bits, exact in FP16, and every partial sum stays below 2^24
 // (L2O_QR, L2O_QE in l2o_launch.h), exact in FP32: the test has no rounding.
 // One matrix instruction tests 32 x 32 candidates; 16 results per lane are
-// combined by their sign bits (v_or3_b32, two results an instruction), so a
-// candidate costs about 0.7 VALU instructions; the 8-bit v_sad_u8 bound it
-// replaces took 2.2.
+// combined by their sign bits (v_or3_b32, two results an instruction); a
+// candidate costs 1.0 VALU instructions in all (33,810 clustered cities), where
+// the 8-bit v_sad_u8 bound it replaces took 2.2.
 //
 // What bounds it.  A tile of 1,024 candidates holds the matrix unit for 32
 // cycles and needs at least 8 v_or3 (32 cycles of VALU issue); the two overlap
 // only in part (a loop of nothing else: 46 cycles a tile, 5.0e13 candidates/s).
-// Measured with one MI355X, whole steps: 100,000 cities 270 -> 145 us (3.4e13
-// candidates/s), 33,810 clustered 57 -> 33 us, 7,397 20 -> 11.6 us (two
-// launches' latency).  Matrix results kept in AGPRs, as the compiler prefers,
+// At 33,810 cities VALU issue takes 58% and the matrix unit 29% of a launch of
+// 25 us.  Measured with one MI355X, whole steps: 100,000 cities 270 -> 133 us
+// (3.8e13 candidates/s), 33,810 clustered 57 -> 27 us, 7,397 20 -> 7.9 us (a
+// launch's latency).  Matrix results kept in AGPRs, as the compiler prefers,
 // cost a copy each: 2.7e13 instead of 4.4e13 tests/s (-amdgpu-mfma-vgpr-form).
 //
 // E' is cut off at 0 (a larger sum only lets more pass): without it a pair of
@@ -45,7 +46,7 @@
 // Survivors.  The 32 sign bits of a pair of tiles are stored in LDS per lane;
 // every row block the wave compacts them into full waves of candidates, which
 // load their four points, take the FP32 estimate and, if that passes, the exact
-// length (FP64 square root and integer fix-up).  Keys go to the instance's
+// length (integers, l2o_device.h).  Keys go to the instance's
 // shared key by atomicMin; the result is exact and independent of wave order.
 #include <hip/hip_runtime.h>
 
@@ -230,7 +231,7 @@ __device__ __forceinline__ void sweep_item(const l2o_sweep_item it, l2o_inst *__
     }
     // half of -C (waves may start with different caps: each is a valid one)
     const float hc = half_cap(cap, qk);
-    float thr = (float)cap + slack;  // tier 2
+    float thr = (float)cap + slack;  // of the FP32 estimate
 
     // PRUNE: the boxes of the columns and of all rows; an item without a pair of
     // tiles whose boxes meet ends here, before any operand is made (60,000

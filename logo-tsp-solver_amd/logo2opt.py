@@ -283,8 +283,8 @@ def tuning_shapes():
     return [tuple(int(v) for v in out[3 * q:3 * q + 3]) for q in range(cnt.value)]
 
 
-TABLE_SINGLE = 0  # fewer than 8 live instances in an engine
-TABLE_BATCH = 1
+TABLE_SINGLE = 0
+TABLE_BATCH = 1  # 8 live instances or more with 1e8 candidates a step
 
 
 def tuning_set(rows, table=TABLE_SINGLE):

@@ -5,16 +5,16 @@
 Writes two tables ("max_n k t waves" per line) that the library loads on first
 use from its own directory:
   tuning_gfx950.txt        one instance in flight (logo2opt_create contexts,
-                           engines with fewer than 8 live instances): each
+                           engines with few or small live instances): each
                            shape is timed on the steps of a local search from
                            the nearest-neighbour start tour
-  tuning_batch_gfx950.txt  batches (8+ live instances): each shape is timed on
+  tuning_batch_gfx950.txt  batches (8+ live instances, 1e8 candidates a step): each shape is timed on
                            an engine holding enough random-start instances of
                            that size to fill the GPU, run to their local optima
 One table serves both sweep variants, so a shape is scored on the full sweep
 plus, where row pruning is in use (batches, and single instances from the
 size LOGO2OPT_PRUNE_AUTO prunes), the pruned sweep: the sum of the two times.
-A shape is {k columns per lane, t rows, waves per workgroup}.  Bucket edges
+A shape is {k times 64 columns per wave, t rows, waves per workgroup}.  Bucket edges
 are the geometric midpoints between the representative sizes.
 """
 import argparse
@@ -46,7 +46,7 @@ def tune_single(reps=REPS, seed=1, verbose=True):
     every shape, so all shapes run the same steps; the first 64 (graph capture
     included) are not timed.  Timing single sweeps on fixed tours instead
     ranks shapes differently, because the key published during a search
-    tightens the first-tier threshold as the sweep proceeds."""
+    tightens the matrix test's threshold as the sweep proceeds."""
     best = []
     for n in reps:
         side = 10**4 if n <= 5000 else 10**6
