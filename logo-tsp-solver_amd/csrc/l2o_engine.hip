@@ -424,8 +424,8 @@ int fetch(logo2opt_engine *e, int32_t id, l2o_inst *in, uint32_t *tour_out)
 // its record, cities and start tour go to HBM, k_load makes the ordered points
 // of them.  (Made on the host, with a copy and a wait each for points, tour,
 // record and counter, a single sweep of 200 cities took 153 us and one of 33,810
-// cities 655 us; now 40 and 127 us, and 512 admissions about 35 ms less.)
-int upload_instance(logo2opt_engine *e, int32_t id, const cities &ct, const uint32_t *route, uint32_t phase)
+// cities 655 us; now 38 and 97 us, and 512 admissions about 35 ms less.)
+int upload_instance(logo2opt_engine *e, int32_t id, const cities &ct, const uint32_t *route, uint32_t phase, bool count)
 {
     slot_t &s = e->slots[id];
     const uint32_t n = s.n;
@@ -480,7 +480,7 @@ int upload_instance(logo2opt_engine *e, int32_t id, const cities &ct, const uint
     std::memcpy(h, &in, sizeof(in));
     std::memcpy(h + rec, ct.xy.data(), 8ull * n);
     std::memcpy(h + rec + 8ull * n, route, 4ull * n);
-    L2O_TRY(l2o::launch_load(e->d_insts, (uint32_t)id, n, (const l2o_inst *)h, h + rec, e->d_live, e->stream));
+    L2O_TRY(l2o::launch_load(e->d_insts, (uint32_t)id, n, (const l2o_inst *)h, h + rec, e->d_live, count, e->stream));
     return LOGO2OPT_OK;
 }
 
@@ -949,7 +949,8 @@ int engine_run(logo2opt_engine *e, uint32_t max_steps, uint32_t sync_every, uint
 
 // admits an instance into slot `id` (free); group_lead / group_size as in l2o_inst
 int engine_add_at(logo2opt_engine *e, int32_t id, uint32_t n, const cities &ct, const uint32_t *route,
-                  const logo2opt_job *job, uint32_t group_lead, uint32_t group_size, bool sweep_only = false)
+                  const logo2opt_job *job, uint32_t group_lead, uint32_t group_size, bool sweep_only = false,
+                  bool count = true)
 {
     int rc = check_tour(n, route);
     if (rc) return rc;
@@ -972,7 +973,7 @@ int engine_add_at(logo2opt_engine *e, int32_t id, uint32_t n, const cities &ct, 
     s.group_lead = group_lead;
     s.group_size = group_size;
     s.sweep_only = sweep_only;
-    rc = upload_instance(e, id, ct, route, L2O_LO);
+    rc = upload_instance(e, id, ct, route, L2O_LO, count);
     if (rc) {
         e->ar.release(off, bytes);
         s = slot_t();
@@ -991,7 +992,7 @@ int cities_of(uint32_t n, const logo2opt_city_coords *coords, cities &ct)
 }
 
 int engine_add(logo2opt_engine *e, uint32_t n, const cities &ct, const uint32_t *route, const logo2opt_job *job,
-               int32_t *slot_out, bool sweep_only = false)
+               int32_t *slot_out, bool sweep_only = false, bool count = true)
 {
     int32_t id = -1;
     for (uint32_t k = 0; k < e->max_slots; ++k)
@@ -1000,12 +1001,12 @@ int engine_add(logo2opt_engine *e, uint32_t n, const cities &ct, const uint32_t 
             break;
         }
     if (id < 0) return LOGO2OPT_EAGAIN;
-    const int rc = engine_add_at(e, id, n, ct, route, job, L2O_NO_GROUP, 0, sweep_only);
+    const int rc = engine_add_at(e, id, n, ct, route, job, L2O_NO_GROUP, 0, sweep_only, count);
     if (rc == LOGO2OPT_OK) *slot_out = id;
     return rc;
 }
 
-int engine_remove(logo2opt_engine *e, int32_t id);
+int engine_remove(logo2opt_engine *e, int32_t id, bool clear = true);
 
 // `chains` ILS chains of one instance in consecutive slots; chain c uses the
 // seed job->seed + c
@@ -1060,7 +1061,8 @@ int engine_result(logo2opt_engine *e, int32_t id, uint32_t *route_out, logo2opt_
     return LOGO2OPT_OK;
 }
 
-int engine_remove(logo2opt_engine *e, int32_t id)
+// clear = false: the slot's record stays, live if it was, for an admission that replaces it
+int engine_remove(logo2opt_engine *e, int32_t id, bool clear)
 {
     if (id < 0 || (uint32_t)id >= e->max_slots || !e->slots[id].used) return LOGO2OPT_ENOTFOUND;
     {
@@ -1079,7 +1081,8 @@ int engine_remove(logo2opt_engine *e, int32_t id)
     slot_t &s = e->slots[id];
     // (the host knows: a run ends with the state of its finished instances read)
     if (!s.done) e->live -= 1;
-    L2O_TRY(l2o::launch_free(e->d_insts, (uint32_t)id, e->d_live, !s.done, !s.done && !s.sweep_only, e->stream));
+    if (clear)
+        L2O_TRY(l2o::launch_free(e->d_insts, (uint32_t)id, e->d_live, !s.done, !s.done && !s.sweep_only, e->stream));
     e->ar.release(s.off, s.bytes);
     s = slot_t();
     e->dirty = true;
@@ -1469,9 +1472,16 @@ void ctx_accumulate(logo2opt_ctx *c)
 int ctx_load(logo2opt_ctx *c, const uint32_t *route, logo2opt_job job, bool sweep_only = false)
 {
     job.metric = c->metric;
+    bool live = false, freed = true;  // the slot's record on the device
     if (c->slot >= 0) {
         ctx_accumulate(c);
-        int rc = engine_remove(c->e, c->slot);
+        // the one slot's next instance takes over its record, unless a search
+        // was left half-way (its pool holds moves)
+        const slot_t &s = c->e->slots[c->slot];
+        const bool over = s.done || s.sweep_only;
+        live = over && !s.done;
+        freed = !over;
+        int rc = engine_remove(c->e, c->slot, !over);
         if (rc) return rc;
         c->slot = -1;
     }
@@ -1480,18 +1490,33 @@ int ctx_load(logo2opt_ctx *c, const uint32_t *route, logo2opt_job job, bool swee
         // for: replace it by a larger one with the same settings
         logo2opt_engine *old = c->e, *e = nullptr;
         int rc = engine_create(old->device, ctx_budget(c->n, job), 1, &e);
-        if (rc) return rc;
+        if (rc) {
+            if (!freed) L2O_TRY(l2o::launch_free(old->d_insts, 0, old->d_live, live, false, old->stream));
+            return rc;
+        }
         e->timing = old->timing;
         e->graphs = old->graphs;
         e->prune = old->prune;
         c->sweep_ms += old->sweep_ms;
         logo2opt_engine_destroy(old);
         c->e = e;
+        live = false;
+        freed = true;
     }
-    return engine_add(c->e, c->n, c->ct, route, &job, &c->slot, sweep_only);
+    const int rc = engine_add(c->e, c->n, c->ct, route, &job, &c->slot, sweep_only, !live);
+    if (rc && !freed) L2O_TRY(l2o::launch_free(c->e->d_insts, 0, c->e->d_live, live, false, c->e->stream));
+    return rc;
 }
 
 }  // namespace
+
+// A single sweep of at least this many cities gets a first cap from k_prime,
+// 3.7 us of launch: whole calls without and with it, nearest-neighbour tours of
+// 1,000 cities 38.3 and 38.2 us, 8,000 49.5 and 47.7, 33,810 118 and 96; random
+// tours of 1,000 cities 66 and 38 us, 4,000 152 and 44, 33,810 1,116 and 87;
+// local optima, where there is nothing to find, 3,000 36.4 and 40.7, 33,810 86
+// and 92; 200 cities 38 and 42 us.
+#define L2O_PRIME_MIN_N 1000u
 
 int logo2opt_step(logo2opt_ctx *ctx, const uint32_t *route, logo2opt_best2_out *out, logo2opt_process_time *t)
 {
@@ -1508,6 +1533,7 @@ int logo2opt_step(logo2opt_ctx *ctx, const uint32_t *route, logo2opt_best2_out *
     if (rc) return rc;
     const double h1 = now_ms();
     L2O_TRY(hipEventRecord(e->ev0, e->stream));
+    if (ctx->n >= L2O_PRIME_MIN_N) L2O_TRY(l2o::launch_prime(e->d_insts, (uint32_t)ctx->slot, ctx->n, e->stream));
     for (const auto &g : e->groups)
         L2O_TRY(launch_group_sweep(e, g));
     L2O_TRY(hipEventRecord(e->ev1, e->stream));

@@ -242,8 +242,10 @@ __global__ __launch_bounds__(256) void k_stage(l2o_inst *__restrict__ in, const 
 }
 
 // the tour-ordered points of an admitted instance: coordinates, exact edge
-// lengths, quantised coordinates; city ids and the tour's length
-__global__ __launch_bounds__(256) void k_load(l2o_inst *__restrict__ insts, uint32_t slot, unsigned *__restrict__ live)
+// lengths, quantised coordinates; city ids and the tour's length.  Behind the raw
+// cities each wave leaves the position of its longest edge's end (0: none).
+__global__ __launch_bounds__(256) void k_load(l2o_inst *__restrict__ insts, uint32_t slot, unsigned *__restrict__ live,
+                                              int count)
 {
     l2o_inst *in = insts + slot;
     const int n = (int)in->n;
@@ -252,7 +254,7 @@ __global__ __launch_bounds__(256) void k_load(l2o_inst *__restrict__ insts, uint
     const uint32_t *__restrict__ route = (const uint32_t *)(xy + n);
     l2o_pt *__restrict__ P = in->pts[0];
     uint32_t *__restrict__ R = in->tour[0];
-    unsigned long long sum = 0;
+    unsigned long long sum = 0, longest = ~0ull;
     for (int k = (int)(blockIdx.x * 256 + threadIdx.x); k < n; k += (int)gridDim.x * 256) {
         const uint32_t c = route[k], pc = route[k ? k - 1 : n - 1];
         const int2 a = xy[c], b = xy[pc];
@@ -264,10 +266,47 @@ __global__ __launch_bounds__(256) void k_load(l2o_inst *__restrict__ insts, uint
         sum += (unsigned long long)r.d;
         P[k] = r;
         R[k] = c;
+        const unsigned long long e = (unsigned long long)(uint32_t)~r.d << 32 | (uint32_t)k;
+        if (k && e < longest) longest = e;  // (edge 0 closes the tour: no candidate's)
     }
     sum = wave_sum_u64(sum);
+    longest = wave_min_u64(longest);
+    if ((threadIdx.x & 63) == 0)
+        ((uint32_t *)(route + n))[blockIdx.x * 4 + (threadIdx.x >> 6)] = longest == ~0ull ? 0u : (uint32_t)longest;
     if ((threadIdx.x & 63) == 0 && sum) atomicAdd(&in->length, sum);
-    if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(live, 1u);
+    if (count && blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(live, 1u);
+}
+
+// A cap for the first sweep of an instance: the best candidate between the `m`
+// long edges k_load found, into in->cap.  The best move of a tour nearly always
+// removes two of them, so the sweep's test passes little else.  Latency: three
+// dependent loads, one exact gain per lane and turn.
+__global__ __launch_bounds__(256) void k_prime(l2o_inst *__restrict__ insts, uint32_t slot, uint32_t m)
+{
+    l2o_inst *in = insts + slot;
+    const uint32_t metric = in->metric;
+    const l2o_pt *__restrict__ P = in->pts[0];
+    const uint32_t *__restrict__ ends = (const uint32_t *)in->pts[1] + 3 * in->n;
+    __shared__ int s_best;
+    if (threadIdx.x == 0) s_best = -1;
+    __syncthreads();
+    const uint32_t q = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const uint32_t ka = q < m ? ends[q] : 0u;
+    int best = -1;
+    if (ka) {
+        const l2o_pt a0 = P[ka - 1], a1 = P[ka];
+        for (uint32_t r = q + 1 + lane; r < m; r += 64) {
+            const uint32_t kb = ends[r];
+            if (kb == 0 || (kb < ka ? ka - kb : kb - ka) < 2) continue;  // edges with a common end
+            const l2o_pt b0 = P[kb - 1], b1 = P[kb];
+            best = min(best, exact_dist(a0.x, a0.y, b0.x, b0.y, metric) + exact_dist(a1.x, a1.y, b1.x, b1.y, metric) -
+                                 a1.d - b1.d);
+        }
+    }
+    if (best < -1) atomicMin(&s_best, best);
+    __syncthreads();
+    if (threadIdx.x == 0 && s_best < __hip_atomic_load(&in->cap, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicMin(&in->cap, s_best);
 }
 
 // release of a slot: its record blank, its pool empty (`running`: it was live)
@@ -370,14 +409,21 @@ hipError_t launch_group(l2o_inst *insts, uint32_t nslots, unsigned *live, hipStr
 static uint32_t blocks_for(uint32_t n) { return n < 256 * 256 ? (n + 255) / 256 : 256; }
 
 hipError_t launch_load(l2o_inst *insts, uint32_t slot, uint32_t n, const l2o_inst *rec, const void *raw, unsigned *live,
-                       hipStream_t stream)
+                       bool count, hipStream_t stream)
 {
     const uint32_t words = (12 * n + 15) / 16;  // (the point buffer holds 16 n bytes)
     hipLaunchKernelGGL(k_stage, dim3(blocks_for(words)), dim3(256), 0, stream, insts + slot, rec, (uint4 *)rec->pts[1],
                        (const uint4 *)raw, words);
     const hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
-    hipLaunchKernelGGL(k_load, dim3(blocks_for(n)), dim3(256), 0, stream, insts, slot, live);
+    hipLaunchKernelGGL(k_load, dim3(blocks_for(n)), dim3(256), 0, stream, insts, slot, live, count ? 1 : 0);
+    return hipGetLastError();
+}
+
+hipError_t launch_prime(l2o_inst *insts, uint32_t slot, uint32_t n, hipStream_t stream)
+{
+    const uint32_t blocks = blocks_for(n);  // as many waves as k_load's
+    hipLaunchKernelGGL(k_prime, dim3(blocks), dim3(256), 0, stream, insts, slot, 4 * blocks);
     return hipGetLastError();
 }
 

@@ -107,9 +107,11 @@ hipError_t launch_local(int waves, const uint32_t *ids, uint32_t count, uint32_t
 uint32_t local_lds_bytes(uint32_t n, int waves);
 hipError_t launch_group(l2o_inst *insts, uint32_t nslots, unsigned *live, hipStream_t stream);
 // admission, release and result of a slot (l2o_kernels.hip)
-// (`rec` and `raw`: pinned host memory, 16-byte aligned, a multiple of 16 bytes)
+// (`rec` and `raw`: pinned host memory, 16-byte aligned, a multiple of 16 bytes;
+// `count`: the slot was not live)
 hipError_t launch_load(l2o_inst *insts, uint32_t slot, uint32_t n, const l2o_inst *rec, const void *raw, unsigned *live,
-                       hipStream_t stream);
+                       bool count, hipStream_t stream);
+hipError_t launch_prime(l2o_inst *insts, uint32_t slot, uint32_t n, hipStream_t stream);  // after launch_load
 hipError_t launch_free(l2o_inst *insts, uint32_t slot, unsigned *live, bool running, bool clear_pool, hipStream_t stream);
 hipError_t launch_fetch(const l2o_inst *insts, uint32_t slot, uint32_t n, l2o_inst *rec, uint32_t *tour,
                         hipStream_t stream);
